@@ -17,10 +17,10 @@
 //       g_sl at x - ts*v, g_v(x) -= ts * <grad S(sl), -g/2>
 //   B2  scatter g_sl into g_rho at x + ts*v, g_v(x) += ts * <grad S(rho), g_sl>
 //   B3  staggered: g_face = (g_v(left cell) + g_v(right cell)) / 2
-// For 1-2 channels the scatters of B1 / B2 accumulate in LDS tiles per brick
-// of cells and are summed by the consumer (no global atomics unless a
-// displacement leaves the tile halo); the reference-normalised gradient and
-// 3-4 channels scatter with hardware fp32 atomics.
+// The scatters of B1 / B2 accumulate in LDS tiles per brick of cells and are
+// summed by the consumer (no global atomics unless a displacement leaves the
+// tile halo); the reference-normalised gradient scatters with hardware fp32
+// atomics.
 #include <algorithm>
 
 #include "ngt_host.hpp"
@@ -44,6 +44,18 @@ NGT_DEVICE void pair_indices(const AdvArgs& a, int pair, int& n, int& v) {
   if (a.separate) { n = pair / a.n_vel; v = pair % a.n_vel; }
   else { n = pair; v = pair; }
 }
+
+// The centered velocity gradient of the adjoint: the caller's [V,D,H,W,3]
+// (centered velocity), or workspace planes [V,3,D,H,W] (staggered: consecutive
+// cells' values are consecutive, for the stores and for the face gather).
+struct GradVel {
+  float* p;
+  int64_t cells;
+  int cell_step;  // 3 or 1
+  NGT_DEVICE float* at(int v, int64_t cell, int k) const {
+    return p + static_cast<int64_t>(v) * cells * 3 + cell * cell_step + (cell_step == 3 ? k : k * cells);
+  }
+};
 
 NGT_DEVICE void load_velocity(const AdvArgs& a, int v, int x, int y, int z, float& ux, float& uy, float& uz) {
   const Dims& d = a.d;
@@ -148,14 +160,14 @@ __global__ __launch_bounds__(256) void advect_mc_kernel(AdvArgs a, const float* 
   advect_mc_kernel_body<C, BM, CLAMPM>(VBlock{static_cast<int>(blockIdx.x), static_cast<int>(blockIdx.y), static_cast<int>(blockIdx.z)}, a, rho, sl, out);
 }
 
-// B1 (order 2): route g to the SL field and the direct rho term; scatter the
-// back-step adjoint into g_sl.  REF: scatter into tmp with hit counts.
-template <int C, int BM, int CLAMPM, bool REF>
+// Reference gradient semantics, B1 (order 2): route g to the SL field and the
+// direct rho term; scatter the back-step adjoint into tmp with hit counts.
+template <int C, int BM, int CLAMPM>
 __global__ __launch_bounds__(256) void advect_mc_bwd_kernel(AdvArgs a, const float* __restrict__ rho,
                                                             const float* __restrict__ sl,
                                                             const float* __restrict__ g_out,
                                                             float* __restrict__ g_sl, float* __restrict__ g_rho,
-                                                            float* __restrict__ g_vc, float* __restrict__ tmp,
+                                                            GradVel gv, float* __restrict__ tmp,
                                                             uint32_t* __restrict__ hits) {
   const ThreadCell t = thread_cell(a, VBlock{static_cast<int>(blockIdx.x), static_cast<int>(blockIdx.y), static_cast<int>(blockIdx.z)});
   if (!t.ok) return;
@@ -199,24 +211,18 @@ __global__ __launch_bounds__(256) void advect_mc_bwd_kernel(AdvArgs a, const flo
     atomic_add(g_rho + (n * cells + cell) * C + i, 0.5f * keep.v[i] * g.v[i]);
     gback.v[i] = -0.5f * keep.v[i] * g.v[i];
   }
-  if constexpr (REF) {
-    scatter_linear<C, BM, true>(tmp + (t.pair * cells) * C, a.d, bx, by, bz, gback, hits + t.pair * cells);
-  } else {
-    scatter_linear<C, BM, false>(gsl, a.d, bx, by, bz, gback);
-  }
-  float* gv = g_vc + (static_cast<int64_t>(v) * cells + cell) * 3;
-  atomic_add(gv + 0, -a.ts * vdot(gback, dx));
-  atomic_add(gv + 1, -a.ts * vdot(gback, dy));
-  atomic_add(gv + 2, -a.ts * vdot(gback, dz));
+  scatter_linear<C, BM, true>(tmp + (t.pair * cells) * C, a.d, bx, by, bz, gback, hits + t.pair * cells);
+  atomic_add(gv.at(v, cell, 0), -a.ts * vdot(gback, dx));
+  atomic_add(gv.at(v, cell, 1), -a.ts * vdot(gback, dy));
+  atomic_add(gv.at(v, cell, 2), -a.ts * vdot(gback, dz));
 }
 
-// B2: adjoint of the semi-Lagrangian read.  For order 1, g_sl is g_out with
-// the NEGATIVE mask applied on the fly (NEG).
-template <int C, int BM, bool NEG, bool REF>
+// Reference gradient semantics, B2: adjoint of the semi-Lagrangian read into
+// tmp with hit counts.  For order 1, g_sl is g_out with the NEGATIVE mask
+// applied on the fly (NEG).
+template <int C, int BM, bool NEG>
 __global__ __launch_bounds__(256) void advect_sl_bwd_kernel(AdvArgs a, const float* __restrict__ rho,
-                                                            const float* __restrict__ g_sl,
-                                                            const float* __restrict__ sl_out,
-                                                            float* __restrict__ g_rho, float* __restrict__ g_vc,
+                                                            const float* __restrict__ g_sl, GradVel gv,
                                                             float* __restrict__ tmp, uint32_t* __restrict__ hits) {
   const ThreadCell t = thread_cell(a, VBlock{static_cast<int>(blockIdx.x), static_cast<int>(blockIdx.y), static_cast<int>(blockIdx.z)});
   if (!t.ok) return;
@@ -237,18 +243,12 @@ __global__ __launch_bounds__(256) void advect_sl_bwd_kernel(AdvArgs a, const flo
     for (int i = 0; i < C; ++i)
       if (!(r.v[i] >= 0.f)) g.v[i] = 0.f;
   }
-  (void)sl_out;
-  if constexpr (REF) {
-    scatter_linear<C, BM, true>(tmp + (t.pair * cells) * C, a.d, px, py, pz, g, hits + t.pair * cells);
-  } else {
-    scatter_linear<C, BM, false>(g_rho + n * cells * C, a.d, px, py, pz, g);
-  }
+  scatter_linear<C, BM, true>(tmp + (t.pair * cells) * C, a.d, px, py, pz, g, hits + t.pair * cells);
   Vec<C> dx, dy, dz;
   read_gradient<C, BM>(src, a.d, px, py, pz, dx, dy, dz);
-  float* gv = g_vc + (static_cast<int64_t>(v) * cells + cell) * 3;
-  atomic_add(gv + 0, a.ts * vdot(g, dx));
-  atomic_add(gv + 1, a.ts * vdot(g, dy));
-  atomic_add(gv + 2, a.ts * vdot(g, dz));
+  atomic_add(gv.at(v, cell, 0), a.ts * vdot(g, dx));
+  atomic_add(gv.at(v, cell, 1), a.ts * vdot(g, dy));
+  atomic_add(gv.at(v, cell, 2), a.ts * vdot(g, dz));
 }
 
 // dst(pair or n) += tmp / hits (reference count normalisation), one cell per
@@ -274,7 +274,7 @@ __global__ __launch_bounds__(256) void add_normalized_kernel(AdvArgs a, const fl
 
 // B3: centered-velocity gradient -> MAC face gradients (adjoint of the face
 // average).  A work-group covers 64 x 4 (x, y) columns of one velocity over
-// kFaceZ planes; each work-item walks its column in z, so g_vc is read once:
+// kFaceZ planes; each work-item walks its column in z, so the gradient is read once:
 // the z - 1 term is the previous plane's value kept in a register, the x - 1
 // and y - 1 terms hit the lines the neighbouring work-items just read.  The
 // last cell of an axis also writes the closing face (x = d.x, y = d.y,
@@ -285,7 +285,7 @@ inline int64_t face_tiles(const Dims& d) {
   return static_cast<int64_t>((d.x + 63) / 64) * ((d.y + 3) / 4) * ((d.z + kFaceZ - 1) / kFaceZ);
 }
 
-NGT_DEVICE void faces_from_centered_grad_kernel_body(const VBlock& vb, Dims d, int n_vel, const float* __restrict__ g_vc,
+NGT_DEVICE void faces_from_centered_grad_kernel_body(const VBlock& vb, Dims d, int n_vel, const GradVel& gv,
                                                      float* __restrict__ gx, float* __restrict__ gy,
                                                      float* __restrict__ gz) {
   const int ntx = (d.x + 63) / 64, nty = (d.y + 3) / 4, nzc = (d.z + kFaceZ - 1) / kFaceZ;
@@ -300,16 +300,15 @@ NGT_DEVICE void faces_from_centered_grad_kernel_body(const VBlock& vb, Dims d, i
   const int64_t ny = static_cast<int64_t>(d.z) * (d.y + 1) * d.x;
   const int64_t nz = static_cast<int64_t>(d.z + 1) * d.y * d.x;
   const int64_t cells = static_cast<int64_t>(d.x) * d.y * d.z;
-  const float* g = g_vc + static_cast<int64_t>(v) * cells * 3;
   float* ox = gx + static_cast<int64_t>(v) * nx;
   float* oy = gy + static_cast<int64_t>(v) * ny;
   float* oz = gz + static_cast<int64_t>(v) * nz;
-  float prev = z0 > 0 ? g[cell_offset(d, x, y, z0 - 1) * 3 + 2] : 0.f;
+  float prev = z0 > 0 ? *gv.at(v, cell_offset(d, x, y, z0 - 1), 2) : 0.f;
   for (int z = z0; z < z1; ++z) {
     const int64_t c = cell_offset(d, x, y, z);
-    const float g0 = g[c * 3 + 0], g1 = g[c * 3 + 1], g2 = g[c * 3 + 2];
-    const float l0 = x > 0 ? g[(c - 1) * 3 + 0] : 0.f;
-    const float l1 = y > 0 ? g[(c - d.x) * 3 + 1] : 0.f;
+    const float g0 = *gv.at(v, c, 0), g1 = *gv.at(v, c, 1), g2 = *gv.at(v, c, 2);
+    const float l0 = x > 0 ? *gv.at(v, c - 1, 0) : 0.f;
+    const float l1 = y > 0 ? *gv.at(v, c - d.x, 1) : 0.f;
     const int64_t fx = (static_cast<int64_t>(z) * d.y + y) * (d.x + 1) + x;
     ox[fx] = 0.5f * (l0 + g0);
     if (x == d.x - 1) ox[fx + 1] = 0.5f * g0;
@@ -322,14 +321,14 @@ NGT_DEVICE void faces_from_centered_grad_kernel_body(const VBlock& vb, Dims d, i
   if (z1 == d.z) oz[cells + static_cast<int64_t>(y) * d.x + x] = 0.5f * prev;
 }
 
-__global__ __launch_bounds__(256) void faces_from_centered_grad_kernel(Dims d, int n_vel, const float* __restrict__ g_vc,
+__global__ __launch_bounds__(256) void faces_from_centered_grad_kernel(Dims d, int n_vel, GradVel gv,
                                                                       float* __restrict__ gx, float* __restrict__ gy,
                                                                       float* __restrict__ gz) {
-  faces_from_centered_grad_kernel_body(VBlock{static_cast<int>(blockIdx.x), static_cast<int>(blockIdx.y), static_cast<int>(blockIdx.z)}, d, n_vel, g_vc, gx, gy, gz);
+  faces_from_centered_grad_kernel_body(VBlock{static_cast<int>(blockIdx.x), static_cast<int>(blockIdx.y), static_cast<int>(blockIdx.z)}, d, n_vel, gv, gx, gy, gz);
 }
 
 // ---------------------------------------------------------------------------
-// Brick-tiled exact backward (C <= 2).  A work-group owns a brick of
+// Brick-tiled exact backward.  A work-group owns a brick of
 // kBrickX x kBrickY x kBrickZ cells and an LDS tile of the brick grown by
 // kHalo cells on every side.  The trilinear scatter of the brick's samples
 // lands in the tile whenever the displacement s = ts*v per axis satisfies
@@ -339,13 +338,20 @@ __global__ __launch_bounds__(256) void faces_from_centered_grad_kernel(Dims d, i
 // to an overflow field with global fp32 atomics.  Each tile is stored whole
 // to a per-brick partial buffer with plain coalesced stores, and the
 // consumer gathers, for every cell, the (at most 2 per axis) tiles that
-// cover it in a fixed order: no global atomics in the common case.  (Within
-// a tile the LDS float atomics add in no fixed order.)  The halo sets the
-// partial-buffer traffic: tile cells per brick cell 2.11 with kHalo = 2,
-// 2.86 with 3.  16 cells in z (rather than 8) shorten that ratio and give
-// the column walks of the scatter more shared corner planes; 32 was slower.
+// cover it in a fixed order: no global atomics in the common case.
+//
+// The tile holds doubles: the LDS adds fp64 atomically at 6.7 lanes per clock
+// and CU (3.0 at random addresses) but fp32 at 0.33, so a sample's 8 corners
+// are added as they are.  (Within a tile the atomics add in no fixed order;
+// in fp64 that changes the stored fp32 partials hardly ever.)  One channel's
+// tile is 69 KB, two work-groups per CU; several channels take turns in it.
+// Measured: 128^3, one channel, B1 / B2 45.6 / 45.7 us with fp32 tiles and
+// merged neighbours -> 40.1 / 38.6; 96x160x96, three channels, 717 / 597 us
+// with global fp32 atomics -> 68 / 71.
+// The halo sets the partial-buffer traffic: tile cells per brick cell 2.11
+// with kHalo = 2, 2.86 with 3.
 constexpr int kBrickX = 32, kBrickY = 8, kBrickZ = 16, kHalo = 2;
-// a work-group is kBrickX x kBrickY x kBrickZT work-items; each walks
+// a work-group is kBrickX x kBrickY x kBrickZT work-items; each visits
 // kBrickZ / kBrickZT cells of its (x, y) column
 constexpr int kBrickZT = 2, kBrickZPer = kBrickZ / kBrickZT;
 constexpr int kBrickThreads = kBrickX * kBrickY * kBrickZT;
@@ -362,178 +368,41 @@ inline BrickGrid brick_grid(const Dims& d) {
                    static_cast<int>(blocks_for(d.z, kBrickZ))};
 }
 
-// The upper-z corner plane of the last in-tile scatter of a z-column walk,
-// held in registers: the next cell of the column usually has these four
-// corners as its lower plane, and the two contributions then reach the LDS
-// tile with one atomic add per corner instead of two.
-template <int C>
-struct HeldPlane {
-  int base = -1;  // tile slot of corner (x0, y0), -1 = nothing held
-  int dx = 0;     // slot step from x0 to x1: 0 or 1, or across the tile where WRAP wraps x1
-  int dy = 0;     // slot step from y0 to y1: 0 or kTileX, or across the tile under WRAP
-  Vec<C> v[4];    // corners (x0,y0), (x1,y0), (x0,y1), (x1,y1)
-};
-
-template <int C>
-NGT_DEVICE void plane_add(float* tile, int base, int dx, int dy, const Vec<C> (&v)[4]) {
-  const int off[4] = {0, dx, dy, dx + dy};
-#pragma unroll
-  for (int k = 0; k < 4; ++k) {
-    float* t = tile + (base + off[k]) * C;
-#pragma unroll
-    for (int i = 0; i < C; ++i) lds_add(t + i, v[k].v[i]);
-  }
-}
-
-// Value of the previous / next lane of the 16-lane DPP row (row_shr:1 /
-// row_shl:1); 0 where that lane is outside the row or disabled.
-NGT_DEVICE int from_prev_lane(int v) { return __builtin_amdgcn_update_dpp(0, v, 0x111, 0xF, 0xF, false); }
-NGT_DEVICE int from_next_lane(int v) { return __builtin_amdgcn_update_dpp(0, v, 0x101, 0xF, 0xF, false); }
-NGT_DEVICE float from_prev_lane(float v) {
-  return __builtin_bit_cast(float, from_prev_lane(__builtin_bit_cast(int, v)));
-}
-// Value of lane (l + 32) % 64 (v_permlane32_swap of the wave's two halves).
-NGT_DEVICE int from_other_half(int v) {
-  const auto r = __builtin_amdgcn_permlane32_swap(v, v, false, false);
-  return __lane_id() < 32 ? static_cast<int>(r[1]) : static_cast<int>(r[0]);
-}
-NGT_DEVICE float from_other_half(float v) {
-  return __builtin_bit_cast(float, from_other_half(__builtin_bit_cast(int, v)));
-}
-
-// plane_add for the lanes with `on` set, with the corners that neighbouring
-// lanes share added once.  A wave holds two brick rows, y (lanes 0-31) and
-// y + 1 (lanes 32-63), of consecutive x cells, so usually
-//  - a lane's x1 column is the x0 column of the next lane of its DPP row: it
-//    hands that column over;
-//  - then a lane of row y has as its y1 row the y0 row of lane + 32, which
-//    takes it where it still adds those slots itself.
-// Every lane of the calling loop executes it (the exchanges read the other
-// lanes' registers); a lane whose partner is outside the row or disabled
-// sees 0 and keeps its own adds.
-template <int C>
-NGT_DEVICE void plane_add_row_merged(float* tile, bool on, int base, int dx, int dy, Vec<C> (&v)[4]) {
-  static_assert(kBrickX == 32 && kBrickY % 2 == 0, "the two halves of a wave are consecutive brick rows");
-  // keys carry the exact slot steps (WRAP can make them anything across the
-  // tile): x column = (first slot, y row step), y row = (first slot, x step);
-  // 0 = nothing offered
-  static_assert(kTileX <= 64 && kTileY <= 16 && kTileCells < (1 << 18), "merge key ranges");
-  const int ry = dy / kTileX + 16;  // 5 bits
-  const int rx = dx + 64;           // 7 bits
-  // x: my x1 column (slots base + dx, base + dx + dy) to the next lane
-  const int give_key = on ? ((base + dx + 1) << 5) | ry : 0;
-  const bool take_x = on && from_prev_lane(give_key) == (((base + 1) << 5) | ry);
-#pragma unroll
-  for (int i = 0; i < C; ++i) {
-    const float r0 = from_prev_lane(v[1].v[i]), r1 = from_prev_lane(v[3].v[i]);
-    if (take_x) {
-      v[0].v[i] += r0;
-      v[2].v[i] += r1;
-    }
-  }
-  const bool own1 = !(from_next_lane(take_x ? 1 : 0) != 0);  // still adds its x1 column
-  // y: the y1 row (slots base + dy, base + dy + dx) of a lane of row y to lane + 32
-  const bool upper = __lane_id() >= 32;
-  const int ykey = (on && !upper) ? ((((base + dy + 1) << 7) | rx) << 1) | (own1 ? 1 : 0) : 0;
-  const int got = from_other_half(ykey);
-  const bool take_y = on && upper && (got >> 1) == (((base + 1) << 7) | rx);
-  const bool take_y3 = take_y && (got & 1) && own1;  // the x1 slot of the row, where both still own it
-#pragma unroll
-  for (int i = 0; i < C; ++i) {
-    const float r2 = from_other_half(v[2].v[i]), r3 = from_other_half(v[3].v[i]);
-    if (take_y) v[0].v[i] += r2;
-    if (take_y3) v[1].v[i] += r3;
-  }
-  const int back = from_other_half((take_y ? 1 : 0) | (take_y3 ? 2 : 0));
-  const bool own2 = upper || !(back & 1);
-  const bool own3 = own1 && (upper || !(back & 2));
-  if (on) {
-    const int off[4] = {0, dx, dy, dx + dy};
-    const bool own[4] = {true, own1, own2, own3};
-#pragma unroll
-    for (int k = 0; k < 4; ++k) {
-      if (!own[k]) continue;
-      float* t = tile + (base + off[k]) * C;
-#pragma unroll
-      for (int i = 0; i < C; ++i) lds_add(t + i, v[k].v[i]);
-    }
-  }
-}
-
-// Adds what `held` holds to the tile and empties it.  Executed by every lane
-// of the walk at its end.
-template <int C>
-NGT_DEVICE void flush_plane(float* tile, HeldPlane<C>& held) {
-  plane_add_row_merged<C>(tile, held.base >= 0, held.base, held.dx, held.dy, held.v);
-  held.base = -1;
+// fp64 atomic add into LDS (ds_add_f64); t must point into __shared__ memory.
+typedef __attribute__((address_space(3))) double lds_double;
+NGT_DEVICE void lds_add(double* t, float v) {
+  __hip_atomic_fetch_add((lds_double*)t, static_cast<double>(v), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
 }
 
 // Scatter val * w to the 8 corners of q: into the LDS tile (origin o*) when
-// the corner lies in it, else atomically into `ovf` (a full field).  Called
-// by every lane of a z-column walk for its consecutive cells (`on` false for
-// a lane that scatters nothing), with one `held` plane per walk that
-// flush_plane empties at the end of the walk.
-template <int C, int BM>
-NGT_DEVICE void scatter_linear_tile(float* tile, HeldPlane<C>& held, bool on, int ox, int oy, int oz,
-                                    float* __restrict__ ovf, const Dims& d, float qx, float qy, float qz,
-                                    const Vec<C>& val) {
+// the corner lies in it, else atomically into `ovf`, every `ovf_step`-th
+// value of a full field.
+template <int BM>
+NGT_DEVICE void scatter_linear_tile(double* tile, int ox, int oy, int oz, float* __restrict__ ovf, int ovf_step,
+                                    const Dims& d, float qx, float qy, float qz, float val) {
   const Corners c = make_corners<BM>(d, qx, qy, qz);
-  bool inside = on;
-  if constexpr (BM == BORDER) inside = on && c.inside;
-  const float fw[2][3] = {{1.f - c.wx, 1.f - c.wy, 1.f - c.wz}, {c.wx, c.wy, c.wz}};
-  const int lx0 = c.x0 - ox, lx1 = c.x1 - ox, ly0 = c.y0 - oy, ly1 = c.y1 - oy, lz0 = c.z0 - oz, lz1 = c.z1 - oz;
-  const bool in_tile = inside && static_cast<unsigned>(lx0) < static_cast<unsigned>(kTileX) &&
-                       static_cast<unsigned>(lx1) < static_cast<unsigned>(kTileX) &&
-                       static_cast<unsigned>(ly0) < static_cast<unsigned>(kTileY) &&
-                       static_cast<unsigned>(ly1) < static_cast<unsigned>(kTileY) &&
-                       static_cast<unsigned>(lz0) < static_cast<unsigned>(kTileZ) &&
-                       static_cast<unsigned>(lz1) < static_cast<unsigned>(kTileZ);
-  // the common case, all 8 corners in the tile (a BORDER corner outside the
-  // grid adds 0 to its halo slot instead of being skipped, which leaves every
-  // sum unchanged)
-  float wx[2] = {fw[0][0], fw[1][0]}, wy[2] = {fw[0][1], fw[1][1]}, wz[2] = {fw[0][2], fw[1][2]};
   if constexpr (BM == BORDER) {
-    wx[0] = c.vx0 ? wx[0] : 0.f;
-    wx[1] = c.vx1 ? wx[1] : 0.f;
-    wy[0] = c.vy0 ? wy[0] : 0.f;
-    wy[1] = c.vy1 ? wy[1] : 0.f;
-    wz[0] = c.vz0 ? wz[0] : 0.f;
-    wz[1] = c.vz1 ? wz[1] : 0.f;
+    if (!c.inside) return;
   }
-  const int dx = lx1 - lx0, dy = (ly1 - ly0) * kTileX;
-  const int base0 = (lz0 * kTileY + ly0) * kTileX + lx0;
-  const int base1 = base0 + (lz1 - lz0) * (kTileX * kTileY);
-  Vec<C> lo[4], hi[4];
+  const float fw[2][3] = {{1.f - c.wx, 1.f - c.wy, 1.f - c.wz}, {c.wx, c.wy, c.wz}};
+  const int lx0 = c.x0 - ox, ly0 = c.y0 - oy, lz0 = c.z0 - oz;
+  if constexpr (BM == BORDER) {
+    // the common case, floor and floor + 1 of every axis in the tile, at fixed
+    // offsets from one address (where ceil is floor, at an integer position,
+    // the upper weight is 0; a corner outside the grid has a tile slot of its
+    // own, which no cell reads)
+    if (static_cast<unsigned>(lx0) < static_cast<unsigned>(kTileX - 1) &&
+        static_cast<unsigned>(ly0) < static_cast<unsigned>(kTileY - 1) &&
+        static_cast<unsigned>(lz0) < static_cast<unsigned>(kTileZ - 1)) {
+      double* t = tile + (lz0 * kTileY + ly0) * kTileX + lx0;
 #pragma unroll
-  for (int k = 0; k < 4; ++k) {
-    const int bx = k & 1, by = k >> 1;
-    const float w0 = wx[bx] * wy[by] * wz[0], w1 = wx[bx] * wy[by] * wz[1];
-#pragma unroll
-    for (int i = 0; i < C; ++i) {
-      lo[k].v[i] = val.v[i] * w0;
-      hi[k].v[i] = val.v[i] * w1;
+      for (int k = 0; k < 8; ++k) {
+        const int bx = k & 1, by = (k >> 1) & 1, bz = k >> 2;
+        lds_add(t + (bz * kTileY + by) * kTileX + bx, val * (fw[bx][0] * fw[by][1] * fw[bz][2]));
+      }
+      return;
     }
   }
-  if (in_tile) {
-    if (held.base == base0 && held.dx == dx && held.dy == dy) {
-#pragma unroll
-      for (int k = 0; k < 4; ++k)
-#pragma unroll
-        for (int i = 0; i < C; ++i) lo[k].v[i] += held.v[k].v[i];
-    } else if (held.base >= 0) {
-      plane_add<C>(tile, held.base, held.dx, held.dy, held.v);
-    }
-  }
-  plane_add_row_merged<C>(tile, in_tile, base0, dx, dy, lo);
-  if (in_tile) {
-    held.base = base1;
-    held.dx = dx;
-    held.dy = dy;
-#pragma unroll
-    for (int k = 0; k < 4; ++k) held.v[k] = hi[k];
-    return;
-  }
-  if (!inside) return;
 #pragma unroll
   for (int k = 0; k < 8; ++k) {
     const int bx = k & 1, by = (k >> 1) & 1, bz = (k >> 2) & 1;
@@ -547,19 +416,16 @@ NGT_DEVICE void scatter_linear_tile(float* tile, HeldPlane<C>& held, bool on, in
     if (static_cast<unsigned>(lx) < static_cast<unsigned>(kTileX) &&
         static_cast<unsigned>(ly) < static_cast<unsigned>(kTileY) &&
         static_cast<unsigned>(lz) < static_cast<unsigned>(kTileZ)) {
-      float* t = tile + ((lz * kTileY + ly) * kTileX + lx) * C;
-#pragma unroll
-      for (int i = 0; i < C; ++i) lds_add(t + i, val.v[i] * w);
+      lds_add(tile + (lz * kTileY + ly) * kTileX + lx, val * w);
     } else {
-      const int64_t o = cell_offset(d, ix, iy, iz);
-#pragma unroll
-      for (int i = 0; i < C; ++i) atomic_add(ovf + o * C + i, val.v[i] * w);
+      atomic_add(ovf + cell_offset(d, ix, iy, iz) * ovf_step, val * w);
     }
   }
 }
 
 // Sum of the tile partials of `slot` covering cell (x, y, z), bricks in
-// ascending z, y, x order.
+// ascending z, y, x order.  A brick's partials hold its channels one after
+// another.
 template <int C>
 NGT_DEVICE Vec<C> gather_tiles(const float* __restrict__ tiles, int64_t slot, const BrickGrid& bg, int x, int y,
                                int z) {
@@ -578,7 +444,9 @@ NGT_DEVICE Vec<C> gather_tiles(const float* __restrict__ tiles, int64_t slot, co
     t[q] = vzero<C>();
     if (ok[q]) {
       const int64_t brick = (slot * bg.nz + bz) * bg.ny * bg.nx + static_cast<int64_t>(by) * bg.nx + bx;
-      t[q] = vload<C>(tiles + (brick * kTileCells + (lz * kTileY + ly) * kTileX + lx) * C);
+      const float* p = tiles + brick * (kTileCells * C) + (lz * kTileY + ly) * kTileX + lx;
+#pragma unroll
+      for (int i = 0; i < C; ++i) t[q].v[i] = p[i * kTileCells];
     }
   }
   Vec<C> s = vzero<C>();
@@ -609,189 +477,198 @@ NGT_DEVICE BrickCell brick_cell(const BrickGrid& bg, const VBlock& vb) {
   return b;
 }
 
-template <int C>
-NGT_DEVICE void tile_clear(float* tile) {
-  const int tid = (threadIdx.z * kBrickY + threadIdx.y) * kBrickX + threadIdx.x;
-  for (int i = tid; i < kTileCells * C; i += kBrickThreads) tile[i] = 0.f;
+NGT_DEVICE int brick_thread() { return (threadIdx.z * kBrickY + threadIdx.y) * kBrickX + threadIdx.x; }
+
+NGT_DEVICE void tile_clear(double* tile) {
+  for (int i = brick_thread(); i < kTileCells; i += kBrickThreads) tile[i] = 0.0;
   __syncthreads();
 }
 
+// The finished tile of channel c to the brick's partials; with `again` the
+// tile is empty for the next channel.
 template <int C>
-NGT_DEVICE void tile_store(const float* tile, float* __restrict__ tiles, const BrickGrid& bg, const BrickCell& b) {
+NGT_DEVICE void tile_store(double* tile, float* __restrict__ tiles, const BrickGrid& bg, const BrickCell& b, int c,
+                           bool again) {
   __syncthreads();
-  const int tid = (threadIdx.z * kBrickY + threadIdx.y) * kBrickX + threadIdx.x;
-  float* dst = tiles + (static_cast<int64_t>(b.pair) * bg.count() + b.brick) * kTileCells * C;
-  for (int i = tid; i < kTileCells * C; i += kBrickThreads) dst[i] = tile[i];
+  float* dst = tiles + ((static_cast<int64_t>(b.pair) * bg.count() + b.brick) * C + c) * kTileCells;
+  for (int i = brick_thread(); i < kTileCells; i += kBrickThreads) {
+    dst[i] = static_cast<float>(tile[i]);
+    if (again) tile[i] = 0.0;
+  }
+  if (again) __syncthreads();
 }
 
 // Velocity-gradient contribution of one cell: plain store / read-add-store
 // when each velocity has one (data, velocity) pair, atomics when several
 // pairs share it.
-NGT_DEVICE void add_vel_grad(float* gv, float gx, float gy, float gz, int mode) {
+NGT_DEVICE void add_vel_grad(const GradVel& gv, int v, int64_t cell, float gx, float gy, float gz, int mode) {
+  float* px = gv.at(v, cell, 0);
+  float* py = gv.at(v, cell, 1);
+  float* pz = gv.at(v, cell, 2);
   if (mode == 0) {
-    gv[0] = gx; gv[1] = gy; gv[2] = gz;
+    *px = gx; *py = gy; *pz = gz;
   } else if (mode == 1) {
-    gv[0] += gx; gv[1] += gy; gv[2] += gz;
+    *px += gx; *py += gy; *pz += gz;
   } else {
-    atomic_add(gv + 0, gx); atomic_add(gv + 1, gy); atomic_add(gv + 2, gz);
+    atomic_add(px, gx); atomic_add(py, gy); atomic_add(pz, gz);
+  }
+}
+
+// Visits the work-item's cells of the brick: f(cell, z, displacement).
+template <typename F>
+NGT_DEVICE void for_brick_cells(const AdvArgs& a, const BrickCell& b, int v, F&& f) {
+  if (b.x >= a.d.x || b.y >= a.d.y) return;
+  const int zb = b.z0 + static_cast<int>(threadIdx.z) * kBrickZPer;
+  const int z1 = min(zb + kBrickZPer, a.d.z);
+#pragma unroll 1
+  for (int z = zb; z < z1; ++z) {
+    float ux, uy, uz;
+    load_velocity(a, v, b.x, b.y, z, ux, uy, uz);
+    f(cell_offset(a.d, b.x, b.y, z), z, a.ts * ux, a.ts * uy, a.ts * uz);
   }
 }
 
 // B1 brick form: g_dir = g (direct path to the SL field), r_dir = g/2 where the
 // corrected value is kept (direct path to rho), the back-step adjoint into
 // the tile (overflow into ovf), and the back-step velocity gradient.
+// Several channels: the first walk forms and stores everything, and each
+// channel then scatters in a walk of its own, from the r_dir that its own
+// work-item stored.
 template <int C, int BM, int CLAMPM>
 NGT_DEVICE void advect_mc_bwd_brick_kernel_body(const VBlock& vb, const AdvArgs& a, BrickGrid bg, const float* __restrict__ rho,
-                                                                  const float* __restrict__ sl,
-                                                                  const float* __restrict__ g_out,
-                                                                  float* __restrict__ g_dir, float* __restrict__ r_dir,
-                                                                  float* __restrict__ ovf, float* __restrict__ tiles,
-                                                                  float* __restrict__ g_vc, int vel_mode) {
-  __shared__ float tile[kTileCells * C];
-  tile_clear<C>(tile);
+                                                const float* __restrict__ sl, const float* __restrict__ g_out,
+                                                float* __restrict__ g_dir, float* r_dir, float* __restrict__ ovf,
+                                                float* __restrict__ tiles, const GradVel& gv, int vel_mode) {
+  __shared__ double tile[kTileCells];
+  tile_clear(tile);
   const BrickCell b = brick_cell(bg, vb);
   int n, v;
   pair_indices(a, b.pair, n, v);
   const int64_t cells = static_cast<int64_t>(a.d.x) * a.d.y * a.d.z;
   const float* src = rho + n * cells * C;
   const float* slp = sl + b.pair * cells * C;
+  const float fx = static_cast<float>(b.x), fy = static_cast<float>(b.y);
+  float* rdp = r_dir + b.pair * cells * C;
   float* ovp = ovf + b.pair * cells * C;
-  // every lane of the wave runs the walk (the tile scatter exchanges values
-  // between neighbouring lanes): a lane outside the grid reads its clamped
-  // edge cell, stores nothing and scatters nothing
-  const bool lane_ok = b.x < a.d.x && b.y < a.d.y;
-  const int cx = min(b.x, a.d.x - 1), cy = min(b.y, a.d.y - 1);
-  {
-    const int zb = b.z0 + static_cast<int>(threadIdx.z) * kBrickZPer;
-    const int z1 = min(zb + kBrickZPer, a.d.z);
-    HeldPlane<C> held;
-#pragma unroll 2
-    for (int z = zb; z < z1; ++z) {
-      float ux, uy, uz;
-      load_velocity(a, v, cx, cy, z, ux, uy, uz);
-      const int64_t cell = cell_offset(a.d, cx, cy, z);
-      const float fx = static_cast<float>(cx), fy = static_cast<float>(cy), fz = static_cast<float>(z);
-      const float tx = a.ts * ux, ty = a.ts * uy, tz = a.ts * uz;
-      const float bx = fx + (-tx), by = fy + (-ty), bz = fz + (-tz);
-      Vec<C> g = vload<C>(g_out + (b.pair * cells + cell) * C);
-      const Vec<C> fwd = vload<C>(slp + cell * C);
-      // the back-step read and its position gradient share one corner fetch
-      Vec<C> dx, dy, dz;
-      const Vec<C> back = read_linear_gradient<C, BM>(slp, a.d, bx, by, bz, dx, dy, dz);
-      const Vec<C> cur = vload<C>(src + cell * C);
-      Vec<C> corr;
+  for_brick_cells(a, b, v, [&](int64_t cell, int z, float tx, float ty, float tz) {
+    const float fz = static_cast<float>(z);
+    const float bx = fx + (-tx), by = fy + (-ty), bz = fz + (-tz);
+    Vec<C> g = vload<C>(g_out + (b.pair * cells + cell) * C);
+    const Vec<C> fwd = vload<C>(slp + cell * C);
+    // the back-step read and its position gradient share one corner fetch
+    Vec<C> dx, dy, dz;
+    const Vec<C> back = read_linear_gradient<C, BM>(slp, a.d, bx, by, bz, dx, dy, dz);
+    const Vec<C> cur = vload<C>(src + cell * C);
+    Vec<C> corr;
 #pragma unroll
-      for (int i = 0; i < C; ++i) corr.v[i] = fwd.v[i] + 0.5f * (cur.v[i] - back.v[i]);
-      Vec<C> keep = vfill<C>(1.f);
-      if constexpr (CLAMPM == NGT_CLAMP_MC_SMOOTH) {
-        Vec<C> mn, mx;
-        read_minmax2<C, BM>(src, a.d, fx + tx, fy + ty, fz + tz, mn, mx);
+    for (int i = 0; i < C; ++i) corr.v[i] = fwd.v[i] + 0.5f * (cur.v[i] - back.v[i]);
+    Vec<C> keep = vfill<C>(1.f);
+    if constexpr (CLAMPM == NGT_CLAMP_MC_SMOOTH) {
+      Vec<C> mn, mx;
+      read_minmax2<C, BM>(src, a.d, fx + tx, fy + ty, fz + tz, mn, mx);
 #pragma unroll
-        for (int i = 0; i < C; ++i)
-          if (corr.v[i] < mn.v[i] || corr.v[i] > mx.v[i]) keep.v[i] = 0.f;
-      }
-      if constexpr (CLAMPM == NGT_CLAMP_NEGATIVE) {
-#pragma unroll
-        for (int i = 0; i < C; ++i)
-          if (!(corr.v[i] >= 0.f)) g.v[i] = 0.f;
-      }
-      Vec<C> rd, gback;
-#pragma unroll
-      for (int i = 0; i < C; ++i) {
-        rd.v[i] = 0.5f * keep.v[i] * g.v[i];
-        gback.v[i] = -rd.v[i];
-      }
-      if (lane_ok) {
-        if (g_dir) vstore<C>(g_dir + (b.pair * cells + cell) * C, g);
-        vstore<C>(r_dir + (b.pair * cells + cell) * C, rd);
-        add_vel_grad(g_vc + (static_cast<int64_t>(v) * cells + cell) * 3, -a.ts * vdot(gback, dx),
-                     -a.ts * vdot(gback, dy), -a.ts * vdot(gback, dz), vel_mode == 1 ? 0 : vel_mode);
-      }
-      scatter_linear_tile<C, BM>(tile, held, lane_ok, b.ox, b.oy, b.oz, ovp, a.d, bx, by, bz, gback);
+      for (int i = 0; i < C; ++i)
+        if (corr.v[i] < mn.v[i] || corr.v[i] > mx.v[i]) keep.v[i] = 0.f;
     }
-    flush_plane<C>(tile, held);
+    if constexpr (CLAMPM == NGT_CLAMP_NEGATIVE) {
+#pragma unroll
+      for (int i = 0; i < C; ++i)
+        if (!(corr.v[i] >= 0.f)) g.v[i] = 0.f;
+    }
+    Vec<C> rd, gback;
+#pragma unroll
+    for (int i = 0; i < C; ++i) {
+      rd.v[i] = 0.5f * keep.v[i] * g.v[i];
+      gback.v[i] = -rd.v[i];
+    }
+    if (g_dir) vstore<C>(g_dir + (b.pair * cells + cell) * C, g);
+    vstore<C>(rdp + cell * C, rd);
+    add_vel_grad(gv, v, cell, -a.ts * vdot(gback, dx), -a.ts * vdot(gback, dy), -a.ts * vdot(gback, dz),
+                 vel_mode == 1 ? 0 : vel_mode);
+    if constexpr (C == 1) scatter_linear_tile<BM>(tile, b.ox, b.oy, b.oz, ovp, 1, a.d, bx, by, bz, gback.v[0]);
+  });
+  if constexpr (C == 1) {
+    tile_store<C>(tile, tiles, bg, b, 0, false);
+  } else {
+    for (int c = 0; c < C; ++c) {
+      for_brick_cells(a, b, v, [&](int64_t cell, int z, float tx, float ty, float tz) {
+        scatter_linear_tile<BM>(tile, b.ox, b.oy, b.oz, ovp + c, C, a.d, fx + (-tx), fy + (-ty),
+                                static_cast<float>(z) + (-tz), -rdp[cell * C + c]);
+      });
+      tile_store<C>(tile, tiles, bg, b, c, c + 1 < C);
+    }
   }
-  tile_store<C>(tile, tiles, bg, b);
 }
 
 template <int C, int BM, int CLAMPM>
-__global__ __launch_bounds__(kBrickThreads) void advect_mc_bwd_brick_kernel(AdvArgs a, BrickGrid bg, const float* __restrict__ rho,
-                                                                  const float* __restrict__ sl,
-                                                                  const float* __restrict__ g_out,
-                                                                  float* __restrict__ g_dir, float* __restrict__ r_dir,
-                                                                  float* __restrict__ ovf, float* __restrict__ tiles,
-                                                                  float* __restrict__ g_vc, int vel_mode) {
-  advect_mc_bwd_brick_kernel_body<C, BM, CLAMPM>(VBlock{static_cast<int>(blockIdx.x), static_cast<int>(blockIdx.y), static_cast<int>(blockIdx.z)}, a, bg, rho, sl, g_out, g_dir, r_dir, ovf, tiles, g_vc, vel_mode);
+__global__ __launch_bounds__(kBrickThreads) void advect_mc_bwd_brick_kernel(
+    AdvArgs a, BrickGrid bg, const float* __restrict__ rho, const float* __restrict__ sl,
+    const float* __restrict__ g_out, float* __restrict__ g_dir, float* r_dir, float* __restrict__ ovf,
+    float* __restrict__ tiles, GradVel gv, int vel_mode) {
+  advect_mc_bwd_brick_kernel_body<C, BM, CLAMPM>(VBlock{static_cast<int>(blockIdx.x), 0, 0}, a, bg, rho, sl, g_out,
+                                                 g_dir, r_dir, ovf, tiles, gv, vel_mode);
 }
 
 // B2 brick form: g_sl = g_dir + ovf + tiles1 (order 2) or g_out with the
 // NEGATIVE mask (order 1); scatter into the tile (overflow straight into
-// g_rho, which starts at zero), SL velocity gradient.
+// g_rho, which starts at zero), SL velocity gradient.  Several channels: g_sl
+// is stored to `val` and scattered channel by channel, as in B1.
 template <int C, int BM, bool NEG, bool ORDER2>
 NGT_DEVICE void advect_sl_bwd_brick_kernel_body(const VBlock& vb, const AdvArgs& a, BrickGrid bg, const float* __restrict__ rho,
-                                                                  const float* __restrict__ g_in,
-                                                                  const float* __restrict__ ovf1,
-                                                                  const float* __restrict__ tiles1,
-                                                                  float* __restrict__ g_rho, float* __restrict__ tiles2,
-                                                                  float* __restrict__ g_vc, int vel_mode) {
-  __shared__ float tile[kTileCells * C];
-  tile_clear<C>(tile);
+                                                const float* g_in, const float* __restrict__ ovf1,
+                                                const float* __restrict__ tiles1, float* __restrict__ g_rho,
+                                                float* __restrict__ tiles2, const GradVel& gv, int vel_mode,
+                                                float* val) {
+  __shared__ double tile[kTileCells];
+  tile_clear(tile);
   const BrickCell b = brick_cell(bg, vb);
   int n, v;
   pair_indices(a, b.pair, n, v);
   const int64_t cells = static_cast<int64_t>(a.d.x) * a.d.y * a.d.z;
   const float* src = rho + n * cells * C;
   float* ovp = g_rho + n * cells * C;
-  // every lane of the wave runs the walk (the tile scatter exchanges values
-  // between neighbouring lanes): a lane outside the grid reads its clamped
-  // edge cell, stores nothing and scatters nothing
-  const bool lane_ok = b.x < a.d.x && b.y < a.d.y;
-  const int cx = min(b.x, a.d.x - 1), cy = min(b.y, a.d.y - 1);
-  {
-    const int zb = b.z0 + static_cast<int>(threadIdx.z) * kBrickZPer;
-    const int z1 = min(zb + kBrickZPer, a.d.z);
-    HeldPlane<C> held;
-#pragma unroll 2
-    for (int z = zb; z < z1; ++z) {
-      float ux, uy, uz;
-      load_velocity(a, v, cx, cy, z, ux, uy, uz);
-      const int64_t cell = cell_offset(a.d, cx, cy, z);
-      const float px = static_cast<float>(cx) + a.ts * ux;
-      const float py = static_cast<float>(cy) + a.ts * uy;
-      const float pz = static_cast<float>(z) + a.ts * uz;
-      Vec<C> g = vload<C>(g_in + (b.pair * cells + cell) * C);
-      if constexpr (ORDER2) {
-        const Vec<C> o = vload<C>(ovf1 + (b.pair * cells + cell) * C);
-        const Vec<C> t = gather_tiles<C>(tiles1, b.pair, bg, cx, cy, z);
+  const float fx = static_cast<float>(b.x), fy = static_cast<float>(b.y);
+  for_brick_cells(a, b, v, [&](int64_t cell, int z, float tx, float ty, float tz) {
+    const float px = fx + tx, py = fy + ty, pz = static_cast<float>(z) + tz;
+    Vec<C> g = vload<C>(g_in + (b.pair * cells + cell) * C);
+    if constexpr (ORDER2) {
+      const Vec<C> o = vload<C>(ovf1 + (b.pair * cells + cell) * C);
+      const Vec<C> t = gather_tiles<C>(tiles1, b.pair, bg, b.x, b.y, z);
 #pragma unroll
-        for (int i = 0; i < C; ++i) g.v[i] += o.v[i] + t.v[i];
-      }
-      if constexpr (NEG) {
-        const Vec<C> r = read_linear<C, BM>(src, a.d, px, py, pz);
-#pragma unroll
-        for (int i = 0; i < C; ++i)
-          if (!(r.v[i] >= 0.f)) g.v[i] = 0.f;
-      }
-      scatter_linear_tile<C, BM>(tile, held, lane_ok, b.ox, b.oy, b.oz, ovp, a.d, px, py, pz, g);
-      Vec<C> dx, dy, dz;
-      read_gradient<C, BM>(src, a.d, px, py, pz, dx, dy, dz);
-      if (lane_ok)
-        add_vel_grad(g_vc + (static_cast<int64_t>(v) * cells + cell) * 3, a.ts * vdot(g, dx), a.ts * vdot(g, dy),
-                     a.ts * vdot(g, dz), vel_mode);
+      for (int i = 0; i < C; ++i) g.v[i] += o.v[i] + t.v[i];
     }
-    flush_plane<C>(tile, held);
+    if constexpr (NEG) {
+      const Vec<C> r = read_linear<C, BM>(src, a.d, px, py, pz);
+#pragma unroll
+      for (int i = 0; i < C; ++i)
+        if (!(r.v[i] >= 0.f)) g.v[i] = 0.f;
+    }
+    if constexpr (C == 1) scatter_linear_tile<BM>(tile, b.ox, b.oy, b.oz, ovp, 1, a.d, px, py, pz, g.v[0]);
+    else vstore<C>(val + (b.pair * cells + cell) * C, g);
+    Vec<C> dx, dy, dz;
+    read_gradient<C, BM>(src, a.d, px, py, pz, dx, dy, dz);
+    add_vel_grad(gv, v, cell, a.ts * vdot(g, dx), a.ts * vdot(g, dy), a.ts * vdot(g, dz), vel_mode);
+  });
+  if constexpr (C == 1) {
+    tile_store<C>(tile, tiles2, bg, b, 0, false);
+  } else {
+    for (int c = 0; c < C; ++c) {
+      for_brick_cells(a, b, v, [&](int64_t cell, int z, float tx, float ty, float tz) {
+        scatter_linear_tile<BM>(tile, b.ox, b.oy, b.oz, ovp + c, C, a.d, fx + tx, fy + ty, static_cast<float>(z) + tz,
+                                val[(b.pair * cells + cell) * C + c]);
+      });
+      tile_store<C>(tile, tiles2, bg, b, c, c + 1 < C);
+    }
   }
-  tile_store<C>(tile, tiles2, bg, b);
 }
 
 template <int C, int BM, bool NEG, bool ORDER2>
-__global__ __launch_bounds__(kBrickThreads) void advect_sl_bwd_brick_kernel(AdvArgs a, BrickGrid bg, const float* __restrict__ rho,
-                                                                  const float* __restrict__ g_in,
-                                                                  const float* __restrict__ ovf1,
-                                                                  const float* __restrict__ tiles1,
-                                                                  float* __restrict__ g_rho, float* __restrict__ tiles2,
-                                                                  float* __restrict__ g_vc, int vel_mode) {
-  advect_sl_bwd_brick_kernel_body<C, BM, NEG, ORDER2>(VBlock{static_cast<int>(blockIdx.x), static_cast<int>(blockIdx.y), static_cast<int>(blockIdx.z)}, a, bg, rho, g_in, ovf1, tiles1, g_rho, tiles2, g_vc, vel_mode);
+__global__ __launch_bounds__(kBrickThreads) void advect_sl_bwd_brick_kernel(
+    AdvArgs a, BrickGrid bg, const float* __restrict__ rho, const float* g_in, const float* __restrict__ ovf1,
+    const float* __restrict__ tiles1, float* __restrict__ g_rho, float* __restrict__ tiles2, GradVel gv, int vel_mode,
+    float* val) {
+  advect_sl_bwd_brick_kernel_body<C, BM, NEG, ORDER2>(VBlock{static_cast<int>(blockIdx.x), 0, 0}, a, bg, rho, g_in,
+                                                      ovf1, tiles1, g_rho, tiles2, gv, vel_mode, val);
 }
 
 // g_rho(n) += sum over the pairs of n of r_dir (order 2) + the B2 tiles.
@@ -830,16 +707,16 @@ __global__ __launch_bounds__(256) void advect_rho_gather_kernel(AdvArgs a, Brick
 }
 
 // The MAC face gradients that cell (x, y, z) owns, from the centered velocity
-// gradient g (3 per cell): its lower face on each axis, and the upper one at
+// gradient: its lower face on each axis, and the upper one at
 // the grid's far side.  The same sums as faces_from_centered_grad_kernel.
-NGT_DEVICE void faces_of_cell(const Dims& d, const float* __restrict__ g, float* __restrict__ ox,
+NGT_DEVICE void faces_of_cell(const Dims& d, const GradVel& gv, float* __restrict__ ox,
                               float* __restrict__ oy, float* __restrict__ oz, int x, int y, int z) {
   const int64_t plane = static_cast<int64_t>(d.x) * d.y;
   const int64_t c = cell_offset(d, x, y, z);
-  const float g0 = g[c * 3 + 0], g1 = g[c * 3 + 1], g2 = g[c * 3 + 2];
-  const float l0 = x > 0 ? g[(c - 1) * 3 + 0] : 0.f;
-  const float l1 = y > 0 ? g[(c - d.x) * 3 + 1] : 0.f;
-  const float l2 = z > 0 ? g[(c - plane) * 3 + 2] : 0.f;
+  const float g0 = *gv.at(0, c, 0), g1 = *gv.at(0, c, 1), g2 = *gv.at(0, c, 2);
+  const float l0 = x > 0 ? *gv.at(0, c - 1, 0) : 0.f;
+  const float l1 = y > 0 ? *gv.at(0, c - d.x, 1) : 0.f;
+  const float l2 = z > 0 ? *gv.at(0, c - plane, 2) : 0.f;
   const int64_t fx = (static_cast<int64_t>(z) * d.y + y) * (d.x + 1) + x;
   ox[fx] = 0.5f * (l0 + g0);
   if (x == d.x - 1) ox[fx + 1] = 0.5f * g0;
@@ -855,14 +732,14 @@ NGT_DEVICE void faces_of_cell(const Dims& d, const float* __restrict__ g, float*
 template <int C>
 __global__ __launch_bounds__(256) void advect_rho_faces_kernel(AdvArgs a, BrickGrid bg, const float* __restrict__ r_dir,
                                                                const float* __restrict__ tiles2,
-                                                               float* __restrict__ g_rho,
-                                                               const float* __restrict__ g_vc, float* __restrict__ gx,
+                                                               float* __restrict__ g_rho, GradVel gv,
+                                                               float* __restrict__ gx,
                                                                float* __restrict__ gy, float* __restrict__ gz) {
   const VBlock vb{static_cast<int>(blockIdx.x), static_cast<int>(blockIdx.y), static_cast<int>(blockIdx.z)};
   advect_rho_gather_kernel_body<C>(vb, a, bg, r_dir, tiles2, g_rho);
   const int x = vb.x * kBX + static_cast<int>(threadIdx.x), y = vb.y * kBY + static_cast<int>(threadIdx.y);
   if (x >= a.d.x || y >= a.d.y) return;
-  faces_of_cell(a.d, g_vc, gx, gy, gz, x, y, vb.z);
+  faces_of_cell(a.d, gv, gx, gy, gz, x, y, vb.z);
 }
 
 #define NGT_SWITCH_C(C_, ...)                              \
@@ -871,11 +748,6 @@ __global__ __launch_bounds__(256) void advect_rho_faces_kernel(AdvArgs a, BrickG
     case 2: { constexpr int CC = 2; __VA_ARGS__; } break;  \
     case 3: { constexpr int CC = 3; __VA_ARGS__; } break;  \
     default: { constexpr int CC = 4; __VA_ARGS__; } break; \
-  }
-#define NGT_SWITCH_C12(C_, ...)                           \
-  switch (C_) {                                           \
-    case 1: { constexpr int CC = 1; __VA_ARGS__; } break; \
-    default: { constexpr int CC = 2; __VA_ARGS__; } break; \
   }
 #define NGT_SWITCH_BM(B_, ...)                                      \
   switch (B_) {                                                     \
@@ -930,10 +802,10 @@ dim3 adv_grid(const AdvPlan& p) {
   return dim3(blocks_for(p.a.d.x, kBX), blocks_for(p.a.d.y, kBY), static_cast<unsigned>(p.a.d.z * p.pairs));
 }
 
-void launch_faces(const AdvPlan& p, const float* g_vc, float* gx, float* gy, float* gz, hipStream_t s) {
+void launch_faces(const AdvPlan& p, const GradVel& gv, float* gx, float* gy, float* gz, hipStream_t s) {
   const Dims d = p.a.d;
   hipLaunchKernelGGL(faces_from_centered_grad_kernel, dim3(static_cast<unsigned>(face_tiles(d) * p.a.n_vel)), dim3(256),
-                     0, s, d, p.a.n_vel, g_vc, gx, gy, gz);
+                     0, s, d, p.a.n_vel, gv, gx, gy, gz);
 }
 
 // ---------------------------------------------------------------------------
@@ -1087,13 +959,13 @@ __global__ __launch_bounds__(kBrickThreads) void advect_mc_bwd_batch_kernel(cons
     const int i = __builtin_amdgcn_readfirstlane(find_item(v.brick, v.h->n, t));
     const AdvBatchItem& it = v.items[i];
     const AdvBatchBufs b = batch_bufs(it);
-    float* g_vc = v.h->staggered ? ws + it.ws_gvc : b.gvx;
+    const GradVel gv{v.h->staggered ? ws + it.ws_gvc : b.gvx, it.cells, 3};
     // the direct rho term goes straight to input_grad; the masked output
     // gradient is kept only where NEGATIVE changes it
     advect_mc_bwd_brick_kernel_body<1, BM, CLAMPM>(VBlock{t - v.brick[i], 0, 0}, b.a, it.bg, b.input, b.sl,
                                                    b.g_out,
                                                    CLAMPM == NGT_CLAMP_NEGATIVE ? ws + it.ws_gsl : nullptr,
-                                                   b.g_in, ws + it.ws_ovf, ws + it.ws_t1, g_vc, 1);
+                                                   b.g_in, ws + it.ws_ovf, ws + it.ws_t1, gv, 1);
     __syncthreads();  // the LDS tile is cleared again by the next brick
   }
 }
@@ -1105,11 +977,12 @@ __global__ __launch_bounds__(kBrickThreads) void advect_sl_bwd_batch_kernel(cons
     const int i = __builtin_amdgcn_readfirstlane(find_item(v.brick, v.h->n, t));
     const AdvBatchItem& it = v.items[i];
     const AdvBatchBufs b = batch_bufs(it);
-    float* g_vc = v.h->staggered ? ws + it.ws_gvc : b.gvx;
+    const GradVel gv{v.h->staggered ? ws + it.ws_gvc : b.gvx, it.cells, 3};
     const float* g = ORDER2 && v.h->clamp == NGT_CLAMP_NEGATIVE ? ws + it.ws_gsl : b.g_out;
     advect_sl_bwd_brick_kernel_body<1, BM, NEG, ORDER2>(VBlock{t - v.brick[i], 0, 0}, b.a, it.bg, b.input,
                                                         g, ws + it.ws_ovf,
-                                                        ws + it.ws_t1, b.g_in, ws + it.ws_t2, g_vc, ORDER2 ? 1 : 0);
+                                                        ws + it.ws_t1, b.g_in, ws + it.ws_t2, gv, ORDER2 ? 1 : 0,
+                                                        nullptr);
     __syncthreads();
   }
 }
@@ -1127,7 +1000,7 @@ __global__ __launch_bounds__(256) void advect_rho_gather_batch_kernel(const void
       advect_rho_gather_kernel_body<1>(vb, it.a, it.bg, nullptr, ws + it.ws_t2, g_in);
       const int x = vb.x * kBX + static_cast<int>(threadIdx.x), y = vb.y * kBY + static_cast<int>(threadIdx.y);
       if (staggered && x < it.a.d.x && y < it.a.d.y)
-        faces_of_cell(it.a.d, ws + it.ws_gvc, (float*)it.gvx, (float*)it.gvy, (float*)it.gvz, x, y, vb.z);
+        faces_of_cell(it.a.d, GradVel{ws + it.ws_gvc, it.cells, 3}, (float*)it.gvx, (float*)it.gvy, (float*)it.gvz, x, y, vb.z);
     });
   }
 }
@@ -1152,13 +1025,10 @@ size_t ngt_advect_workspace_size(const int64_t* input_shape, int num_velocities,
     floats += static_cast<int64_t>(num_velocities) * cells * 3;  // centered velocity gradient
     const int64_t ref_extra = pairs * cells * C          // reference: scatter staging
                               + pairs * cells;           // reference: hit counts (uint32)
-    int64_t brick_extra = 0;
-    if (C <= 2) {
-      const Dims d{static_cast<int>(input_shape[3]), static_cast<int>(input_shape[2]),
-                   static_cast<int>(input_shape[1])};
-      const int64_t tiles = pairs * brick_grid(d).count() * static_cast<int64_t>(kTileCells) * C;
-      brick_extra = tiles + (order == 2 ? 2 * pairs * cells * C + tiles : 0);  // tiles2 (+ r_dir, ovf1, tiles1)
-    }
+    const Dims d{static_cast<int>(input_shape[3]), static_cast<int>(input_shape[2]),
+                 static_cast<int>(input_shape[1])};
+    const int64_t tiles = pairs * brick_grid(d).count() * static_cast<int64_t>(kTileCells) * C;
+    const int64_t brick_extra = tiles + (order == 2 ? 2 * pairs * cells * C + tiles : 0);  // tiles2 (+ r_dir, ovf1, tiles1)
     floats += std::max(ref_extra, brick_extra);
   }
   return static_cast<size_t>(floats) * sizeof(float) + 256;
@@ -1217,7 +1087,7 @@ int ngt_advect_bwd(const float* input, const int64_t* input_shape, const float* 
   float* g_vc = g_sl + field;
   float* tmp = g_vc + static_cast<int64_t>(p.a.n_vel) * p.cells * 3;
   uint32_t* hits = reinterpret_cast<uint32_t*>(tmp + field);
-  if (!p.a.staggered) g_vc = vel_x_grad;  // centered: accumulate in place
+  const GradVel gv{p.a.staggered ? g_vc : vel_x_grad, p.cells, 3};  // centered: accumulated in place
 
   const float* slp = sl;
   if (order == 2 && slp == nullptr) {
@@ -1225,10 +1095,9 @@ int ngt_advect_bwd(const float* input, const int64_t* input_shape, const float* 
         hipLaunchKernelGGL((advect_sl_kernel<CC, BB, false>), grid, block, 0, s, p.a, input, sl_buf)));
     slp = sl_buf;
   }
-  const bool brick_path = !ref && p.C <= 2;
   // the brick path clears (or has B1 store) input_grad in its order-2 branch
-  if (!(brick_path && order == 2)) fill_zero(input_grad, p.a.n_data * p.cells * p.C, s);
-  if (brick_path) {
+  if (ref || order == 1) fill_zero(input_grad, p.a.n_data * p.cells * p.C, s);
+  if (!ref) {
     // brick-tiled exact adjoint: workspace after g_vc = [tiles2 | r_dir | ovf1 | tiles1]
     const BrickGrid bg = brick_grid(p.a.d);
     const int64_t tiles_n = static_cast<int64_t>(p.pairs) * bg.count() * kTileCells * p.C;
@@ -1238,8 +1107,9 @@ int ngt_advect_bwd(const float* input, const int64_t* input_shape, const float* 
     float* tiles1 = ovf1 + field;
     const bool shared_v = p.a.separate && p.a.n_data > 1;
     const int vel_mode = shared_v ? 2 : (order == 2 ? 1 : 0);
-    if (shared_v) fill_zero(g_vc, static_cast<int64_t>(p.a.n_vel) * p.cells * 3, s);
+    if (shared_v) fill_zero(gv.p, static_cast<int64_t>(p.a.n_vel) * p.cells * 3, s);
     const dim3 bgrid(static_cast<unsigned>(bg.count() * p.pairs)), bblock(kBrickX, kBrickY, kBrickZT);
+    float* val = p.C > 1 ? g_sl : nullptr;  // B2's gradient, scattered channel by channel
     const bool neg = order == 1 && clamp == NGT_CLAMP_NEGATIVE;
     // one (data, velocity) pair per data entry: B1 stores the direct rho term
     // straight into input_grad (each cell once, before B2's overflow atomics
@@ -1253,69 +1123,54 @@ int ngt_advect_bwd(const float* input, const int64_t* input_shape, const float* 
       float* g_dir = pass_g ? nullptr : g_sl;
       float* rd = direct ? input_grad : r_dir;
       const float* g_b2 = pass_g ? output_grad : g_sl;
-      NGT_SWITCH_C12(p.C, NGT_SWITCH_BM(boundary, NGT_SWITCH_CLAMP(clamp,
+      NGT_SWITCH_C(p.C, NGT_SWITCH_BM(boundary, NGT_SWITCH_CLAMP(clamp,
           hipLaunchKernelGGL((advect_mc_bwd_brick_kernel<CC, BB, KK>), bgrid, bblock, 0, s, p.a, bg, input, slp,
-                             output_grad, g_dir, rd, ovf1, tiles1, g_vc, vel_mode);
+                             output_grad, g_dir, rd, ovf1, tiles1, gv, vel_mode);
           hipLaunchKernelGGL((advect_sl_bwd_brick_kernel<CC, BB, false, true>), bgrid, bblock, 0, s, p.a, bg, input,
-                             g_b2, ovf1, tiles1, input_grad, tiles2, g_vc, vel_mode))));
+                             g_b2, ovf1, tiles1, input_grad, tiles2, gv, vel_mode, val))));
     } else {
-      NGT_SWITCH_C12(p.C, NGT_SWITCH_BM(boundary,
+      NGT_SWITCH_C(p.C, NGT_SWITCH_BM(boundary,
           if (neg) hipLaunchKernelGGL((advect_sl_bwd_brick_kernel<CC, BB, true, false>), bgrid, bblock, 0, s, p.a, bg,
-                                      input, output_grad, nullptr, nullptr, input_grad, tiles2, g_vc, vel_mode);
+                                      input, output_grad, nullptr, nullptr, input_grad, tiles2, gv, vel_mode,
+                                      val);
           else hipLaunchKernelGGL((advect_sl_bwd_brick_kernel<CC, BB, false, false>), bgrid, bblock, 0, s, p.a, bg,
-                                  input, output_grad, nullptr, nullptr, input_grad, tiles2, g_vc, vel_mode)));
+                                  input, output_grad, nullptr, nullptr, input_grad, tiles2, gv, vel_mode, val)));
     }
     const dim3 dgrid(blocks_for(p.a.d.x, kBX), blocks_for(p.a.d.y, kBY), static_cast<unsigned>(p.a.d.z * p.a.n_data));
     const float* rd_in = order == 2 && !direct ? r_dir : nullptr;
     if (p.a.staggered && p.a.n_data == 1 && p.a.n_vel == 1) {
-      NGT_SWITCH_C12(p.C, hipLaunchKernelGGL((advect_rho_faces_kernel<CC>), dgrid, block, 0, s, p.a, bg, rd_in, tiles2,
-                                             input_grad, g_vc, vel_x_grad, vel_y_grad, vel_z_grad));
+      NGT_SWITCH_C(p.C, hipLaunchKernelGGL((advect_rho_faces_kernel<CC>), dgrid, block, 0, s, p.a, bg, rd_in, tiles2,
+                                             input_grad, gv, vel_x_grad, vel_y_grad, vel_z_grad));
     } else {
-      NGT_SWITCH_C12(p.C, hipLaunchKernelGGL((advect_rho_gather_kernel<CC>), dgrid, block, 0, s, p.a, bg, rd_in, tiles2,
+      NGT_SWITCH_C(p.C, hipLaunchKernelGGL((advect_rho_gather_kernel<CC>), dgrid, block, 0, s, p.a, bg, rd_in, tiles2,
                                              input_grad));
-      if (p.a.staggered) launch_faces(p, g_vc, vel_x_grad, vel_y_grad, vel_z_grad, s);
+      if (p.a.staggered) launch_faces(p, gv, vel_x_grad, vel_y_grad, vel_z_grad, s);
     }
     return check_launch("ngt_advect_bwd");
   }
-  fill_zero(g_vc, static_cast<int64_t>(p.a.n_vel) * p.cells * 3, s);
+  // reference semantics: scatter into tmp with hit counts, normalised per step
+  fill_zero(gv.p, static_cast<int64_t>(p.a.n_vel) * p.cells * 3, s);
   const float* gsl_in = output_grad;
   if (order == 2) {
     fill_zero(g_sl, field, s);
-    if (ref) {
-      fill_zero(tmp, field, s);
-      fill_zero_u32(hits, p.pairs * p.cells, s);
-    }
-    NGT_SWITCH_C(p.C, NGT_SWITCH_BM(boundary, NGT_SWITCH_CLAMP(clamp,
-        if (ref) hipLaunchKernelGGL((advect_mc_bwd_kernel<CC, BB, KK, true>), grid, block, 0, s, p.a, input, slp,
-                                    output_grad, g_sl, input_grad, g_vc, tmp, hits);
-        else hipLaunchKernelGGL((advect_mc_bwd_kernel<CC, BB, KK, false>), grid, block, 0, s, p.a, input, slp,
-                                output_grad, g_sl, input_grad, g_vc, tmp, hits))));
-    if (ref) {
-      NGT_SWITCH_C(p.C, hipLaunchKernelGGL((add_normalized_kernel<CC>), grid, block, 0, s, p.a, tmp, hits, g_sl, 0));
-    }
-    gsl_in = g_sl;
-  }
-  if (ref) {
     fill_zero(tmp, field, s);
     fill_zero_u32(hits, p.pairs * p.cells, s);
+    NGT_SWITCH_C(p.C, NGT_SWITCH_BM(boundary, NGT_SWITCH_CLAMP(clamp,
+        hipLaunchKernelGGL((advect_mc_bwd_kernel<CC, BB, KK>), grid, block, 0, s, p.a, input, slp, output_grad, g_sl,
+                           input_grad, gv, tmp, hits))));
+    NGT_SWITCH_C(p.C, hipLaunchKernelGGL((add_normalized_kernel<CC>), grid, block, 0, s, p.a, tmp, hits, g_sl, 0));
+    gsl_in = g_sl;
   }
+  fill_zero(tmp, field, s);
+  fill_zero_u32(hits, p.pairs * p.cells, s);
   const bool neg = order == 1 && clamp == NGT_CLAMP_NEGATIVE;
   NGT_SWITCH_C(p.C, NGT_SWITCH_BM(boundary,
-      if (neg) {
-        if (ref) hipLaunchKernelGGL((advect_sl_bwd_kernel<CC, BB, true, true>), grid, block, 0, s, p.a, input, gsl_in,
-                                    nullptr, input_grad, g_vc, tmp, hits);
-        else hipLaunchKernelGGL((advect_sl_bwd_kernel<CC, BB, true, false>), grid, block, 0, s, p.a, input, gsl_in,
-                                nullptr, input_grad, g_vc, tmp, hits);
-      } else {
-        if (ref) hipLaunchKernelGGL((advect_sl_bwd_kernel<CC, BB, false, true>), grid, block, 0, s, p.a, input,
-                                    gsl_in, nullptr, input_grad, g_vc, tmp, hits);
-        else hipLaunchKernelGGL((advect_sl_bwd_kernel<CC, BB, false, false>), grid, block, 0, s, p.a, input, gsl_in,
-                                nullptr, input_grad, g_vc, tmp, hits);
-      }));
-  if (ref) {
-    NGT_SWITCH_C(p.C, hipLaunchKernelGGL((add_normalized_kernel<CC>), grid, block, 0, s, p.a, tmp, hits, input_grad, 1));
-  }
-  if (p.a.staggered) launch_faces(p, g_vc, vel_x_grad, vel_y_grad, vel_z_grad, s);
+      if (neg) hipLaunchKernelGGL((advect_sl_bwd_kernel<CC, BB, true>), grid, block, 0, s, p.a, input, gsl_in, gv, tmp,
+                                  hits);
+      else hipLaunchKernelGGL((advect_sl_bwd_kernel<CC, BB, false>), grid, block, 0, s, p.a, input, gsl_in, gv, tmp,
+                              hits)));
+  NGT_SWITCH_C(p.C, hipLaunchKernelGGL((add_normalized_kernel<CC>), grid, block, 0, s, p.a, tmp, hits, input_grad, 1));
+  if (p.a.staggered) launch_faces(p, gv, vel_x_grad, vel_y_grad, vel_z_grad, s);
   return check_launch("ngt_advect_bwd");
 }
 
