@@ -75,6 +75,49 @@ NGT_DEVICE void load_velocity(const AdvArgs& a, int v, int x, int y, int z, floa
   }
 }
 
+// The velocity along a z column: its addresses are formed once and stepped
+// from plane to plane.
+struct VelocityColumn {
+  const float *px, *py, *pz;   // lower faces of the cell, or px = its vector (centered)
+  int64_t sx, sy, sz;          // plane steps
+  int row;                     // d.x
+  int staggered;
+
+  NGT_DEVICE VelocityColumn(const AdvArgs& a, int v, int x, int y, int z) {
+    const Dims& d = a.d;
+    const int64_t plane = static_cast<int64_t>(d.y) * d.x;
+    row = d.x;
+    staggered = a.staggered;
+    sz = plane;
+    if (!staggered) {
+      sx = 3 * plane;
+      sy = 0;
+      px = a.vx + (static_cast<int64_t>(v) * d.z * plane + cell_offset(d, x, y, z)) * 3;
+      py = pz = nullptr;
+    } else {
+      sx = plane + d.y;
+      sy = plane + d.x;
+      const int64_t vz = static_cast<int64_t>(v) * d.z + z;
+      px = a.vx + vz * sx + static_cast<int64_t>(y) * (d.x + 1) + x;
+      py = a.vy + vz * sy + static_cast<int64_t>(y) * d.x + x;
+      pz = a.vz + (vz + v) * plane + static_cast<int64_t>(y) * d.x + x;
+    }
+  }
+  // the cell's velocity; moves on to the next plane
+  NGT_DEVICE void next(float& ux, float& uy, float& uz) {
+    if (!staggered) {
+      ux = px[0]; uy = px[1]; uz = px[2];
+    } else {
+      ux = (px[1] + px[0]) * 0.5f;
+      uy = (py[row] + py[0]) * 0.5f;
+      uz = (pz[sz] + pz[0]) * 0.5f;
+      py += sy;
+      pz += sz;
+    }
+    px += sx;
+  }
+};
+
 struct ThreadCell {
   int x, y, z, pair;
   bool ok;
@@ -344,28 +387,46 @@ __global__ __launch_bounds__(256) void faces_from_centered_grad_kernel(Dims d, i
 // and CU (3.0 at random addresses) but fp32 at 0.33, so a sample's 8 corners
 // are added as they are.  (Within a tile the atomics add in no fixed order;
 // in fp64 that changes the stored fp32 partials hardly ever.)  One channel's
-// tile is 69 KB, two work-groups per CU; several channels take turns in it.
+// tile is 41 KB, three work-groups per CU; several channels take turns in it.
 // Measured: 128^3, one channel, B1 / B2 45.6 / 45.7 us with fp32 tiles and
-// merged neighbours -> 40.1 / 38.6; 96x160x96, three channels, 717 / 597 us
-// with global fp32 atomics -> 68 / 71.
-// The halo sets the partial-buffer traffic: tile cells per brick cell 2.11
-// with kHalo = 2, 2.86 with 3.
-constexpr int kBrickX = 32, kBrickY = 8, kBrickZ = 16, kHalo = 2;
-// a work-group is kBrickX x kBrickY x kBrickZT work-items; each visits
-// kBrickZ / kBrickZT cells of its (x, y) column
-constexpr int kBrickZT = 2, kBrickZPer = kBrickZ / kBrickZT;
+// merged neighbours -> 40.1 / 38.6 with fp64 tiles -> 31.4 / 37.0 with the
+// unmasked corner reads and the offsets of gather_tiles, at 3.3 / 3.6 TB/s of
+// their fields, tiles and velocity gradients; 96x160x96, three channels, 717 /
+// 597 us with global fp32 atomics -> 58 / 68.  The halo sets the partial-buffer
+// traffic: tile cells per brick cell 2.53 with kHalo = 2 (2.11 with bricks 16
+// deep, which measured the same at 128^3 and 30 % slower at 96x160x96).
+constexpr int kBrickX = 32, kBrickY = 8, kBrickZ = 8, kHalo = 2;
+// a work-group is kBrickX x kBrickY x kBrickZT work-items; each visits the
+// brick's z extent / kBrickZT cells of its (x, y) column
+constexpr int kBrickZT = 2;
 constexpr int kBrickThreads = kBrickX * kBrickY * kBrickZT;
 constexpr int kTileX = kBrickX + 2 * kHalo, kTileY = kBrickY + 2 * kHalo, kTileZ = kBrickZ + 2 * kHalo;
-constexpr int kTileCells = kTileX * kTileY * kTileZ;
+constexpr int kTilePlane = kTileX * kTileY, kTileCells = kTilePlane * kTileZ;
 
+// Bricks are 8 cells deep in z, or 4 where that leaves a CU with fewer than two
+// of them: the halves then run on more CUs (64^3: B1 / B2 14.6 / 15.9 us ->
+// 12.3 / 12.1; at 96x160x96, 720 deep bricks, 30.0 / 26.5 us against 31.4 /
+// 29.1 with flat ones, whose halos weigh more).
 struct BrickGrid {
   int nx, ny, nz;
+  int zl;  // log2 of the z extent
   __host__ __device__ int count() const { return nx * ny * nz; }
+  __host__ __device__ int depth() const { return 1 << zl; }
+  __host__ __device__ int tile_planes() const { return depth() + 2 * kHalo; }
+  __host__ __device__ int tile_cells() const { return kTilePlane * tile_planes(); }
 };
 
-inline BrickGrid brick_grid(const Dims& d) {
+inline BrickGrid brick_grid_of_depth(const Dims& d, int zl) {
   return BrickGrid{static_cast<int>(blocks_for(d.x, kBrickX)), static_cast<int>(blocks_for(d.y, kBrickY)),
-                   static_cast<int>(blocks_for(d.z, kBrickZ))};
+                   static_cast<int>(blocks_for(d.z, 1 << zl)), zl};
+}
+
+constexpr int64_t kFewBricks = 512;  // two per CU
+
+inline BrickGrid brick_grid(const Dims& d, int64_t pairs) {
+  static_assert(kBrickZ == 8, "depths 8 and 4");
+  const BrickGrid deep = brick_grid_of_depth(d, 3);
+  return deep.count() * pairs < kFewBricks ? brick_grid_of_depth(d, 2) : deep;
 }
 
 // fp64 atomic add into LDS (ds_add_f64); t must point into __shared__ memory.
@@ -374,12 +435,12 @@ NGT_DEVICE void lds_add(double* t, float v) {
   __hip_atomic_fetch_add((lds_double*)t, static_cast<double>(v), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
 }
 
-// Scatter val * w to the 8 corners of q: into the LDS tile (origin o*) when
-// the corner lies in it, else atomically into `ovf`, every `ovf_step`-th
+// Scatter val * w to the 8 corners of q: into the LDS tile (origin o*, that
+// many planes) when the corner lies in it, else atomically into `ovf`, every `ovf_step`-th
 // value of a full field.
 template <int BM>
-NGT_DEVICE void scatter_linear_tile(double* tile, int ox, int oy, int oz, float* __restrict__ ovf, int ovf_step,
-                                    const Dims& d, float qx, float qy, float qz, float val) {
+NGT_DEVICE void scatter_linear_tile(double* tile, int planes, int ox, int oy, int oz, float* __restrict__ ovf,
+                                    int ovf_step, const Dims& d, float qx, float qy, float qz, float val) {
   const Corners c = make_corners<BM>(d, qx, qy, qz);
   if constexpr (BM == BORDER) {
     if (!c.inside) return;
@@ -393,7 +454,7 @@ NGT_DEVICE void scatter_linear_tile(double* tile, int ox, int oy, int oz, float*
     // own, which no cell reads)
     if (static_cast<unsigned>(lx0) < static_cast<unsigned>(kTileX - 1) &&
         static_cast<unsigned>(ly0) < static_cast<unsigned>(kTileY - 1) &&
-        static_cast<unsigned>(lz0) < static_cast<unsigned>(kTileZ - 1)) {
+        static_cast<unsigned>(lz0) < static_cast<unsigned>(planes - 1)) {
       double* t = tile + (lz0 * kTileY + ly0) * kTileX + lx0;
 #pragma unroll
       for (int k = 0; k < 8; ++k) {
@@ -415,7 +476,7 @@ NGT_DEVICE void scatter_linear_tile(double* tile, int ox, int oy, int oz, float*
     const int lx = ix - ox, ly = iy - oy, lz = iz - oz;
     if (static_cast<unsigned>(lx) < static_cast<unsigned>(kTileX) &&
         static_cast<unsigned>(ly) < static_cast<unsigned>(kTileY) &&
-        static_cast<unsigned>(lz) < static_cast<unsigned>(kTileZ)) {
+        static_cast<unsigned>(lz) < static_cast<unsigned>(planes)) {
       lds_add(tile + (lz * kTileY + ly) * kTileX + lx, val * w);
     } else {
       atomic_add(ovf + cell_offset(d, ix, iy, iz) * ovf_step, val * w);
@@ -423,36 +484,46 @@ NGT_DEVICE void scatter_linear_tile(double* tile, int ox, int oy, int oz, float*
   }
 }
 
-// Sum of the tile partials of `slot` covering cell (x, y, z), bricks in
-// ascending z, y, x order.  A brick's partials hold its channels one after
-// another.
+// The step, in bricks, to the other brick along an axis whose tile holds the
+// cell as well (0: there is none): the previous one for the first kHalo cells
+// of a brick, the next one for the last kHalo.  b: the cell's brick of n, l:
+// its place among the brick's `size` cells.
+NGT_DEVICE int other_brick(int b, int l, int size, int n) {
+  return l < kHalo ? (b > 0 ? -1 : 0) : (l >= size - kHalo && b + 1 < n ? 1 : 0);
+}
+
+// Sum of the tile partials of `slot` covering cell (x, y, z): its own brick's
+// and those of the (at most 7) neighbours across the axes on which the cell
+// lies in a halo, at offsets that add up over the axes.  A brick's partials
+// hold its channels one after another.  Every load is issued before any is
+// added.
 template <int C>
 NGT_DEVICE Vec<C> gather_tiles(const float* __restrict__ tiles, int64_t slot, const BrickGrid& bg, int x, int y,
                                int z) {
-  // the (up to) 8 bricks whose tiles hold the cell: every load is issued
-  // before any is added, and the sum runs in the order z, y, x of the bricks
-  const int bx1 = min((x + kHalo) / kBrickX, bg.nx - 1), by1 = min((y + kHalo) / kBrickY, bg.ny - 1);
-  const int bz1 = min((z + kHalo) / kBrickZ, bg.nz - 1);
+  const int bx = x / kBrickX, by = y / kBrickY, bz = z >> bg.zl;
+  const int lx = x % kBrickX, ly = y % kBrickY, lz = z & (bg.depth() - 1);
+  const int64_t step = bg.tile_cells();
+  const int64_t brick = step * C;
+  const float* own = tiles + ((slot * bg.nz + bz) * (bg.ny * bg.nx) + by * bg.nx + bx) * brick +
+                     ((lz + kHalo) * kTileY + ly + kHalo) * kTileX + lx + kHalo;
+  const int sx = other_brick(bx, lx, kBrickX, bg.nx), sy = other_brick(by, ly, kBrickY, bg.ny),
+            sz = other_brick(bz, lz, bg.depth(), bg.nz);
+  const int64_t ox = sx * (brick - kBrickX), oy = sy * (bg.nx * brick - kBrickY * kTileX),
+                oz = sz * (bg.nx * bg.ny * brick - bg.depth() * kTilePlane);
   Vec<C> t[8];
-  bool ok[8];
 #pragma unroll
   for (int q = 0; q < 8; ++q) {
-    const int bz = bz1 - 1 + (q >> 2), by = by1 - 1 + ((q >> 1) & 1), bx = bx1 - 1 + (q & 1);
-    const int lz = z - (bz * kBrickZ - kHalo), ly = y - (by * kBrickY - kHalo), lx = x - (bx * kBrickX - kHalo);
-    ok[q] = bz >= 0 && by >= 0 && bx >= 0 && lz >= 0 && lz < kTileZ && ly >= 0 && ly < kTileY && lx >= 0 &&
-            lx < kTileX;
+    const bool on = (!(q & 1) || sx != 0) && (!(q & 2) || sy != 0) && (!(q & 4) || sz != 0);
     t[q] = vzero<C>();
-    if (ok[q]) {
-      const int64_t brick = (slot * bg.nz + bz) * bg.ny * bg.nx + static_cast<int64_t>(by) * bg.nx + bx;
-      const float* p = tiles + brick * (kTileCells * C) + (lz * kTileY + ly) * kTileX + lx;
+    if (on) {
+      const float* p = own + ((q & 1) ? ox : 0) + ((q & 2) ? oy : 0) + ((q & 4) ? oz : 0);
 #pragma unroll
-      for (int i = 0; i < C; ++i) t[q].v[i] = p[i * kTileCells];
+      for (int i = 0; i < C; ++i) t[q].v[i] = p[i * step];
     }
   }
-  Vec<C> s = vzero<C>();
+  Vec<C> s = t[0];
 #pragma unroll
-  for (int q = 0; q < 8; ++q) {
-    if (!ok[q]) continue;
+  for (int q = 1; q < 8; ++q) {
 #pragma unroll
     for (int i = 0; i < C; ++i) s.v[i] += t[q].v[i];
   }
@@ -470,7 +541,7 @@ NGT_DEVICE BrickCell brick_cell(const BrickGrid& bg, const VBlock& vb) {
   const int bx = b.brick % bg.nx, by = (b.brick / bg.nx) % bg.ny, bz = b.brick / (bg.nx * bg.ny);
   b.x = bx * kBrickX + static_cast<int>(threadIdx.x);
   b.y = by * kBrickY + static_cast<int>(threadIdx.y);
-  b.z0 = bz * kBrickZ;
+  b.z0 = bz << bg.zl;
   b.ox = bx * kBrickX - kHalo;
   b.oy = by * kBrickY - kHalo;
   b.oz = b.z0 - kHalo;
@@ -479,8 +550,8 @@ NGT_DEVICE BrickCell brick_cell(const BrickGrid& bg, const VBlock& vb) {
 
 NGT_DEVICE int brick_thread() { return (threadIdx.z * kBrickY + threadIdx.y) * kBrickX + threadIdx.x; }
 
-NGT_DEVICE void tile_clear(double* tile) {
-  for (int i = brick_thread(); i < kTileCells; i += kBrickThreads) tile[i] = 0.0;
+NGT_DEVICE void tile_clear(double* tile, const BrickGrid& bg) {
+  for (int i = brick_thread(); i < bg.tile_cells(); i += kBrickThreads) tile[i] = 0.0;
   __syncthreads();
 }
 
@@ -490,8 +561,9 @@ template <int C>
 NGT_DEVICE void tile_store(double* tile, float* __restrict__ tiles, const BrickGrid& bg, const BrickCell& b, int c,
                            bool again) {
   __syncthreads();
-  float* dst = tiles + ((static_cast<int64_t>(b.pair) * bg.count() + b.brick) * C + c) * kTileCells;
-  for (int i = brick_thread(); i < kTileCells; i += kBrickThreads) {
+  const int cells = bg.tile_cells();
+  float* dst = tiles + ((static_cast<int64_t>(b.pair) * bg.count() + b.brick) * C + c) * cells;
+  for (int i = brick_thread(); i < cells; i += kBrickThreads) {
     dst[i] = static_cast<float>(tile[i]);
     if (again) tile[i] = 0.0;
   }
@@ -516,15 +588,19 @@ NGT_DEVICE void add_vel_grad(const GradVel& gv, int v, int64_t cell, float gx, f
 
 // Visits the work-item's cells of the brick: f(cell, z, displacement).
 template <typename F>
-NGT_DEVICE void for_brick_cells(const AdvArgs& a, const BrickCell& b, int v, F&& f) {
+NGT_DEVICE void for_brick_cells(const AdvArgs& a, const BrickGrid& bg, const BrickCell& b, int v, F&& f) {
   if (b.x >= a.d.x || b.y >= a.d.y) return;
-  const int zb = b.z0 + static_cast<int>(threadIdx.z) * kBrickZPer;
-  const int z1 = min(zb + kBrickZPer, a.d.z);
+  const int per = bg.depth() / kBrickZT;
+  const int zb = b.z0 + static_cast<int>(threadIdx.z) * per;
+  const int z1 = min(zb + per, a.d.z);
+  VelocityColumn vel(a, v, b.x, b.y, zb);
+  const int64_t plane = static_cast<int64_t>(a.d.x) * a.d.y;
+  int64_t cell = cell_offset(a.d, b.x, b.y, zb);
 #pragma unroll 1
-  for (int z = zb; z < z1; ++z) {
+  for (int z = zb; z < z1; ++z, cell += plane) {
     float ux, uy, uz;
-    load_velocity(a, v, b.x, b.y, z, ux, uy, uz);
-    f(cell_offset(a.d, b.x, b.y, z), z, a.ts * ux, a.ts * uy, a.ts * uz);
+    vel.next(ux, uy, uz);
+    f(cell, z, a.ts * ux, a.ts * uy, a.ts * uz);
   }
 }
 
@@ -540,7 +616,7 @@ NGT_DEVICE void advect_mc_bwd_brick_kernel_body(const VBlock& vb, const AdvArgs&
                                                 float* __restrict__ g_dir, float* r_dir, float* __restrict__ ovf,
                                                 float* __restrict__ tiles, const GradVel& gv, int vel_mode) {
   __shared__ double tile[kTileCells];
-  tile_clear(tile);
+  tile_clear(tile, bg);
   const BrickCell b = brick_cell(bg, vb);
   int n, v;
   pair_indices(a, b.pair, n, v);
@@ -550,7 +626,7 @@ NGT_DEVICE void advect_mc_bwd_brick_kernel_body(const VBlock& vb, const AdvArgs&
   const float fx = static_cast<float>(b.x), fy = static_cast<float>(b.y);
   float* rdp = r_dir + b.pair * cells * C;
   float* ovp = ovf + b.pair * cells * C;
-  for_brick_cells(a, b, v, [&](int64_t cell, int z, float tx, float ty, float tz) {
+  for_brick_cells(a, bg, b, v, [&](int64_t cell, int z, float tx, float ty, float tz) {
     const float fz = static_cast<float>(z);
     const float bx = fx + (-tx), by = fy + (-ty), bz = fz + (-tz);
     Vec<C> g = vload<C>(g_out + (b.pair * cells + cell) * C);
@@ -585,14 +661,14 @@ NGT_DEVICE void advect_mc_bwd_brick_kernel_body(const VBlock& vb, const AdvArgs&
     vstore<C>(rdp + cell * C, rd);
     add_vel_grad(gv, v, cell, -a.ts * vdot(gback, dx), -a.ts * vdot(gback, dy), -a.ts * vdot(gback, dz),
                  vel_mode == 1 ? 0 : vel_mode);
-    if constexpr (C == 1) scatter_linear_tile<BM>(tile, b.ox, b.oy, b.oz, ovp, 1, a.d, bx, by, bz, gback.v[0]);
+    if constexpr (C == 1) scatter_linear_tile<BM>(tile, bg.tile_planes(), b.ox, b.oy, b.oz, ovp, 1, a.d, bx, by, bz, gback.v[0]);
   });
   if constexpr (C == 1) {
     tile_store<C>(tile, tiles, bg, b, 0, false);
   } else {
     for (int c = 0; c < C; ++c) {
-      for_brick_cells(a, b, v, [&](int64_t cell, int z, float tx, float ty, float tz) {
-        scatter_linear_tile<BM>(tile, b.ox, b.oy, b.oz, ovp + c, C, a.d, fx + (-tx), fy + (-ty),
+      for_brick_cells(a, bg, b, v, [&](int64_t cell, int z, float tx, float ty, float tz) {
+        scatter_linear_tile<BM>(tile, bg.tile_planes(), b.ox, b.oy, b.oz, ovp + c, C, a.d, fx + (-tx), fy + (-ty),
                                 static_cast<float>(z) + (-tz), -rdp[cell * C + c]);
       });
       tile_store<C>(tile, tiles, bg, b, c, c + 1 < C);
@@ -620,7 +696,7 @@ NGT_DEVICE void advect_sl_bwd_brick_kernel_body(const VBlock& vb, const AdvArgs&
                                                 float* __restrict__ tiles2, const GradVel& gv, int vel_mode,
                                                 float* val) {
   __shared__ double tile[kTileCells];
-  tile_clear(tile);
+  tile_clear(tile, bg);
   const BrickCell b = brick_cell(bg, vb);
   int n, v;
   pair_indices(a, b.pair, n, v);
@@ -628,7 +704,7 @@ NGT_DEVICE void advect_sl_bwd_brick_kernel_body(const VBlock& vb, const AdvArgs&
   const float* src = rho + n * cells * C;
   float* ovp = g_rho + n * cells * C;
   const float fx = static_cast<float>(b.x), fy = static_cast<float>(b.y);
-  for_brick_cells(a, b, v, [&](int64_t cell, int z, float tx, float ty, float tz) {
+  for_brick_cells(a, bg, b, v, [&](int64_t cell, int z, float tx, float ty, float tz) {
     const float px = fx + tx, py = fy + ty, pz = static_cast<float>(z) + tz;
     Vec<C> g = vload<C>(g_in + (b.pair * cells + cell) * C);
     if constexpr (ORDER2) {
@@ -643,7 +719,7 @@ NGT_DEVICE void advect_sl_bwd_brick_kernel_body(const VBlock& vb, const AdvArgs&
       for (int i = 0; i < C; ++i)
         if (!(r.v[i] >= 0.f)) g.v[i] = 0.f;
     }
-    if constexpr (C == 1) scatter_linear_tile<BM>(tile, b.ox, b.oy, b.oz, ovp, 1, a.d, px, py, pz, g.v[0]);
+    if constexpr (C == 1) scatter_linear_tile<BM>(tile, bg.tile_planes(), b.ox, b.oy, b.oz, ovp, 1, a.d, px, py, pz, g.v[0]);
     else vstore<C>(val + (b.pair * cells + cell) * C, g);
     Vec<C> dx, dy, dz;
     read_gradient<C, BM>(src, a.d, px, py, pz, dx, dy, dz);
@@ -653,8 +729,8 @@ NGT_DEVICE void advect_sl_bwd_brick_kernel_body(const VBlock& vb, const AdvArgs&
     tile_store<C>(tile, tiles2, bg, b, 0, false);
   } else {
     for (int c = 0; c < C; ++c) {
-      for_brick_cells(a, b, v, [&](int64_t cell, int z, float tx, float ty, float tz) {
-        scatter_linear_tile<BM>(tile, b.ox, b.oy, b.oz, ovp + c, C, a.d, fx + tx, fy + ty, static_cast<float>(z) + tz,
+      for_brick_cells(a, bg, b, v, [&](int64_t cell, int z, float tx, float ty, float tz) {
+        scatter_linear_tile<BM>(tile, bg.tile_planes(), b.ox, b.oy, b.oz, ovp + c, C, a.d, fx + tx, fy + ty, static_cast<float>(z) + tz,
                                 val[(b.pair * cells + cell) * C + c]);
       });
       tile_store<C>(tile, tiles2, bg, b, c, c + 1 < C);
@@ -959,7 +1035,7 @@ __global__ __launch_bounds__(kBrickThreads) void advect_mc_bwd_batch_kernel(cons
     const int i = __builtin_amdgcn_readfirstlane(find_item(v.brick, v.h->n, t));
     const AdvBatchItem& it = v.items[i];
     const AdvBatchBufs b = batch_bufs(it);
-    const GradVel gv{v.h->staggered ? ws + it.ws_gvc : b.gvx, it.cells, 3};
+    const GradVel gv{v.h->staggered ? ws + it.ws_gvc : b.gvx, it.cells, v.h->staggered ? 1 : 3};
     // the direct rho term goes straight to input_grad; the masked output
     // gradient is kept only where NEGATIVE changes it
     advect_mc_bwd_brick_kernel_body<1, BM, CLAMPM>(VBlock{t - v.brick[i], 0, 0}, b.a, it.bg, b.input, b.sl,
@@ -977,7 +1053,7 @@ __global__ __launch_bounds__(kBrickThreads) void advect_sl_bwd_batch_kernel(cons
     const int i = __builtin_amdgcn_readfirstlane(find_item(v.brick, v.h->n, t));
     const AdvBatchItem& it = v.items[i];
     const AdvBatchBufs b = batch_bufs(it);
-    const GradVel gv{v.h->staggered ? ws + it.ws_gvc : b.gvx, it.cells, 3};
+    const GradVel gv{v.h->staggered ? ws + it.ws_gvc : b.gvx, it.cells, v.h->staggered ? 1 : 3};
     const float* g = ORDER2 && v.h->clamp == NGT_CLAMP_NEGATIVE ? ws + it.ws_gsl : b.g_out;
     advect_sl_bwd_brick_kernel_body<1, BM, NEG, ORDER2>(VBlock{t - v.brick[i], 0, 0}, b.a, it.bg, b.input,
                                                         g, ws + it.ws_ovf,
@@ -1000,7 +1076,7 @@ __global__ __launch_bounds__(256) void advect_rho_gather_batch_kernel(const void
       advect_rho_gather_kernel_body<1>(vb, it.a, it.bg, nullptr, ws + it.ws_t2, g_in);
       const int x = vb.x * kBX + static_cast<int>(threadIdx.x), y = vb.y * kBY + static_cast<int>(threadIdx.y);
       if (staggered && x < it.a.d.x && y < it.a.d.y)
-        faces_of_cell(it.a.d, GradVel{ws + it.ws_gvc, it.cells, 3}, (float*)it.gvx, (float*)it.gvy, (float*)it.gvz, x, y, vb.z);
+        faces_of_cell(it.a.d, GradVel{ws + it.ws_gvc, it.cells, 1}, (float*)it.gvx, (float*)it.gvy, (float*)it.gvz, x, y, vb.z);
     });
   }
 }
@@ -1027,7 +1103,8 @@ size_t ngt_advect_workspace_size(const int64_t* input_shape, int num_velocities,
                               + pairs * cells;           // reference: hit counts (uint32)
     const Dims d{static_cast<int>(input_shape[3]), static_cast<int>(input_shape[2]),
                  static_cast<int>(input_shape[1])};
-    const int64_t tiles = pairs * brick_grid(d).count() * static_cast<int64_t>(kTileCells) * C;
+    const BrickGrid bg = brick_grid(d, pairs);
+    const int64_t tiles = pairs * bg.count() * static_cast<int64_t>(bg.tile_cells()) * C;
     const int64_t brick_extra = tiles + (order == 2 ? 2 * pairs * cells * C + tiles : 0);  // tiles2 (+ r_dir, ovf1, tiles1)
     floats += std::max(ref_extra, brick_extra);
   }
@@ -1087,7 +1164,7 @@ int ngt_advect_bwd(const float* input, const int64_t* input_shape, const float* 
   float* g_vc = g_sl + field;
   float* tmp = g_vc + static_cast<int64_t>(p.a.n_vel) * p.cells * 3;
   uint32_t* hits = reinterpret_cast<uint32_t*>(tmp + field);
-  const GradVel gv{p.a.staggered ? g_vc : vel_x_grad, p.cells, 3};  // centered: accumulated in place
+  const GradVel gv{p.a.staggered ? g_vc : vel_x_grad, p.cells, p.a.staggered ? 1 : 3};  // centered: accumulated in place
 
   const float* slp = sl;
   if (order == 2 && slp == nullptr) {
@@ -1099,8 +1176,8 @@ int ngt_advect_bwd(const float* input, const int64_t* input_shape, const float* 
   if (ref || order == 1) fill_zero(input_grad, p.a.n_data * p.cells * p.C, s);
   if (!ref) {
     // brick-tiled exact adjoint: workspace after g_vc = [tiles2 | r_dir | ovf1 | tiles1]
-    const BrickGrid bg = brick_grid(p.a.d);
-    const int64_t tiles_n = static_cast<int64_t>(p.pairs) * bg.count() * kTileCells * p.C;
+    const BrickGrid bg = brick_grid(p.a.d, p.pairs);
+    const int64_t tiles_n = static_cast<int64_t>(p.pairs) * bg.count() * bg.tile_cells() * p.C;
     float* tiles2 = tmp;
     float* r_dir = tiles2 + tiles_n;
     float* ovf1 = r_dir + field;
@@ -1202,6 +1279,11 @@ int ngt_advect_batch_plan(const ngt_advect_instance* inst, int n, int order, int
   int* brick = blob_at<int>(plan, off_brick);
   int* fill = blob_at<int>(plan, off_fill);
   const int staggered = inst[0].vel_y != nullptr ? 1 : 0;
+  // the bricks of all instances share the CUs, so their depth is one
+  int64_t deep = 0;
+  for (int i = 0; i < n; ++i)
+    deep += brick_grid_of_depth(Dims{inst[i].dhw[2], inst[i].dhw[1], inst[i].dhw[0]}, 3).count();
+  const int zl = deep < kFewBricks ? 2 : 3;
   int64_t tc = 0, tb = 0, tl = 0, ws = 0;
   cell[0] = brick[0] = fill[0] = 0;
   for (int i = 0; i < n; ++i) {
@@ -1219,7 +1301,7 @@ int ngt_advect_batch_plan(const ngt_advect_instance* inst, int n, int order, int
     it.a.ts = q.timestep;
     it.a.vx = q.vel_x; it.a.vy = q.vel_y; it.a.vz = q.vel_z;
     it.a.staggered = staggered;
-    it.bg = brick_grid(it.a.d);
+    it.bg = brick_grid_of_depth(it.a.d, zl);
     it.nbx = static_cast<int>(blocks_for(it.a.d.x, kBX));
     it.nby = static_cast<int>(blocks_for(it.a.d.y, kBY));
     it.cells = static_cast<int64_t>(q.dhw[0]) * q.dhw[1] * q.dhw[2];
@@ -1227,7 +1309,7 @@ int ngt_advect_batch_plan(const ngt_advect_instance* inst, int n, int order, int
     it.input = (gptr<const float>)q.input; it.output = (gptr<float>)q.output; it.sl = (gptr<float>)q.sl;
     it.g_out = (gptr<const float>)q.output_grad; it.g_in = (gptr<float>)q.input_grad;
     it.gvx = (gptr<float>)q.vel_x_grad; it.gvy = (gptr<float>)q.vel_y_grad; it.gvz = (gptr<float>)q.vel_z_grad;
-    const int64_t tiles = static_cast<int64_t>(it.bg.count()) * kTileCells;
+    const int64_t tiles = static_cast<int64_t>(it.bg.count()) * it.bg.tile_cells();
     auto take = [&](int64_t floats) {
       const int64_t off = ws;
       ws += (floats + 63) / 64 * 64;  // 256-byte aligned regions

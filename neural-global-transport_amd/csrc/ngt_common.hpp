@@ -204,13 +204,25 @@ NGT_DEVICE void fetch8_raw(const float* __restrict__ g, const Dims& d, const Cor
     z0 = min(max(z0, 0), d.z - 1); z1 = min(max(z1, 0), d.z - 1);
   }
   const uint32_t W = static_cast<uint32_t>(d.x), H = static_cast<uint32_t>(d.y);
-  const uint32_t rows[4] = {(static_cast<uint32_t>(z0) * H + static_cast<uint32_t>(y0)) * W,
-                            (static_cast<uint32_t>(z0) * H + static_cast<uint32_t>(y1)) * W,
-                            (static_cast<uint32_t>(z1) * H + static_cast<uint32_t>(y0)) * W,
-                            (static_cast<uint32_t>(z1) * H + static_cast<uint32_t>(y1)) * W};
-  const uint32_t xs[2] = {static_cast<uint32_t>(x0), static_cast<uint32_t>(x1)};
+  if constexpr (BM == WRAP) {
+    const uint32_t rows[4] = {(static_cast<uint32_t>(z0) * H + static_cast<uint32_t>(y0)) * W,
+                              (static_cast<uint32_t>(z0) * H + static_cast<uint32_t>(y1)) * W,
+                              (static_cast<uint32_t>(z1) * H + static_cast<uint32_t>(y0)) * W,
+                              (static_cast<uint32_t>(z1) * H + static_cast<uint32_t>(y1)) * W};
+    const uint32_t xs[2] = {static_cast<uint32_t>(x0), static_cast<uint32_t>(x1)};
 #pragma unroll
-  for (int k = 0; k < 8; ++k) v[k] = vload<C>(g + (rows[k >> 1] + xs[k & 1]) * static_cast<uint32_t>(C));
+    for (int k = 0; k < 8; ++k) v[k] = vload<C>(g + (rows[k >> 1] + xs[k & 1]) * static_cast<uint32_t>(C));
+  } else {
+    // the clamped ceil index is the floor index or the next: one address is
+    // multiplied out (32-bit multiplies run at a quarter of the rate), the
+    // other corners are selected steps away
+    const uint32_t base = ((static_cast<uint32_t>(z0) * H + static_cast<uint32_t>(y0)) * W + static_cast<uint32_t>(x0)) * static_cast<uint32_t>(C);
+    const uint32_t sx = x1 != x0 ? static_cast<uint32_t>(C) : 0u, sy = y1 != y0 ? W * static_cast<uint32_t>(C) : 0u,
+                   sz = z1 != z0 ? W * H * static_cast<uint32_t>(C) : 0u;
+    const uint32_t rows[4] = {base, base + sy, base + sz, base + sy + sz};
+#pragma unroll
+    for (int k = 0; k < 8; ++k) v[k] = vload<C>(g + (rows[k >> 1] + ((k & 1) ? sx : 0u)));
+  }
 }
 
 // Haloed brick layout of a grid slice: the grid is cut into 4x4x4-cell
@@ -311,12 +323,44 @@ NGT_DEVICE Vec<C> lerp8(const Vec<C> (&v)[8], const Corners& c) {
   return r;
 }
 
+// The 8 masked corner values of position q, with the weights and validity of
+// q in c (its indices are not set).  A wavefront whose samples all lie between
+// cells of the grid on every axis - nearly all of them - needs no clamps, no
+// masks and no ceil corners: the upper corners are one step up each axis, at
+// four row addresses.  (The kernels that sample are bound by their vector
+// instructions as much as by the loads: about 45 per read here against 100.)
+template <int C, int BM>
+NGT_DEVICE void fetch_corners(const float* __restrict__ g, const Dims& d, float qx, float qy, float qz, Corners& c,
+                              Vec<C> (&v)[8]) {
+  const float fx = floorf(qx), fy = floorf(qy), fz = floorf(qz);
+  const float wx = qx - fx, wy = qy - fy, wz = qz - fz;
+  const int x0 = static_cast<int>(fx), y0 = static_cast<int>(fy), z0 = static_cast<int>(fz);
+  const bool between = (static_cast<unsigned>(x0) < static_cast<unsigned>(d.x - 1)) &
+                       (static_cast<unsigned>(y0) < static_cast<unsigned>(d.y - 1)) &
+                       (static_cast<unsigned>(z0) < static_cast<unsigned>(d.z - 1)) & (wx > 0.f) & (wy > 0.f) &
+                       (wz > 0.f);
+  if (__all(between)) {
+    c.wx = wx; c.wy = wy; c.wz = wz;
+    c.inside = true;
+    const uint32_t row = static_cast<uint32_t>(d.x) * C;
+    const uint32_t plane = static_cast<uint32_t>(d.y) * row;
+    const float* const p = g + ((static_cast<uint32_t>(z0) * static_cast<uint32_t>(d.y) + static_cast<uint32_t>(y0)) * row +
+                                static_cast<uint32_t>(x0) * static_cast<uint32_t>(C));
+    const float* const rows[4] = {p, p + row, p + plane, p + plane + row};
+#pragma unroll
+    for (int k = 0; k < 8; ++k) v[k] = vload<C>(rows[k >> 1] + (k & 1) * C);
+  } else {
+    c = make_corners<BM>(d, qx, qy, qz);
+    fetch8_raw<C, BM>(g, d, c, v);
+    mask8<C, BM>(c, v);
+  }
+}
+
 template <int C, int BM>
 NGT_DEVICE Vec<C> read_linear(const float* __restrict__ g, const Dims& d, float qx, float qy, float qz) {
-  const Corners c = make_corners<BM>(d, qx, qy, qz);
+  Corners c;
   Vec<C> v[8];
-  fetch8_raw<C, BM>(g, d, c, v);
-  mask8<C, BM>(c, v);
+  fetch_corners<C, BM>(g, d, qx, qy, qz, c, v);
   return lerp8<C, BM>(v, c);
 }
 
@@ -464,32 +508,29 @@ NGT_DEVICE Vec<C> read_minmax(const float* __restrict__ g, const Dims& d, float 
   return acc;
 }
 
-// Min and max over the 8 corners from one fetch (read_minmax semantics).
+// Min and max over the 8 corners from one fetch (read_minmax semantics: a
+// corner outside the grid counts as 0, an invalid position is 0).
 template <int C, int BM>
 NGT_DEVICE void read_minmax2(const float* __restrict__ g, const Dims& d, float qx, float qy, float qz, Vec<C>& mn,
                              Vec<C>& mx) {
-  const Corners c = make_corners<BM>(d, qx, qy, qz);
+  Corners c;
+  Vec<C> k[8];
+  fetch_corners<C, BM>(g, d, qx, qy, qz, c, k);
   mn = vfill<C>(kFloatMax);
   mx = vfill<C>(-kFloatMax);
-  if constexpr (BM == BORDER) {
-    if (!(c.vx0 && c.vx1 && c.vy0 && c.vy1 && c.vz0 && c.vz1)) {
-      mn = vzero<C>();
-      mx = vzero<C>();
-    }
-  }
-  const Corner8<C> k = fetch8<C, BM>(g, d, c);
 #pragma unroll
   for (int j = 0; j < 8; ++j) {
 #pragma unroll
     for (int i = 0; i < C; ++i) {
-      mn.v[i] = (k.ok[j] && k.v[j].v[i] < mn.v[i]) ? k.v[j].v[i] : mn.v[i];
-      mx.v[i] = (k.ok[j] && k.v[j].v[i] > mx.v[i]) ? k.v[j].v[i] : mx.v[i];
+      mn.v[i] = k[j].v[i] < mn.v[i] ? k[j].v[i] : mn.v[i];
+      mx.v[i] = k[j].v[i] > mx.v[i] ? k[j].v[i] : mx.v[i];
     }
   }
   if constexpr (BM == BORDER) {
-    if (!c.inside) {
-      mn = vzero<C>();
-      mx = vzero<C>();
+#pragma unroll
+    for (int i = 0; i < C; ++i) {
+      mn.v[i] = c.inside ? mn.v[i] : 0.f;
+      mx.v[i] = c.inside ? mx.v[i] : 0.f;
     }
   }
 }
@@ -627,38 +668,15 @@ NGT_DEVICE Vec<C> read_filtered(const float* __restrict__ g, const Dims& d, floa
   else return read_minmax<C, BM, true>(g, d, qx, qy, qz);
 }
 
-// d read_linear / d q per channel (sampling.hpp:470-565).  Coinciding
-// floor/ceil corners make the derivative along that axis 0 at integer q.
-template <int C, int BM>
-NGT_DEVICE void read_gradient(const float* __restrict__ g, const Dims& d, float qx, float qy, float qz,
-                              Vec<C>& dx, Vec<C>& dy, Vec<C>& dz) {
-  const Corners c = make_corners<BM>(d, qx, qy, qz);
-  const Corner8<C> k = fetch8<C, BM>(g, d, c);
-  dx = vlerp(vlerp(vsub(k.v[1], k.v[0]), vsub(k.v[3], k.v[2]), c.wy),
-             vlerp(vsub(k.v[5], k.v[4]), vsub(k.v[7], k.v[6]), c.wy), c.wz);
-  dy = vlerp(vlerp(vsub(k.v[2], k.v[0]), vsub(k.v[3], k.v[1]), c.wx),
-             vlerp(vsub(k.v[6], k.v[4]), vsub(k.v[7], k.v[5]), c.wx), c.wz);
-  dz = vlerp(vlerp(vsub(k.v[4], k.v[0]), vsub(k.v[5], k.v[1]), c.wx),
-             vlerp(vsub(k.v[6], k.v[2]), vsub(k.v[7], k.v[3]), c.wx), c.wy);
-  if constexpr (BM == BORDER) {
-#pragma unroll
-    for (int i = 0; i < C; ++i) {
-      dx.v[i] = c.inside ? dx.v[i] : 0.f;
-      dy.v[i] = c.inside ? dy.v[i] : 0.f;
-      dz.v[i] = c.inside ? dz.v[i] : 0.f;
-    }
-  }
-}
-
-// read_linear and read_gradient of one position from one fetch of the 8
-// corners (identical results).
+// read_linear and d read_linear / d q per channel (sampling.hpp:470-565) of one
+// position.  Coinciding floor/ceil corners make the derivative along that axis
+// 0 at integer q.
 template <int C, int BM>
 NGT_DEVICE Vec<C> read_linear_gradient(const float* __restrict__ g, const Dims& d, float qx, float qy, float qz,
                                        Vec<C>& dx, Vec<C>& dy, Vec<C>& dz) {
-  const Corners c = make_corners<BM>(d, qx, qy, qz);
+  Corners c;
   Vec<C> k[8];
-  fetch8_raw<C, BM>(g, d, c, k);
-  mask8<C, BM>(c, k);
+  fetch_corners<C, BM>(g, d, qx, qy, qz, c, k);
   dx = vlerp(vlerp(vsub(k[1], k[0]), vsub(k[3], k[2]), c.wy), vlerp(vsub(k[5], k[4]), vsub(k[7], k[6]), c.wy), c.wz);
   dy = vlerp(vlerp(vsub(k[2], k[0]), vsub(k[3], k[1]), c.wx), vlerp(vsub(k[6], k[4]), vsub(k[7], k[5]), c.wx), c.wz);
   dz = vlerp(vlerp(vsub(k[4], k[0]), vsub(k[5], k[1]), c.wx), vlerp(vsub(k[6], k[2]), vsub(k[7], k[3]), c.wx), c.wy);
@@ -671,6 +689,12 @@ NGT_DEVICE Vec<C> read_linear_gradient(const float* __restrict__ g, const Dims& 
     }
   }
   return lerp8<C, BM>(k, c);
+}
+
+template <int C, int BM>
+NGT_DEVICE void read_gradient(const float* __restrict__ g, const Dims& d, float qx, float qy, float qz,
+                              Vec<C>& dx, Vec<C>& dy, Vec<C>& dz) {
+  read_linear_gradient<C, BM>(g, d, qx, qy, qz, dx, dy, dz);
 }
 
 // Scatter ``val`` with trilinear weights to the 8 corners.

@@ -36,3 +36,23 @@ def test_advect_channels_across_bricks(ngt_ops, C, shape, order, clamp, bound, s
     vel_np = tuple(TB.dev(f[None]) for f in faces) if staggered else TB.dev(vc[None])
     gpu = TB._gpu_parts(ngt_ops, TB.dev(rho[None]), vel_np, order, clamp, bound, out)
     TB._check_grads(rt, vel, faces, rho, vc, g, order, clamp, bound, gpu)
+
+
+@pytest.mark.parametrize("C", [1, 3])
+def test_advect_deep_bricks_equal_flat_ones(ngt_ops, C):  # noqa: F811
+    """Twelve instances in one call fill the GPU with 8-cell-deep bricks, each
+    alone runs 4-cell-deep ones: the same gradients up to the rounding of the
+    fp32 tile partials (at most 8 per cell, and twice: 16 * 2^-24 < 1e-6)."""
+    rng = np.random.default_rng(77 + C)
+    N, shape = 12, (37, 20, 70)
+    rho = [TB._case_inputs(rng, shape, C, False, vmax=1.9) for _ in range(N)]
+    dens = TB.dev(np.stack([r[0] for r in rho])).requires_grad_()
+    vel = TB.dev(np.stack([r[2] for r in rho])).requires_grad_()
+    g = TB.dev(rng.standard_normal((N, 1) + shape + (C,)))
+    args = dict(timestep=-1.0, order=2, clamp_extrema="MC_SMOOTH", boundary="BORDER", separate_velocity_batch=False)
+    ngt_ops.advect_grid_semi_langrange(dens, vel, **args).backward(g)
+    for n in range(0, N, 5):
+        d, v = (t.detach()[n:n + 1].clone().requires_grad_() for t in (dens, vel))
+        ngt_ops.advect_grid_semi_langrange(d, v, **args).backward(g[n:n + 1])
+        assert TB.rel(TB.host(dens.grad)[n:n + 1], TB.host(d.grad)) < 1e-6
+        assert TB.rel(TB.host(vel.grad)[n:n + 1], TB.host(v.grad)) < 1e-6
