@@ -8,16 +8,18 @@
 // one launch (grid.z = depth x pairs) instead of the reference's per-camera
 // launch + device sync loop (resample_grid.cu.cc:712-794).
 //
-// Backward: the LUT / transform positions are arbitrary, so the input
-// gradient is a scatter with hardware fp32 atomics; the LUT gradient is a
-// pure gather (data gradient . dy) accumulated over the data batch in
-// registers.
+// Backward: a table's positions are arbitrary, so its input gradient is a
+// scatter with hardware fp32 atomics, and so is a transform's where it is not
+// the gather below; the LUT gradient is a pure gather (data gradient . dy)
+// accumulated over the data batch in registers.
 //
 // Mips: the pyramid of every batch entry is built once per call in the
 // workspace (one launch per level, 2x2x2 means in the reference's pairwise
 // order z, y, x: resample_grid.cu.cc:58-84).  The exact adjoint scatters into
 // per-level gradient buffers and collapses them coarse to fine, each fine
 // cell adding 1/8 of its parent (no atomics in the collapse).
+#include <cmath>
+
 #include "ngt_host.hpp"
 
 namespace ngt {
@@ -100,16 +102,30 @@ NGT_DEVICE Vec<C> read_level(const MipSet& s, int n, int m, float px, float py, 
   return read_filtered<C, FM, BM>(g, dm, px * sc - cco, py * sc - cco, pz * sc - cco);
 }
 
-// Mip-mapped read of position p (before the cell-centre offset).
+// Mip-mapped read of position p (before the cell-centre offset).  The levels
+// are visited one by one, those that no lane of the wavefront reads skipped:
+// a level's address and extents are then scalar (a level of its own per lane
+// walks the pyramid's offsets in 64-bit vector arithmetic, twice).
 template <int C, int FM, int BM, int MM>
 NGT_DEVICE Vec<C> read_mip(const MipSet& s, int n, float px, float py, float pz, float lod_raw, float bias,
                            float cco) {
   const MipPick k = mip_pick<MM>(lod_raw, bias, s.num_levels);
-  Vec<C> r = read_level<C, FM, BM>(s, n, k.lf, px, py, pz, cco);
-  if constexpr (MM == NGT_MIP_LINEAR) {
-    if (k.two) r = vlerp(r, read_level<C, FM, BM>(s, n, k.lc, px, py, pz, cco), k.wc);
+  Vec<C> rf = vzero<C>(), rc = vzero<C>();
+  for (int m = 0; m <= s.num_levels; ++m) {
+    const bool low = k.lf == m, high = MM == NGT_MIP_LINEAR && k.two && k.lc == m;
+    if (low || high) {
+      const Vec<C> v = read_level<C, FM, BM>(s, n, m, px, py, pz, cco);
+#pragma unroll
+      for (int i = 0; i < C; ++i) {
+        rf.v[i] = low ? v.v[i] : rf.v[i];
+        rc.v[i] = high ? v.v[i] : rc.v[i];
+      }
+    }
   }
-  return r;
+  if constexpr (MM == NGT_MIP_LINEAR) {
+    if (k.two) rf = vlerp(rf, rc, k.wc);
+  }
+  return rf;
 }
 
 template <int C, int FM, int BM>
@@ -427,6 +443,14 @@ NGT_DEVICE float xform_lod(const XformArgs& a, const CamParams& cp, float ix, fl
   return log2_lod(l[0], l[1], l[2]);
 }
 
+// Whether position p may be valid under BORDER at any level: level m is read
+// at q = p / 2^m - 0.5 (rounded), valid for 0 <= q + 0.5 < dims >> m, and
+// (dims >> m) << m <= dims; one cell of slack covers the roundings.
+NGT_DEVICE bool xform_inside(const Dims& d, float px, float py, float pz) {
+  return (px > -1.f) & (px < static_cast<float>(d.x) + 1.f) & (py > -1.f) & (py < static_cast<float>(d.y) + 1.f) &
+         (pz > -1.f) & (pz < static_cast<float>(d.z) + 1.f);
+}
+
 template <int C, int FM, int BM, int MM>
 __global__ __launch_bounds__(256) void xform_fwd_kernel(XformArgs a, CamBatch cb, MipSet mips,
                                                         float* __restrict__ out) {
@@ -444,8 +468,13 @@ __global__ __launch_bounds__(256) void xform_fwd_kernel(XformArgs a, CamBatch cb
   if constexpr (BM == WRAP) {
     r = vzero<C>();  // Sampler2 has no WRAP path (sampling.hpp:802-826)
   } else if constexpr (MM != NGT_MIP_NONE) {
-    const float lod = xform_lod(a, cp, ix, iy, iz, px, py, pz);
-    r = read_mip<C, FM, BM, MM>(mips, cp.data_index, px, py, pz, lod, a.mip_bias, 0.5f);
+    r = vzero<C>();
+    // a position outside the finest level's valid range is outside every
+    // level's, and most of a frustum is: no LoD, no reads (BORDER, LINEAR)
+    if (!(FM == LINEAR && BM == BORDER) || xform_inside(a.din, px, py, pz)) {
+      const float lod = xform_lod(a, cp, ix, iy, iz, px, py, pz);
+      r = read_mip<C, FM, BM, MM>(mips, cp.data_index, px, py, pz, lod, a.mip_bias, 0.5f);
+    }
   } else if constexpr (FM == LINEAR) {
     r = read_linear<C, BM>(a.input + cp.data_index * in_slice, a.din, px - 0.5f, py - 0.5f, pz - 0.5f);
   } else if constexpr (FM == QUADRATIC) {
@@ -492,6 +521,222 @@ __global__ __launch_bounds__(256) void xform_bwd_kernel(XformArgs a, CamBatch cb
     if constexpr (FM == LINEAR) scatter_linear<C, BM, false>(g, a.din, px - 0.5f, py - 0.5f, pz - 0.5f, dy);
     else if constexpr (FM == QUADRATIC) scatter_quadratic<C, BM>(g, a.din, px - 0.5f, py - 0.5f, pz - 0.5f, dy);
     else scatter_nearest<C, BM>(g, a.din, px - 0.5f, py - 0.5f, pz - 0.5f, dy);
+  }
+}
+
+// ------------------------------------------- transform adjoint as a gather ---
+// The exact adjoint of LINEAR BORDER sampling in the forward modes, without
+// global atomics: one work-group per brick of voxels of one level takes the
+// output cells whose positions can fall into the brick's trilinear support -
+// the bounding box, in output cells, of the support's 8 corners mapped through
+// the camera - and adds the corner contributions of those that do to fp64
+// accumulators in LDS (ds_add_f64, 3 to 7 lanes per clock and CU); the brick's
+// voxels are then stored once, so nothing has to be cleared first.  Global
+// fp32 atomics scatter at 21 to 85 G/s here: the frustum adjoint of a 96^3 grid
+// of 4 channels with 2 mips into three 128x72x96 views took 1697 us, this 96:
+// about 25 us of it finding the boxes and storing the voxels, 30 testing the
+// candidates (2 to 3 for each sample in the support), the rest the LoDs, the
+// gradients' loads and 11 us of LDS atomics.
+//
+// The accumulator is the brick grown by one cell on every side, so that the 8
+// corners of every sample whose floor cell lies in b0 - 1 .. b1 land in it.
+struct BrickList {
+  int nx, ny, nz;
+  __host__ __device__ int count() const { return nx * ny * nz; }
+};
+
+// The output index that object position p maps to, and the clip-space w (not
+// positive behind the camera).  Linear depth is taken from view space, where
+// it is affine in p.
+template <typename T>
+NGT_HOST_DEVICE_INLINE T output_index(const CamParams& cp, const Dims& d, bool linear_depth, T x, T y, T z, T o[3]) {
+  T v[4], c[4];
+  for (int r = 0; r < 4; ++r) v[r] = cp.mv[4 * r] * x + cp.mv[4 * r + 1] * y + cp.mv[4 * r + 2] * z + cp.mv[4 * r + 3];
+  for (int r = 0; r < 4; ++r)
+    c[r] = cp.p[4 * r] * v[0] + cp.p[4 * r + 1] * v[1] + cp.p[4 * r + 2] * v[2] + cp.p[4 * r + 3] * v[3];
+  o[0] = (c[0] / c[3] * T(0.5) + T(0.5)) * d.x;
+  o[1] = (c[1] / c[3] * T(0.5) + T(0.5)) * d.y;
+  o[2] = linear_depth ? -(v[2] + cp.near_) / (cp.far_ - cp.near_) * d.z : (c[2] / c[3] * T(0.5) + T(0.5)) * d.z;
+  return c[3];
+}
+
+// A brick of level m: BX x BY x BZ voxels of the finest level, 8x4x4 of the
+// next and 4x4x4 of the ones after, whose voxels see 8 and 64 times the
+// samples and which are few.
+template <int BX, int BY, int BZ>
+NGT_HOST_DEVICE_INLINE Dims level_brick(int m) {
+  return m == 0 ? Dims{BX, BY, BZ} : (m == 1 ? Dims{8, 4, 4} : Dims{4, 4, 4});
+}
+
+template <int BX, int BY, int BZ>
+NGT_HOST_DEVICE_INLINE BrickList level_bricks(const Dims& d, int m) {
+  const Dims dm = level_dims(d, m), b = level_brick<BX, BY, BZ>(m);
+  return BrickList{(dm.x + b.x - 1) / b.x, (dm.y + b.y - 1) / b.y, (dm.z + b.z - 1) / b.z};
+}
+
+typedef __attribute__((address_space(3))) double lds_double;
+NGT_DEVICE void lds_add(double* t, float v) {
+  __hip_atomic_fetch_add((lds_double*)t, static_cast<double>(v), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+}
+
+// i / n and i % n for 0 <= i < 2^30, n > 0, from a float estimate that is off
+// by at most a few hundred (by one for i below 2^22).
+NGT_DEVICE int div_rem(int i, int n, float inv, int& rem) {
+  int q = static_cast<int>(static_cast<float>(i) * inv);
+  rem = i - q * n;
+  while (rem < 0) { rem += n; --q; }
+  while (rem >= n) { rem -= n; ++q; }
+  return q;
+}
+
+template <int C, int MM, int BX, int BY, int BZ>
+__global__ __launch_bounds__(256) void xform_bwd_gather_kernel(XformArgs a, CamBatch cb, MipSet grad,
+                                                               const float* __restrict__ out_grad, int accumulate) {
+  static_assert(BX >= 8 && BY >= 4 && BZ >= 4, "the coarser levels' bricks fit the finest one's accumulator");
+  // one plane per channel: consecutive cells on consecutive banks
+  constexpr int NP = (BX + 2) * (BY + 2) * (BZ + 2);
+  __shared__ double acc[NP * C];
+  __shared__ int box[kMaxCamsPerLaunch][6];  // x0, y0, z0 and the extents (0: view skipped)
+  const int tid = threadIdx.x;
+  // the coarsest level's bricks, which see the most samples, come first
+  int bid = blockIdx.x, m = grad.num_levels;
+  BrickList bl = level_bricks<BX, BY, BZ>(grad.d0, m);
+  while (m > 0 && bid >= bl.count() * grad.n_data) {
+    bid -= bl.count() * grad.n_data;
+    bl = level_bricks<BX, BY, BZ>(grad.d0, --m);
+  }
+  const int n = bid / bl.count(), brem = bid % bl.count();
+  Dims dm;
+  float* const out = level_ptr<C>(grad, n, m, dm);
+  const Dims lb = level_brick<BX, BY, BZ>(m);
+  const int PX = lb.x + 2, PXY = PX * (lb.y + 2);
+  const int b0x = brem % bl.nx * lb.x, b0y = brem / bl.nx % bl.ny * lb.y, b0z = brem / (bl.nx * bl.ny) * lb.z;
+  const int b1x = min(b0x + lb.x, dm.x) - 1, b1y = min(b0y + lb.y, dm.y) - 1, b1z = min(b0z + lb.z, dm.z) - 1;
+  for (int i = tid; i < NP * C; i += 256) acc[i] = 0.0;
+
+  // lane = view * 8 + corner of the support box, in finest-level cells
+  if (tid < 64) {
+    const int ci = tid >> 3, c = tid & 7;
+    const bool view = ci < cb.count && cb.cam[ci < cb.count ? ci : 0].data_index == n;
+    const float s = static_cast<float>(1 << m);
+    float lo[3] = {3.0e38f, 3.0e38f, 3.0e38f}, hi[3] = {-3.0e38f, -3.0e38f, -3.0e38f};
+    int unknown = 0;
+    if (view) {
+      const CamParams& cp = cb.cam[ci];
+      const float px = s * ((c & 1) ? static_cast<float>(b1x) + 1.502f : static_cast<float>(b0x) - 0.502f);
+      const float py = s * ((c & 2) ? static_cast<float>(b1y) + 1.502f : static_cast<float>(b0y) - 0.502f);
+      const float pz = s * ((c & 4) ? static_cast<float>(b1z) + 1.502f : static_cast<float>(b0z) - 0.502f);
+      float o[3];
+      const float cw = output_index<float>(cp, a.dout, a.coord_mode != NGT_COORD_TRANSFORM, px, py, pz, o);
+      // behind the camera, or no number: every output cell is a candidate
+      unknown = !(cw > 0.f) || !(fabsf(o[0]) < 1.0e9f) || !(fabsf(o[1]) < 1.0e9f) || !(fabsf(o[2]) < 1.0e9f);
+#pragma unroll
+      for (int k = 0; k < 3; ++k) lo[k] = hi[k] = o[k];
+    }
+#pragma unroll
+    for (int off = 1; off < 8; off <<= 1) {
+#pragma unroll
+      for (int k = 0; k < 3; ++k) {
+        lo[k] = fminf(lo[k], __shfl_xor(lo[k], off, 64));
+        hi[k] = fmaxf(hi[k], __shfl_xor(hi[k], off, 64));
+      }
+      unknown |= __shfl_xor(unknown, off, 64);
+    }
+    if (c == 0 && ci < cb.count) {
+      const int dims[3] = {a.dout.x, a.dout.y, a.dout.z};
+      int ext[3], at[3];
+#pragma unroll
+      for (int k = 0; k < 3; ++k) {
+        // cell i has its centre at index i + 0.5; 0.1 cells cover the rounding
+        // of the two maps (checked on the host)
+        const float f = static_cast<float>(dims[k]);
+        const int i0 = unknown ? 0 : max(0, static_cast<int>(ceilf(fminf(fmaxf(lo[k], -2.f), f + 2.f) - 0.6f)));
+        const int i1 = unknown ? dims[k] - 1
+                               : min(dims[k] - 1, static_cast<int>(floorf(fminf(fmaxf(hi[k], -2.f), f + 2.f) - 0.4f)));
+        at[k] = i0;
+        ext[k] = view ? max(0, i1 - i0 + 1) : 0;
+      }
+      const bool empty = ext[0] == 0 || ext[1] == 0 || ext[2] == 0;
+#pragma unroll
+      for (int k = 0; k < 3; ++k) {
+        box[ci][k] = at[k];
+        box[ci][3 + k] = empty ? 0 : ext[k];
+      }
+    }
+  }
+  __syncthreads();
+
+  const float sc = level_scale(m);
+  const float fdx = static_cast<float>(dm.x), fdy = static_cast<float>(dm.y), fdz = static_cast<float>(dm.z);
+  const int64_t out_cells = static_cast<int64_t>(a.dout.x) * a.dout.y * a.dout.z;
+  bool any = false;
+  for (int ci = 0; ci < cb.count; ++ci) {
+    const int nx = box[ci][3], ny = box[ci][4], total = nx * ny * box[ci][5];
+    if (total == 0) continue;
+    any = true;
+    const CamParams& cp = cb.cam[ci];
+    const float* const g = out_grad + static_cast<int64_t>(cp.out_index) * out_cells * C;
+    const float inv_nx = 1.f / static_cast<float>(nx), inv_ny = 1.f / static_cast<float>(ny);
+    for (int i = tid; i < total; i += 256) {
+      int x, y;
+      const int row = div_rem(i, nx, inv_nx, x);
+      const int z = box[ci][2] + div_rem(row, ny, inv_ny, y);
+      x += box[ci][0]; y += box[ci][1];
+      // every candidate's gradient is loaded, so that the load is in flight
+      // while the position is formed
+      const Vec<C> dy = vload<C>(g + cell_offset(a.dout, x, y, z) * C);
+      const float ix = static_cast<float>(x) + 0.5f, iy = static_cast<float>(y) + 0.5f, iz = static_cast<float>(z) + 0.5f;
+      float px, py, pz;
+      xform_pos(a, cp, ix, iy, iz, px, py, pz);
+      const float qx = px * sc - 0.5f, qy = py * sc - 0.5f, qz = pz * sc - 0.5f;
+      const float fx = floorf(qx), fy = floorf(qy), fz = floorf(qz);
+      const float lx = fx - static_cast<float>(b0x - 1), ly = fy - static_cast<float>(b0y - 1),
+                  lz = fz - static_cast<float>(b0z - 1);
+      // the forward's validity, and the floor cell in b0 - 1 .. b1
+      if (!((qx + 0.5f >= 0.f) & (qx + 0.5f < fdx) & (qy + 0.5f >= 0.f) & (qy + 0.5f < fdy) & (qz + 0.5f >= 0.f) &
+            (qz + 0.5f < fdz) & (lx >= 0.f) & (lx <= static_cast<float>(b1x - b0x + 1)) & (ly >= 0.f) &
+            (ly <= static_cast<float>(b1y - b0y + 1)) & (lz >= 0.f) & (lz <= static_cast<float>(b1z - b0z + 1))))
+        continue;
+      float weight = 1.f;
+      if constexpr (MM != NGT_MIP_NONE) {
+        const MipPick k = mip_pick<MM>(xform_lod(a, cp, ix, iy, iz, px, py, pz), a.mip_bias, grad.num_levels);
+        if (k.lf == m) weight = 1.f - k.wc;
+        else if (k.two && k.lc == m) weight = k.wc;
+        else continue;
+      }
+      const Vec<C> val = vscale(dy, weight);
+      const float wx = qx - fx, wy = qy - fy, wz = qz - fz;
+      const float fw[2][3] = {{1.f - wx, 1.f - wy, 1.f - wz}, {wx, wy, wz}};
+      // an integer coordinate's ceil corner is its floor corner
+      const int sx = wx != 0.f ? 1 : 0, sy = wy != 0.f ? PX : 0, sz = wz != 0.f ? PXY : 0;
+      double* const t = acc + static_cast<int>(lz) * PXY + static_cast<int>(ly) * PX + static_cast<int>(lx);
+#pragma unroll
+      for (int k = 0; k < 8; ++k) {
+        const int bx = k & 1, by = (k >> 1) & 1, bz = k >> 2;
+        const float w = fw[bx][0] * fw[by][1] * fw[bz][2];
+        double* const q = t + (bx ? sx : 0) + (by ? sy : 0) + (bz ? sz : 0);
+#pragma unroll
+        for (int j = 0; j < C; ++j) lds_add(q + j * NP, val.v[j] * w);
+      }
+    }
+  }
+  if (accumulate && !any) return;  // uniform
+  __syncthreads();
+  for (int i = tid; i < lb.x * lb.y * lb.z; i += 256) {
+    const int lx = i % lb.x, ly = i / lb.x % lb.y, lz = i / (lb.x * lb.y);  // powers of two, uniform
+    const int x = b0x + lx, y = b0y + ly, z = b0z + lz;
+    if (x > b1x || y > b1y || z > b1z) continue;
+    const double* const t = acc + (lz + 1) * PXY + (ly + 1) * PX + lx + 1;
+    float* const o = out + cell_offset(dm, x, y, z) * C;
+    Vec<C> v;
+#pragma unroll
+    for (int j = 0; j < C; ++j) v.v[j] = static_cast<float>(t[j * NP]);
+    if (accumulate) {
+      const Vec<C> old = vload<C>(o);
+#pragma unroll
+      for (int j = 0; j < C; ++j) v.v[j] += old.v[j];
+    }
+    vstore<C>(o, v);
   }
 }
 
@@ -689,6 +934,63 @@ CamBatch cam_batch(const std::vector<Pair>& pairs, size_t b, const float* M, con
   return cb;
 }
 
+// Whether output_index inverts the forward's positions (output cell -> grid
+// through the inverse matrices, in float as the kernels form them) to 0.02
+// cells on a 3x3x3 lattice of the output: the gather finds its candidates with
+// the one, with 0.1 cells to spare, and takes them by the other.  (It does not
+// for a singular matrix, whose inverse is taken as 0, nor where a depth range
+// of many orders costs the projection its float digits.)
+bool maps_agree(const CamParams& cp, const Dims& dout, int coord_mode) {
+  const float dims[3] = {static_cast<float>(dout.x), static_cast<float>(dout.y), static_cast<float>(dout.z)};
+  auto apply = [](const float* m, const float v[3], float o[4]) {
+    for (int r = 0; r < 4; ++r) o[r] = m[4 * r] * v[0] + m[4 * r + 1] * v[1] + m[4 * r + 2] * v[2] + m[4 * r + 3];
+  };
+  const bool linear_depth = coord_mode != NGT_COORD_TRANSFORM;
+  for (int i = 0; i < 27; ++i) {
+    const int at[3] = {i % 3, i / 3 % 3, i / 9};
+    float idx[3], ndc[3], v[4], o[4];
+    for (int k = 0; k < 3; ++k) {
+      idx[k] = 0.5f + std::floor(0.5f * static_cast<float>(at[k]) * (dims[k] - 1.f));
+      ndc[k] = idx[k] / dims[k] * 2.f - 1.f;
+    }
+    if (linear_depth)
+      ndc[2] = -cp.p[10] - cp.p[11] / -((cp.far_ - cp.near_) * (idx[2] / dims[2]) + cp.near_);
+    apply(cp.p_inv, ndc, v);
+    const float iw = 1.f / v[3];
+    for (int k = 0; k < 3; ++k) v[k] *= iw;
+    apply(cp.mv_inv, v, o);
+    double back[3];
+    const double w = output_index<double>(cp, dout, linear_depth, o[0], o[1], o[2], back);
+    if (!(w > 0.0)) return false;
+    for (int k = 0; k < 3; ++k)
+      if (!(std::fabs(back[k] - idx[k]) < 0.02)) return false;
+  }
+  return true;
+}
+
+// The gather serves LINEAR, BORDER and the forward modes, for cameras whose
+// maps agree; other calls scatter.
+bool use_xform_gather(const std::vector<Pair>& pairs, const float* M, const float* V, const float* P, const float* F,
+                      const XformArgs& a, int64_t n_data, int interpolation, int boundary) {
+  if (interpolation != LINEAR || boundary != BORDER) return false;
+  if (a.coord_mode != NGT_COORD_TRANSFORM && a.coord_mode != NGT_COORD_TRANSFORM_LINDEPTH) return false;
+  if (dims_cells(a.dout) >= (int64_t(1) << 30) || dims_cells(a.din) * n_data >= (int64_t(1) << 36)) return false;
+  for (const Pair& p : pairs)
+    if (!maps_agree(make_cam(M + 16 * p.n, V + 16 * p.v, P + 16 * p.v, F + 6 * p.v, p.n, p.out), a.dout, a.coord_mode))
+      return false;
+  return true;
+}
+
+template <int C, int MM, int BX, int BY, int BZ>
+void launch_xform_gather(const XformArgs& a, const CamBatch& cb, const MipSet& grad, const float* out_grad,
+                         int accumulate, hipStream_t s) {
+  int64_t bricks = 0;
+  for (int m = 0; m <= grad.num_levels; ++m)
+    bricks += static_cast<int64_t>(level_bricks<BX, BY, BZ>(grad.d0, m).count()) * grad.n_data;
+  hipLaunchKernelGGL((xform_bwd_gather_kernel<C, MM, BX, BY, BZ>), dim3(static_cast<unsigned>(bricks)), dim3(256), 0, s,
+                     a, cb, grad, out_grad, accumulate);
+}
+
 }  // namespace
 }  // namespace ngt
 
@@ -870,6 +1172,22 @@ int ngt_sample_grid_transform_bwd(const float* input, const int64_t* input_shape
   const bool mip = mipmapping != NGT_MIP_NONE;
   const MipSet grad = make_mips(input_grad, input_shape, mip ? workspace : nullptr, mip ? num_mipmaps : 0);
   hipStream_t s = as_stream(stream);
+  if (!ref && use_xform_gather(pairs, matrix_m, matrix_v, matrix_p, frustum, a, si.n, interpolation, boundary)) {
+    for (size_t b = 0; b < pairs.size(); b += kMaxCamsPerLaunch) {
+      const CamBatch cb = cam_batch(pairs, b, matrix_m, matrix_v, matrix_p, frustum);
+      // 8x8x8 bricks visit fewer samples twice and pay fewer prologues than
+      // 8x4x4 ones (64^3 grid of 1 channel into 96^3 cells 17.5 us against
+      // 21.2; 96^3 of 4 channels into frustums 96 against 110), which keep the
+      // CUs busy on grids too small to give each two; 16x8x8 leave them too
+      // few and too uneven (22.2 and 160 us)
+      const bool large = level_bricks<8, 8, 8>(grad.d0, 0).count() * si.n >= 512;
+      NGT_SWITCH_C(si.c, NGT_SWITCH_MM(mipmapping,
+          if (large) launch_xform_gather<CC, MMM, 8, 8, 8>(a, cb, grad, output_grad, b > 0, s);
+          else launch_xform_gather<CC, MMM, 8, 4, 4>(a, cb, grad, output_grad, b > 0, s)));
+    }
+    if (mip) NGT_SWITCH_C(si.c, launch_mip_collapse<CC>(grad, s));
+    return check_launch("ngt_sample_grid_transform_bwd");
+  }
   fill_zero(input_grad, si.elems(), s);
   uint32_t* hits = ref ? static_cast<uint32_t*>(workspace) : nullptr;
   if (ref) fill_zero_u32(hits, si.n * si.cells(), s);
