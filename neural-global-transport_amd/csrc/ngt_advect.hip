@@ -429,12 +429,6 @@ inline BrickGrid brick_grid(const Dims& d, int64_t pairs) {
   return deep.count() * pairs < kFewBricks ? brick_grid_of_depth(d, 2) : deep;
 }
 
-// fp64 atomic add into LDS (ds_add_f64); t must point into __shared__ memory.
-typedef __attribute__((address_space(3))) double lds_double;
-NGT_DEVICE void lds_add(double* t, float v) {
-  __hip_atomic_fetch_add((lds_double*)t, static_cast<double>(v), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-}
-
 // Scatter val * w to the 8 corners of q: into the LDS tile (origin o*, that
 // many planes) when the corner lies in it, else atomically into `ovf`, every `ovf_step`-th
 // value of a full field.

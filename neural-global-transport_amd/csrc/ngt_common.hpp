@@ -113,12 +113,13 @@ NGT_DEVICE float vdot(const Vec<C>& a, const Vec<C>& b) {
 // Hardware fp32 atomic add (global_atomic_add_f32, no CAS loop).
 NGT_DEVICE void atomic_add(float* p, float v) { unsafeAtomicAdd(p, v); }
 
-// fp32 atomic add into LDS (ds_add_f32).  p must point into __shared__
-// memory: a plain float* reaching an atomic is otherwise compiled as a flat
-// atomic, which goes through the vector-memory path.
-typedef __attribute__((address_space(3))) float lds_float;
-NGT_DEVICE void lds_add(float* p, float v) {
-  __hip_atomic_fetch_add((lds_float*)p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+// fp64 atomic add into LDS (ds_add_f64: 3 to 7 lanes per clock and CU; ds_add_f32
+// runs at 0.33).  p must point into __shared__ memory: a plain double* reaching
+// an atomic is otherwise compiled as a flat atomic, which goes through the
+// vector-memory path.
+typedef __attribute__((address_space(3))) double lds_double;
+NGT_DEVICE void lds_add(double* p, float v) {
+  __hip_atomic_fetch_add((lds_double*)p, static_cast<double>(v), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
 }
 
 // Block coordinates of a work-group's tile.  Kernel bodies take them as an
@@ -152,6 +153,12 @@ struct Corners {
   bool inside;                  // BORDER forward validity of the position
 };
 
+NGT_DEVICE bool inside_border(const Dims& d, float qx, float qy, float qz) {
+  return (qx + 0.5f >= 0.f) & (qx + 0.5f < static_cast<float>(d.x)) &
+         (qy + 0.5f >= 0.f) & (qy + 0.5f < static_cast<float>(d.y)) &
+         (qz + 0.5f >= 0.f) & (qz + 0.5f < static_cast<float>(d.z));
+}
+
 template <int BM>
 NGT_DEVICE Corners make_corners(const Dims& d, float qx, float qy, float qz) {
   Corners c;
@@ -161,9 +168,7 @@ NGT_DEVICE Corners make_corners(const Dims& d, float qx, float qy, float qz) {
   c.x1 = static_cast<int>(ceilf(qx)); c.y1 = static_cast<int>(ceilf(qy)); c.z1 = static_cast<int>(ceilf(qz));
   if constexpr (BM == BORDER) {
     // bitwise & keeps the masks branch-free
-    c.inside = (qx + 0.5f >= 0.f) & (qx + 0.5f < static_cast<float>(d.x)) &
-               (qy + 0.5f >= 0.f) & (qy + 0.5f < static_cast<float>(d.y)) &
-               (qz + 0.5f >= 0.f) & (qz + 0.5f < static_cast<float>(d.z));
+    c.inside = inside_border(d, qx, qy, qz);
     c.vx0 = (c.x0 > -1) & (c.x0 < d.x); c.vx1 = (c.x1 > -1) & (c.x1 < d.x);
     c.vy0 = (c.y0 > -1) & (c.y0 < d.y); c.vy1 = (c.y1 > -1) & (c.y1 < d.y);
     c.vz0 = (c.z0 > -1) & (c.z0 < d.z); c.vz1 = (c.z1 > -1) & (c.z1 < d.z);
