@@ -495,7 +495,10 @@ __global__ __launch_bounds__(256) void raymarch_bwd_exact_kernel(RayArgs a, CamB
 constexpr int kGPix = 8, kGQuad = 4;
 inline __host__ __device__ int64_t g_pixels(int64_t npix) { return (npix + kGPix - 1) / kGPix * kGPix; }
 // offset of sample k from sample 0 of the same pixel
-NGT_DEVICE int64_t g_step(int k) { return static_cast<int64_t>(k / kGQuad) * (kGPix * kGQuad) + k % kGQuad; }
+NGT_DEVICE uint32_t g_step(int k) {
+  const uint32_t u = static_cast<uint32_t>(k);
+  return u / kGQuad * (kGPix * kGQuad) + u % kGQuad;
+}
 NGT_DEVICE int64_t g_offset(int k, int64_t pixel, int kcap) {
   return (pixel / kGPix) * kcap * kGPix + (pixel % kGPix) * kGQuad + g_step(k);
 }
@@ -719,24 +722,16 @@ __global__ __launch_bounds__(256) void raymarch_fwd_record_kernel(RayArgs a, Cam
   raymarch_fwd_record_kernel_body<MODE>(vb, a, cb, out, pair_base, G, rays, bound, kcap, grid_slot(vb));
 }
 
-// Inclusive scan of one int per work-item over a 256-wide work-group: a
-// shuffle scan inside each wavefront, then the wavefront totals through LDS
-// (one barrier).  The caller synchronises before s_wtot is written again.
-NGT_DEVICE int block_inclusive_scan(int v, int* s_wtot) {
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-#pragma unroll
-  for (int o = 1; o < 64; o <<= 1) {
-    const int t = __shfl_up(v, o, 64);
-    if (lane >= o) v += t;
-  }
-  if (lane == 63) s_wtot[wave] = v;
-  __syncthreads();
-  int pre = 0;
-#pragma unroll
-  for (int w = 0; w < 3; ++w)
-    if (w < wave) pre += s_wtot[w];
-  return v + pre;
+// Orders a wavefront's LDS writes before its later reads by other lanes (its
+// LDS operations run in order: no wait, only the compiler's order).
+NGT_DEVICE void wave_lds_sync() {
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
 }
+
+// Where positions leave a BORDER grid of n cells: q + 0.5f < n in float is
+// q < border_end(n).  (n = 1 has the one q below n - 0.5 that rounds up to it.)
+NGT_DEVICE float border_end(int n) { return n == 1 ? 0.5f - 0x1p-25f : static_cast<float>(n) - 0.5f; }
 
 // Pass 2: one work-group per brick of BX x BY x BZ voxels.  For every view it
 // projects the brick's sample-support box (positions whose trilinear corners
@@ -850,24 +845,43 @@ NGT_DEVICE void raymarch_bwd_brick_kernel_body(const VBlock& vb, const RayArgs& 
 
   const int64_t npix = static_cast<int64_t>(a.out_w) * a.out_h;
   const int total = ray_begin[cb.count];
-  const int fb0m1x = b0x - 1, fb0m1y = b0y - 1, fb0m1z = b0z - 1;
+  // first rays of views 1 .. 7 in the brick's list, in scalar registers
+  int begins[kMaxCamsPerLaunch - 1];
+#pragma unroll
+  for (int c = 1; c < kMaxCamsPerLaunch; ++c)
+    begins[c - 1] = c < cb.count ? __builtin_amdgcn_readfirstlane(ray_begin[c]) : total;
   // ray r of the brick's list (r < total): its record, and the G offset of its sample 0
   auto fetch_ray = [&](int r, RayRec& rr, int64_t& gofs) {
     int ci = 0;
-    while (ci + 1 < cb.count && r >= ray_begin[ci + 1]) ++ci;
-    const int local = r - ray_begin[ci];
-    const int px = rect[ci][0] + local % rect[ci][2];
-    const int py = rect[ci][1] + local / rect[ci][2];
-    gofs = static_cast<int64_t>(pair_base + ci) * kcap * g_pixels(npix) +
-           g_offset(0, static_cast<int64_t>(py) * a.out_w + px, kcap);
-    rr = rays[(pair_base + ci) * static_cast<int>(npix) + py * a.out_w + px];
+#pragma unroll
+    for (int c = 1; c < kMaxCamsPerLaunch; ++c) ci += r >= begins[c - 1] ? 1 : 0;
+    const int local = r - ray_begin[ci], nx = rect[ci][2];
+    // local / nx: the float quotient is at most one off
+    int row = static_cast<int>(static_cast<float>(local) * __builtin_amdgcn_rcpf(static_cast<float>(nx)));
+    int col = local - row * nx;
+    if (col < 0) { --row; col += nx; }
+    if (col >= nx) { ++row; col -= nx; }
+    const uint32_t pixel = static_cast<uint32_t>((rect[ci][1] + row) * a.out_w + rect[ci][0] + col);
+    const uint32_t pair = static_cast<uint32_t>(pair_base + ci);
+    gofs = static_cast<int64_t>(static_cast<uint64_t>(pair * static_cast<uint32_t>(g_pixels(npix) / kGPix) +
+                                                      pixel / kGPix) *
+                                static_cast<uint32_t>(kcap * kGPix)) +
+           pixel % kGPix * kGQuad;
+    rr = rays[pair * static_cast<uint32_t>(npix) + pixel];
   };
+  // Rays are taken 256 at a time, every fourth one by a wavefront: the samples
+  // that its lanes add at one time are then some cells apart (neighbouring rays
+  // add to the same cells, and equal addresses in one LDS atomic are taken one
+  // by one: 340 -> 293 us at 160^3 x 8 views of 480x270, the rays there being
+  // closer than cells)
+  const int lane = tid & 63, wave = tid >> 6;
+  const int slot = lane * 4 + wave;
   // each work-item's ray of the next chunk is loaded one chunk ahead, so that
   // its latency overlaps the current chunk's samples (the first one overlaps
   // the gradient bounds' loads)
   RayRec next_rr{};
   int64_t next_gofs = 0;
-  if (tid < total) fetch_ray(tid, next_rr, next_gofs);
+  if (slot < total) fetch_ray(slot, next_rr, next_gofs);
   // the brick's fixed-point unit from the largest gradient bound of its rays' tiles
   {
     float m = 0.f;
@@ -898,7 +912,12 @@ NGT_DEVICE void raymarch_bwd_brick_kernel_body(const VBlock& vb, const RayArgs& 
   // |contribution| <= wmax < 2^e  ->  |contribution * 2^S| < 2^30 with S = 30 - e
   const int S = wmax > 0.f && finite ? 30 - ilogbf(wmax) - 1 : 0;
 
-  const float fdx = static_cast<float>(a.din.x), fdy = static_cast<float>(a.din.y), fdz = static_cast<float>(a.din.z);
+  // the samples that count: inside the grid, floor cell in b0 - 1 .. b1
+  const float fox = static_cast<float>(b0x - 1), foy = static_cast<float>(b0y - 1), foz = static_cast<float>(b0z - 1);
+  const float qlx = fmaxf(fox, -0.5f), qly = fmaxf(foy, -0.5f), qlz = fmaxf(foz, -0.5f);
+  const float qhx = fminf(static_cast<float>(b1x + 1), border_end(a.din.x));
+  const float qhy = fminf(static_cast<float>(b1y + 1), border_end(a.din.y));
+  const float qhz = fminf(static_cast<float>(b1z + 1), border_end(a.din.z));
   // the support box widened by 1e-3 cells: far above the rounding of the
   // slab test, so no sample in the box is lost; the per-sample test below
   // decides exactly
@@ -906,25 +925,27 @@ NGT_DEVICE void raymarch_bwd_brick_kernel_body(const VBlock& vb, const RayArgs& 
                         static_cast<float>(b0z) - 0.501f};
   const float hi3[3] = {static_cast<float>(b1x) + 1.501f, static_cast<float>(b1y) + 1.501f,
                         static_cast<float>(b1z) + 1.501f};
-  // Rays are taken 256 at a time: each work-item clips one ray to the support
-  // box (slab test) and counts its samples there;
-  // after a block-wide scan the chunk's samples are dealt out in sub-chunks of
-  // kItems, kPer per work-item, and each sample adds its 8 corner
-  // contributions to the accumulator.  (A corner at floor+1 where the
+  // Each work-item clips one ray to the support box (slab test) and counts its
+  // samples there; after a scan over the wavefront the samples of its 64 rays
+  // are dealt out in rounds of kPer per work-item, and each sample adds its 8
+  // corner contributions to the accumulator.  (A corner at floor+1 where the
   // reference uses ceil = floor at integer positions carries weight exactly 0.)
-  // The walk is bound by the latency of its loads at 4 waves / SIMD: 8 samples'
-  // G loads in flight per work-item measured fastest at 128^3 x 5 views (52 us;
-  // 1: 57.7, 4: 54.4; 16 needs more than 128 VGPRs, which halves the waves).
-  constexpr int kItems = 2048, kPer = kItems / 256;
-  __shared__ int s_off[257];
-  __shared__ int s_kb[256];        // each ray's first k in the box minus its first item
-  __shared__ int64_t s_gofs[256];  // G offset of each ray's sample 0
-  __shared__ float4 s_ps[256];     // each ray's start and step x
-  __shared__ float4 s_pd[256];     // each ray's step y, z and loss-gradient scale, offset
-  __shared__ int s_wtot[4];
-  __shared__ unsigned char s_ray[kItems];
+  // The wavefronts do not wait for each other, so that one's address arithmetic
+  // runs beside another's LDS atomics, which bound the kernel about equally.
+  // 128^3 x 5 views of 256x144: 51 -> 46 us, 160^3 x 8 of 480x270: 340 -> 240,
+  // four channels at 96^3 x 5: 125 -> 101 (a work-group-wide scan and deal, with
+  // a barrier before and after each 2048 samples, is what it was measured
+  // against).  6 samples in flight per work-item: 4 take 44.7 / 264 / 102 us,
+  // where 6 take 44.2 / 255 / 100; 9 need more than 128 VGPRs, which halves the
+  // wavefronts (62.5 / 278).
+  constexpr int kMark = 768, kPer = 6;
+  __shared__ int s_kb[256];           // each ray's first k in the box minus its first item
+  __shared__ int64_t s_gofs[256];     // each ray's sample 0 in G
+  __shared__ float4 s_ps[256];        // each ray's start and step x
+  __shared__ float4 s_pd[256];        // each ray's step y, z and loss-gradient scale, offset
+  __shared__ unsigned char s_ray[4][kMark];
   for (int base_r = 0; base_r < total; base_r += 256) {
-    const int r = base_r + tid;
+    const int r = base_r + slot;
     const RayRec rr = next_rr;
     const int64_t gofs = r < total ? next_gofs : 0;
     if (r + 256 < total) fetch_ray(r + 256, next_rr, next_gofs);
@@ -940,7 +961,7 @@ NGT_DEVICE void raymarch_bwd_brick_kernel_body(const VBlock& vb, const RayArgs& 
 #pragma unroll
         for (int ax = 0; ax < 3; ++ax) {
           if (fabsf(dv[ax]) > 1e-30f) {
-            const float inv = 1.f / dv[ax];
+            const float inv = __builtin_amdgcn_rcpf(dv[ax]);
             const float t0 = (lo3[ax] - sv[ax]) * inv, t1 = (hi3[ax] - sv[ax]) * inv;
             lo = fmaxf(lo, fminf(t0, t1));
             hi = fminf(hi, fmaxf(t0, t1));
@@ -956,78 +977,80 @@ NGT_DEVICE void raymarch_bwd_brick_kernel_body(const VBlock& vb, const RayArgs& 
         }
       }
     }
-    // inclusive block scan of the counts
-    const int incl = block_inclusive_scan(cnt, s_wtot);
-    s_off[tid + 1] = incl;
-    if (tid == 0) s_off[0] = 0;
+    int incl = cnt;  // inclusive scan of the counts
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+      const int t = __shfl_up(incl, o, 64);
+      if (lane >= o) incl += t;
+    }
+    const int items = __builtin_amdgcn_readlane(incl, 63);
     s_kb[tid] = k0 - (incl - cnt);
     s_gofs[tid] = gofs;
-    __syncthreads();
-    const int items = s_off[256];
-    for (int i0 = 0; i0 < items; i0 += kItems) {
-      const int i_end = min(i0 + kItems, items);
-      {  // the ray of every sample of this sub-chunk: each ray marks its own range
-        const int r0 = max(s_off[tid], i0), r1 = min(s_off[tid + 1], i_end);
-        for (int i = r0; i < r1; ++i) s_ray[i - i0] = static_cast<unsigned char>(tid);
-      }
-      __syncthreads();
-      // a work-item's kPer samples of the sub-chunk: all their G loads are
-      // issued before any of their atomics
-      float wxs[kPer], wys[kPer], wzs[kPer], gss[kPer], gos[kPer];
-      int cell[kPer];
-      bool oks[kPer];
-      Vec<CG> gvs[kPer];
-#pragma unroll
-      for (int u = 0; u < kPer; ++u) {
-        const int i = i0 + tid + u * 256;
-        oks[u] = false;
-        if (i < i_end) {
-          const int lo_j = s_ray[i - i0];
-          const int k = s_kb[lo_j] + i;
-          const float4 ps = s_ps[lo_j];
-          const float4 pd = s_pd[lo_j];
-          const float kf = static_cast<float>(k);
-          const float qx = fmaf(kf, ps.w, ps.x) - 0.5f;
-          const float qy = fmaf(kf, pd.x, ps.y) - 0.5f;
-          const float qz = fmaf(kf, pd.y, ps.z) - 0.5f;
-          const float fx = floorf(qx), fy = floorf(qy), fz = floorf(qz);
-          wxs[u] = qx - fx; wys[u] = qy - fy; wzs[u] = qz - fz;
-          const int lx = static_cast<int>(fmaxf(fminf(fx, 1e8f), -1e8f)) - fb0m1x;
-          const int ly = static_cast<int>(fmaxf(fminf(fy, 1e8f), -1e8f)) - fb0m1y;
-          const int lz = static_cast<int>(fmaxf(fminf(fz, 1e8f), -1e8f)) - fb0m1z;
-          // forward (BORDER) mask, floor cell in b0-1 .. b1 on every axis
-          oks[u] = (qx + 0.5f >= 0.f) & (qx + 0.5f < fdx) & (qy + 0.5f >= 0.f) & (qy + 0.5f < fdy) &
-                   (qz + 0.5f >= 0.f) & (qz + 0.5f < fdz) & (lx >= 0) & (lx <= b1x - fb0m1x) & (ly >= 0) &
-                   (ly <= b1y - fb0m1y) & (lz >= 0) & (lz <= b1z - fb0m1z);
-          cell[u] = (lz * PY + ly) * PX + lx;
-          gss[u] = pd.z; gos[u] = pd.w;
-          if (oks[u]) gvs[u] = vload<CG>(G + (s_gofs[lo_j] + g_step(k)) * CG);
+    for (int m0 = 0; m0 < items; m0 += kMark) {
+      const int m_end = min(m0 + kMark, items);
+      {  // the ray of every sample of this part: each ray marks its own range
+        const int r0 = max(incl - cnt, m0), r1 = min(incl, m_end);
+#pragma clang loop unroll(disable)
+        for (int i = r0; i < r1; ++i) {
+          s_ray[wave][i - m0] = static_cast<unsigned char>(tid);
+          asm volatile("");  // a few bytes: no fill routine
         }
       }
+      wave_lds_sync();
+      for (int i0 = m0; i0 < m_end; i0 += 64 * kPer) {
+        // a work-item's kPer samples of the sub-chunk: all their G loads are
+        // issued before any of their atomics
+        float wxs[kPer], wys[kPer], wzs[kPer], gss[kPer], gos[kPer];
+        int cell[kPer];
+        bool oks[kPer];
+        Vec<CG> gvs[kPer];
 #pragma unroll
-      for (int u = 0; u < kPer; ++u) {
-        if (!oks[u]) continue;
-        // corner weights: z, then y, then the x pair
-        const float wz0 = 1.f - wzs[u], wy0 = 1.f - wys[u], wx0 = 1.f - wxs[u];
-        const float w00 = wz0 * wy0, w01 = wz0 * wys[u], w10 = wzs[u] * wy0, w11 = wzs[u] * wys[u];
-        const float wyz[4] = {w00, w01, w10, w11};
-        unsigned long long* const p0 = &acc[0][cell[u]];
+        for (int u = 0; u < kPer; ++u) {
+          const int i = i0 + lane + u * 64;
+          oks[u] = false;
+          if (i < m_end) {
+            const int lo_j = s_ray[wave][i - m0];
+            const int k = s_kb[lo_j] + i;
+            const float4 ps = s_ps[lo_j];
+            const float4 pd = s_pd[lo_j];
+            const float kf = static_cast<float>(k);
+            const float qx = fmaf(kf, ps.w, ps.x) - 0.5f;
+            const float qy = fmaf(kf, pd.x, ps.y) - 0.5f;
+            const float qz = fmaf(kf, pd.y, ps.z) - 0.5f;
+            const float fx = floorf(qx), fy = floorf(qy), fz = floorf(qz);
+            wxs[u] = qx - fx; wys[u] = qy - fy; wzs[u] = qz - fz;
+            oks[u] = (qx >= qlx) & (qx < qhx) & (qy >= qly) & (qy < qhy) & (qz >= qlz) & (qz < qhz);
+            // exact in float: below 2^24 where the sample counts
+            cell[u] = static_cast<int>(fmaf(fmaf(fz - foz, PY, fy - foy), PX, fx - fox));
+            gss[u] = pd.z; gos[u] = pd.w;
+            if (oks[u]) gvs[u] = vload<CG>(G + (s_gofs[lo_j] + g_step(k)) * CG);
+          }
+        }
 #pragma unroll
-        for (int ch = 0; ch < CG; ++ch) {
-          const float g = ldexpf(gss[u] * (gvs[u].v[ch] - gos[u]), S);
+        for (int u = 0; u < kPer; ++u) {
+          if (!oks[u]) continue;
+          // corner weights: z, then y, then the x pair
+          const float wz0 = 1.f - wzs[u], wy0 = 1.f - wys[u], wx0 = 1.f - wxs[u];
+          const float w00 = wz0 * wy0, w01 = wz0 * wys[u], w10 = wzs[u] * wy0, w11 = wzs[u] * wys[u];
+          const float wyz[4] = {w00, w01, w10, w11};
+          unsigned long long* const p0 = &acc[0][cell[u]];
 #pragma unroll
-          for (int yz = 0; yz < 4; ++yz) {
-            const float t = g * wyz[yz];
-            const int off = ch * NP + (yz >> 1) * PX * PY + (yz & 1) * PX;
-            // truncation: at most one unit (2^-S) off, far below the sum's rounding
-            const long long c0 = static_cast<long long>(static_cast<int>(t * wx0));
-            const long long c1 = static_cast<long long>(static_cast<int>(t * wxs[u]));
-            atomicAdd(p0 + off, static_cast<unsigned long long>(c0));
-            atomicAdd(p0 + off + 1, static_cast<unsigned long long>(c1));
+          for (int ch = 0; ch < CG; ++ch) {
+            const float g = ldexpf(gss[u] * (gvs[u].v[ch] - gos[u]), S);
+#pragma unroll
+            for (int yz = 0; yz < 4; ++yz) {
+              const float t = g * wyz[yz];
+              const int off = ch * NP + (yz >> 1) * PX * PY + (yz & 1) * PX;
+              // truncation: at most one unit (2^-S) off, far below the sum's rounding
+              const long long c0 = static_cast<long long>(static_cast<int>(t * wx0));
+              const long long c1 = static_cast<long long>(static_cast<int>(t * wxs[u]));
+              atomicAdd(p0 + off, static_cast<unsigned long long>(c0));
+              atomicAdd(p0 + off + 1, static_cast<unsigned long long>(c1));
+            }
           }
         }
       }
-      __syncthreads();  // s_ray is rewritten by the next sub-chunk
+      wave_lds_sync();  // s_ray is written again
     }
   }
   __syncthreads();
@@ -1463,9 +1486,12 @@ void run_gather(const std::vector<Pair>& pairs, const float* M, const float* V, 
                              base, output, output_grad, gp.G, gp.rays, gp.bound, gp.kcap)));
     }
     // bricks: larger ones visit fewer samples twice (the support box is one
-    // cell wider than the brick), but the 64-bit accumulators of 2 or 4
-    // channels must fit the LDS
-    constexpr int BX = 16, BY = 8, BZ = 8;
+    // cell wider than the brick), smaller ones leave room for more work-groups
+    // beside their 64-bit accumulators.  One channel, 128^3 x 5 views / 160^3 x 8:
+    // 16 x 16 x 8 takes 49 / 285 us, 16 x 8 x 8 58 / 306, 8 x 8 x 8 71 / 350,
+    // 16 x 16 x 16 56 / 358; four channels at 96^3 x 5: 8 x 8 x 8 105 us,
+    // 16 x 8 x 8 113.
+    constexpr int BX = 8, BY = 8, BZ = 8;
     constexpr int BX1 = 16, BY1 = 16, BZ1 = 8;
     const int accumulate = b > 0 ? 1 : 0;
     const int CG = LIGHT ? 1 : C;
