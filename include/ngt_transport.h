@@ -316,6 +316,17 @@ int ngt_advect_fwd(const float* input, const int64_t* input_shape, const float* 
                    const float* vel_z, int num_velocities, float timestep, int order, int clamp, int boundary,
                    int separate_velocity_batch, float* output, float* sl_out, void* workspace,
                    size_t workspace_bytes, ngt_stream_t stream);
+/* The MAC components {x, y, z} ([N,D,H,W+1,1], [N,D,H+1,W,1], [N,D+1,H,W,1])
+ * read at each component's faces and multiplied by `scale`: luts {x, y, z} of
+ * [N,D,H,W+1,3] and so on, entry s of table t the LINEAR read of component s
+ * half a cell off along t and s (itself where s = t): the tables of a
+ * velocity's self-advection (data_structures.py:1081-1164).  centered_shape
+ * is [N,D,H,W,1]; boundary BORDER or CLAMP.  _bwd is the exact adjoint; it
+ * overwrites the component gradients. */
+int ngt_mac_component_luts(const float* const* components, const int64_t* centered_shape, float scale, int boundary,
+                           float* const* luts, ngt_stream_t stream);
+int ngt_mac_component_luts_bwd(const float* const* lut_grads, const int64_t* centered_shape, float scale, int boundary,
+                               float* const* component_grads, ngt_stream_t stream);
 /* Gradients: input_grad [N,D,H,W,C]; velocity grads in the velocity layout
  * (vel_x_grad [V,D,H,W,3] centered, or the three face arrays).  All outputs
  * are fully overwritten.  `sl` (nullable) = the sl_out of the forward. */

@@ -371,6 +371,108 @@ __global__ __launch_bounds__(256) void faces_from_centered_grad_kernel(Dims d, i
 }
 
 // ---------------------------------------------------------------------------
+// The three MAC components read at each component's faces (the tables of a
+// velocity's self-advection): table T of component T's grid holds, per face,
+// component T itself and the LINEAR reads of the other two, half a cell off
+// along T and their own axis, all times `scale`.
+struct MacFields {
+  const float* p[3];  // x, y, z components, or their gradients' tables
+};
+struct MacOut {
+  float* p[3];
+};
+
+NGT_DEVICE Dims mac_dims(const Dims& d, int axis) {
+  return Dims{d.x + (axis == 0), d.y + (axis == 1), d.z + (axis == 2)};
+}
+NGT_DEVICE bool mac_has(const Dims& d, int axis, int x, int y, int z) {
+  const Dims m = mac_dims(d, axis);
+  return (x < m.x) & (y < m.y) & (z < m.z);
+}
+
+// One work-item per (instance, corner of a cell): the faces that share its
+// index.  d: extents of the centered grid.  One pass, bound by its 24 corner
+// reads per cell (64^3: 15 us, its adjoint 14), that stands for 6 constant
+// tables copied to the device and expanded, 6 table reads, 3 concatenations and
+// 3 products (and mac_component_luts_bwd_kernel for their adjoints, with
+// gradients of the constant tables that nobody uses): a self-advection of a
+// 64^3 velocity with its gradient 1150 -> 405 us, of which the device 190.
+template <int BM>
+__global__ __launch_bounds__(256) void mac_component_luts_kernel(Dims d, MacFields in, float scale, MacOut out) {
+  const int x = blockIdx.x * kBX + threadIdx.x, y = blockIdx.y * kBY + threadIdx.y;
+  const int z = blockIdx.z % (d.z + 1), n = blockIdx.z / (d.z + 1);
+  if (x > d.x || y > d.y) return;
+#pragma unroll
+  for (int t = 0; t < 3; ++t) {
+    if (!mac_has(d, t, x, y, z)) continue;
+    const Dims dt = mac_dims(d, t);
+    float v[3];
+#pragma unroll
+    for (int s = 0; s < 3; ++s) {
+      const Dims ds = mac_dims(d, s);
+      const float* src = in.p[s] + n * dims_cells(ds);
+      if (s == t) {
+        v[s] = src[cell_offset(ds, x, y, z)];
+      } else {
+        const float q[3] = {static_cast<float>(x), static_cast<float>(y), static_cast<float>(z)};
+        const float qx = q[0] + (t == 0 ? -0.5f : (s == 0 ? 0.5f : 0.f));
+        const float qy = q[1] + (t == 1 ? -0.5f : (s == 1 ? 0.5f : 0.f));
+        const float qz = q[2] + (t == 2 ? -0.5f : (s == 2 ? 0.5f : 0.f));
+        v[s] = read_linear<1, BM>(src, ds, qx, qy, qz).v[0];
+      }
+    }
+    float* o = out.p[t] + (n * dims_cells(dt) + cell_offset(dt, x, y, z)) * 3;
+#pragma unroll
+    for (int s = 0; s < 3; ++s) o[s] = v[s] * scale;
+  }
+}
+
+// Its adjoint as a gather: a face of component S gets its own entry of table S
+// and, from each table T != S, the entries of up to 4 faces, one quarter each:
+// along S, faces s - 1 and s of T's grid (extent n); along T, faces t and t + 1
+// (extent n + 1), of which BORDER leaves out the last one, n, and CLAMP counts
+// faces 0 and n twice for the cell at the end.
+template <int BM>
+__global__ __launch_bounds__(256) void mac_component_luts_bwd_kernel(Dims d, MacFields g, float scale, MacOut out) {
+  static_assert(BM == BORDER || BM == CLAMP, "modes that keep to the neighbouring faces");
+  const int x = blockIdx.x * kBX + threadIdx.x, y = blockIdx.y * kBY + threadIdx.y;
+  const int z = blockIdx.z % (d.z + 1), n = blockIdx.z / (d.z + 1);
+  if (x > d.x || y > d.y) return;
+  const int at[3] = {x, y, z};
+  const int ext[3] = {d.x, d.y, d.z};
+#pragma unroll
+  for (int s = 0; s < 3; ++s) {
+    if (!mac_has(d, s, x, y, z)) continue;
+    const Dims ds = mac_dims(d, s);
+    const int64_t own = n * dims_cells(ds) + cell_offset(ds, x, y, z);
+    float sum = g.p[s][own * 3 + s];
+#pragma unroll
+    for (int t = 0; t < 3; ++t) {
+      if (t == s) continue;
+      const Dims dt = mac_dims(d, t);
+      const float* gt = g.p[t] + n * dims_cells(dt) * 3 + s;
+#pragma unroll
+      for (int b = 0; b < 2; ++b) {  // along T
+        float wt = 0.5f;
+        const int it = at[t] + b;
+        if (BM == BORDER && it == ext[t]) continue;
+        if (BM == CLAMP && (it == 0 || it == ext[t])) wt = 1.f;
+#pragma unroll
+        for (int c = 0; c < 2; ++c) {  // along S
+          const int is = at[s] - 1 + c;
+          if (is < 0 || is >= ext[s]) continue;
+          int i[3] = {x, y, z};
+          i[t] = it;
+          i[s] = is;
+          sum += 0.5f * wt * gt[cell_offset(dt, i[0], i[1], i[2]) * 3];
+        }
+      }
+    }
+    out.p[s][own] = sum * scale;
+  }
+}
+
+// ---------------------------------------------------------------------------
 // Brick-tiled exact backward.  A work-group owns a brick of
 // kBrickX x kBrickY x kBrickZ cells and an LDS tile of the brick grown by
 // kHalo cells on every side.  The trilinear scatter of the brick's samples
@@ -868,6 +970,19 @@ int plan_advect(const int64_t* input_shape, const float* vx, const float* vy, co
   return NGT_OK;
 }
 
+int check_mac(const float* const* in, const int64_t* centered_shape, int boundary, float* const* out, Dims& d, int& n) {
+  const int rc = check_grid_shape(centered_shape, "centered", true);
+  if (rc) return rc;
+  NGT_REQUIRE(centered_shape[4] == 1, NGT_ERR_INVALID_ARGUMENT, "MAC components have one channel");
+  NGT_REQUIRE(boundary == BORDER || boundary == CLAMP, NGT_ERR_UNIMPLEMENTED, "boundary must be BORDER or CLAMP");
+  NGT_REQUIRE(in && out && in[0] && in[1] && in[2] && out[0] && out[1] && out[2], NGT_ERR_INVALID_ARGUMENT,
+              "all three components must be given");
+  const Shape5 s5 = shape5(centered_shape);
+  d = s5.dims();
+  n = static_cast<int>(s5.n);
+  return NGT_OK;
+}
+
 dim3 adv_grid(const AdvPlan& p) {
   return dim3(blocks_for(p.a.d.x, kBX), blocks_for(p.a.d.y, kBY), static_cast<unsigned>(p.a.d.z * p.pairs));
 }
@@ -1133,6 +1248,38 @@ int ngt_advect_fwd(const float* input, const int64_t* input_shape, const float* 
       NGT_SWITCH_CLAMP(clamp,
           hipLaunchKernelGGL((advect_mc_kernel<CC, BB, KK>), grid, block, 0, s, p.a, input, sl, output))));
   return check_launch("ngt_advect_fwd");
+}
+
+int ngt_mac_component_luts(const float* const* components, const int64_t* centered_shape, float scale, int boundary,
+                           float* const* luts, ngt_stream_t stream) {
+  Dims d;
+  int n = 0;
+  const int rc = check_mac(components, centered_shape, boundary, luts, d, n);
+  if (rc) return rc;
+  const MacFields in{{components[0], components[1], components[2]}};
+  const MacOut out{{luts[0], luts[1], luts[2]}};
+  const dim3 grid(blocks_for(d.x + 1, kBX), blocks_for(d.y + 1, kBY), static_cast<unsigned>((d.z + 1) * n));
+  if (boundary == BORDER)
+    hipLaunchKernelGGL(mac_component_luts_kernel<BORDER>, grid, dim3(kBX, kBY), 0, as_stream(stream), d, in, scale, out);
+  else
+    hipLaunchKernelGGL(mac_component_luts_kernel<CLAMP>, grid, dim3(kBX, kBY), 0, as_stream(stream), d, in, scale, out);
+  return check_launch("ngt_mac_component_luts");
+}
+
+int ngt_mac_component_luts_bwd(const float* const* lut_grads, const int64_t* centered_shape, float scale, int boundary,
+                               float* const* component_grads, ngt_stream_t stream) {
+  Dims d;
+  int n = 0;
+  const int rc = check_mac(lut_grads, centered_shape, boundary, component_grads, d, n);
+  if (rc) return rc;
+  const MacFields g{{lut_grads[0], lut_grads[1], lut_grads[2]}};
+  const MacOut out{{component_grads[0], component_grads[1], component_grads[2]}};
+  const dim3 grid(blocks_for(d.x + 1, kBX), blocks_for(d.y + 1, kBY), static_cast<unsigned>((d.z + 1) * n));
+  if (boundary == BORDER)
+    hipLaunchKernelGGL(mac_component_luts_bwd_kernel<BORDER>, grid, dim3(kBX, kBY), 0, as_stream(stream), d, g, scale, out);
+  else
+    hipLaunchKernelGGL(mac_component_luts_bwd_kernel<CLAMP>, grid, dim3(kBX, kBY), 0, as_stream(stream), d, g, scale, out);
+  return check_launch("ngt_mac_component_luts_bwd");
 }
 
 int ngt_advect_bwd(const float* input, const int64_t* input_shape, const float* vel_x, const float* vel_y,

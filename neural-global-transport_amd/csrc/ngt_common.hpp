@@ -142,6 +142,10 @@ NGT_DEVICE int wrap_index(int i, int m) {
   return r < 0 ? r + m : r;
 }
 
+__host__ __device__ inline int64_t dims_cells(const Dims& d) {
+  return static_cast<int64_t>(d.x) * d.y * d.z;
+}
+
 NGT_DEVICE int64_t cell_offset(const Dims& d, int x, int y, int z) {
   return (static_cast<int64_t>(z) * d.y + y) * d.x + x;
 }

@@ -31,10 +31,6 @@ constexpr int kMaxMips = 16;
 // ----------------------------------------------------------------- mips -----
 
 NGT_HOST_DEVICE_INLINE Dims level_dims(const Dims& d, int m) { return Dims{d.x >> m, d.y >> m, d.z >> m}; }
-NGT_HOST_DEVICE_INLINE int64_t dims_cells(const Dims& d) {
-  return static_cast<int64_t>(d.x) * d.y * d.z;
-}
-
 // A pyramid of n_data grids: level 0 is the caller's buffer (`base`, N
 // slices); levels 1..L follow each other in `levels`, level m holding
 // [N][dims >> m][C].

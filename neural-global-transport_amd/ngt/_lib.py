@@ -19,6 +19,7 @@ _c_i64p = ctypes.POINTER(ctypes.c_int64)
 _c_i32p = ctypes.POINTER(ctypes.c_int32)
 _c_fp = ctypes.POINTER(ctypes.c_float)
 _vp = ctypes.c_void_p
+_vpp = ctypes.POINTER(ctypes.c_void_p)
 _i = ctypes.c_int
 _f = ctypes.c_float
 _sz = ctypes.c_size_t
@@ -70,6 +71,8 @@ _SIGNATURES = {
                                        _c_i32p, _i, _i, _i, _vp, _i, _vp, _vp, _sz, _vp]),
     "ngt_advect_workspace_size": (_sz, [_c_i64p, _i, _i, _i, _i]),
     "ngt_advect_fwd": (_i, [_vp, _c_i64p, _vp, _vp, _vp, _i, _f, _i, _i, _i, _i, _vp, _vp, _vp, _sz, _vp]),
+    "ngt_mac_component_luts": (_i, [_vpp, _c_i64p, _f, _i, _vpp, _vp]),
+    "ngt_mac_component_luts_bwd": (_i, [_vpp, _c_i64p, _f, _i, _vpp, _vp]),
     "ngt_advect_bwd": (_i, [_vp, _c_i64p, _vp, _vp, _vp, _i, _f, _i, _i, _i, _i, _vp, _vp, _i, _vp, _vp, _vp, _vp,
                             _vp, _sz, _vp]),
 }
@@ -206,6 +209,10 @@ def empty_grad(t):
 
 def ptr(t):
     return ctypes.c_void_p(t.data_ptr()) if t is not None else None
+
+
+def ptr3(tensors):
+    return (ctypes.c_void_p * 3)(*(t.data_ptr() for t in tensors))
 
 
 def stream(device):

@@ -433,14 +433,35 @@ class VelocityGrid:
     def warped(self, vel_grid=None, order=1, dt=1.0, clamp="NONE"):
         """Self-advect the three MAC components (vel_grid None) or advect them
         with another velocity grid of the same centered shape."""
+        source = self if vel_grid is None else vel_grid
+        luts = source._fused_component_luts(-dt) if source.centered_shape == self.centered_shape else None
         res = []
-        for comp, data in (("X", self.x), ("Y", self.y), ("Z", self.z)):
-            if vel_grid is None:
+        for i, (comp, data) in enumerate((("X", self.x), ("Y", self.y), ("Z", self.z))):
+            if luts is not None:
+                lut = luts[i]
+            elif vel_grid is None:
                 lut = self._sampled_to_component_shape(comp) * (-dt)
             else:
                 lut = vel_grid._sampled_to_component_shape_of(self, comp) * (-dt)
             res.append(self._warp_vel_component(data, lut, order=order, dt=dt, clamp=clamp))
         return tuple(res)
+
+    def _fused_component_luts(self, scale):
+        """``_sampled_to_component_shape(c) * scale`` of the three components
+        in one launch, or None where the composed reads are needed: another
+        filter, mips, WRAP (its reads reach the other end of the grid), the
+        reference's count-normalised gradients, a scale that is a tensor, or
+        components of other shapes or places than the kernel's."""
+        r = self.warp_renderer
+        comps = (self.x, self.y, self.z)
+        if (not self._can_fuse() or r.boundary_mode not in ("BORDER", "CLAMP") or ops.gradient_semantics != "exact"
+                or type(scale) not in (int, float)):
+            return None
+        n = self.x.shape[0]
+        for c, s in zip(comps, (self.x_shape, self.y_shape, self.z_shape)):
+            if list(c.shape) != [n] + s + [1] or c.dtype != torch.float32 or c.device != self.x.device or not c.is_cuda:
+                return None
+        return ops.mac_component_luts(*comps, scale=scale, boundary=r.boundary_mode)
 
     def _sampled_to_component_shape_of(self, other, comp):
         if other.centered_shape != self.centered_shape:

@@ -21,6 +21,7 @@ Matrices and frustum parameters are host arrays (numpy, lists or CPU
 tensors), exactly what the reference ops received.
 """
 import contextlib
+import ctypes
 
 import torch
 
@@ -707,6 +708,44 @@ def advect_grid_semi_langrange(input, velocity_centered, timestep=1.0, order=1, 
         vx, vy, vz = velocity_centered, None, None
     return _Advect.apply(input, float(timestep), int(order), _enum(CLAMP, clamp, "clamp"),
                          _enum(BOUNDARY, boundary, "boundary"), bool(separate_velocity_batch), vx, vy, vz)
+
+
+# --- tables of a MAC velocity's self-advection ----------------------------------------
+
+class _MacComponentLuts(torch.autograd.Function):
+    @staticmethod
+    def forward(ctx, x, y, z, shape, scale, boundary):
+        lib = _lib.load()
+        comps = [_lib.device_tensor(c, "input") for c in (x, y, z)]
+        luts = tuple(torch.empty(tuple(c.shape[:4]) + (3,), dtype=torch.float32, device=c.device) for c in comps)
+        _lib.check(lib.ngt_mac_component_luts(_lib.ptr3(comps), (ctypes.c_int64 * 5)(*shape), scale, boundary,
+                                              _lib.ptr3(luts), _lib.stream(x.device)))
+        ctx.args = (shape, scale, boundary)
+        return luts
+
+    @staticmethod
+    def backward(ctx, gx, gy, gz):
+        lib = _lib.load()
+        shape, scale, boundary = ctx.args
+        lut_grads = [_lib.device_tensor(g, "output_grad") for g in (gx, gy, gz)]
+        grads = tuple(torch.empty(tuple(g.shape[:4]) + (1,), dtype=torch.float32, device=g.device) for g in lut_grads)
+        _lib.check(lib.ngt_mac_component_luts_bwd(_lib.ptr3(lut_grads), (ctypes.c_int64 * 5)(*shape), scale, boundary,
+                                                  _lib.ptr3(grads), _lib.stream(gx.device)))
+        return grads + (None, None, None)
+
+
+def mac_component_luts(x, y, z, scale=1.0, boundary="BORDER"):
+    """The MAC components [N,D,H,W+1,1], [N,D,H+1,W,1], [N,D+1,H,W,1] read at
+    the faces of each of them (LINEAR, boundary BORDER or CLAMP) and multiplied
+    by ``scale``: three [..., 3] fields (x, y, z) of the components' shapes, the
+    relative tables of a velocity's self-advection
+    (data_structures.py:1081-1164).  The gradient is the exact adjoint."""
+    n, d, h, w = x.shape[0], x.shape[1], x.shape[2], x.shape[3] - 1
+    want = ((n, d, h, w + 1, 1), (n, d, h + 1, w, 1), (n, d + 1, h, w, 1))
+    if tuple(tuple(c.shape) for c in (x, y, z)) != want:
+        raise ValueError("shapes of components do not fit. x: %s, y: %s, z: %s"
+                         % (list(x.shape), list(y.shape), list(z.shape)))
+    return _MacComponentLuts.apply(x, y, z, (n, d, h, w, 1), float(scale), _enum(BOUNDARY, boundary, "boundary"))
 
 
 # --- namespaces mirroring ops_loader ------------------------------------------------
