@@ -525,31 +525,28 @@ class _RenderDensityL2(torch.autograd.Function):
         out = torch.empty(img_shape + (4,), dtype=torch.float32, device=density.device)
         loss = torch.empty((), dtype=torch.float32, device=density.device)
         lp, _, keep = _lib.host_floats(light_rgb, 3)
-        s_d = _lib.shape5(density)
+        s_d, od, st = _lib.shape5(density), _lib.dhw(out_shape), _lib.stream(density.device)
         # one haloed brick copy of the density serves the forward and the backward
         bricked = None
         if interp == INTERPOLATION["LINEAR"] and use_bricked_layout:
             nb = lib.ngt_bricked_grid_bytes(s_d)
             if nb > 0:
                 bricked, _ = _lib.workspace(nb, density.device)
-                _lib.check(lib.ngt_bricked_grid(_lib.ptr(density), s_d, boundary, _lib.ptr(bricked),
-                                                _lib.stream(density.device)))
-        ws, nbytes = _lib.workspace(lib.ngt_render_density_l2_fwd_workspace_size(s_d, interp, cams.nv,
-                                                                                 _lib.dhw(out_shape)), density.device)
+                _lib.check(lib.ngt_bricked_grid(_lib.ptr(density), s_d, boundary, _lib.ptr(bricked), st))
+        ws, nbytes = _lib.workspace(lib.ngt_render_density_l2_fwd_workspace_size(s_d, interp, cams.nv, od),
+                                    density.device)
         # with a gradient to come, the forward also records the gather adjoint's
         # rays and per-sample gradients (LINEAR, BORDER)
         record, rbytes = None, 0
         if (ctx.needs_input_grad[0] and use_gather_adjoint and bricked is not None
                 and boundary == BOUNDARY["BORDER"]):
-            rb = lib.ngt_render_density_l2_record_size(s_d, cams.m, cams.v, cams.p, cams.f, cams.nv,
-                                                       _lib.dhw(out_shape))
+            rb = lib.ngt_render_density_l2_record_size(s_d, cams.m, cams.v, cams.p, cams.f, cams.nv, od)
             if rb > 0:
                 record, rbytes = _lib.workspace(rb, density.device)
         _lib.check(lib.ngt_render_density_l2_fwd(
             _lib.ptr(density), s_d, lp, float(depth_step), cams.m, cams.v, cams.p, cams.f, cams.nv,
-            _lib.dhw(out_shape), interp, boundary, mode, _lib.ptr(target), float(weight),
-            None if bricked is None else _lib.ptr(bricked), None if record is None else _lib.ptr(record), rbytes,
-            _lib.ptr(out), _lib.ptr(loss), _lib.ptr(ws), nbytes, _lib.stream(density.device)))
+            od, interp, boundary, mode, _lib.ptr(target), float(weight), _lib.ptr(bricked), _lib.ptr(record), rbytes,
+            _lib.ptr(out), _lib.ptr(loss), _lib.ptr(ws), nbytes, st))
         # the brick copy and the recorded gradients are saved like the inputs,
         # so that a checkpointed caller drops them with everything else and
         # the recomputed forward makes them again
@@ -584,7 +581,7 @@ class _RenderDensityL2(torch.autograd.Function):
         _lib.check(lib.ngt_render_density_l2_bwd(
             _lib.ptr(density), s_d, lp, float(depth_step), _lib.ptr(out), _lib.ptr(target), float(weight),
             _lib.ptr(gl), cams.m, cams.v, cams.p, cams.f, cams.nv, _lib.dhw(out_shape), interp, boundary, mode,
-            None if bricked is None else _lib.ptr(bricked), 0 if record is None else 1, _lib.ptr(g), _lib.ptr(ws),
+            _lib.ptr(bricked), 0 if record is None else 1, _lib.ptr(g), _lib.ptr(ws),
             nbytes, _lib.stream(density.device)))
         return g, None, None, None, None, None, None, None, None, None
 
@@ -619,12 +616,12 @@ def _adv_layout(velocity):
 def _check_vel_shape(inp, vx, vy, vz, order):
     D, H, W = inp.shape[1:4]
     if vy is None:
-        if tuple(vx.shape[1:4]) != (D, H, W):
+        if vx.shape[1:4] != (D, H, W):
             raise ValueError("Shape mismatch in centered warp: data %s, velocity %s"
                              % (list(inp.shape[1:4]), list(vx.shape[1:4])))
     else:
-        if (tuple(vx.shape[1:4]) != (D, H, W + 1) or tuple(vy.shape[1:4]) != (D, H + 1, W)
-                or tuple(vz.shape[1:4]) != (D + 1, H, W)):
+        if (vx.shape[1:4] != (D, H, W + 1) or vy.shape[1:4] != (D, H + 1, W)
+                or vz.shape[1:4] != (D + 1, H, W)):
             raise ValueError("shapes of components do not fit. x: %s, y: %s, z: %s"
                              % (list(vx.shape), list(vy.shape), list(vz.shape)))
 

@@ -42,7 +42,7 @@ class _NullProfiler:
 
 
 def _mat_list(mats):
-    return np.stack([np.asarray(m, dtype=np.float32).reshape(16) for m in mats])
+    return np.array(mats, dtype=np.float32).reshape(-1, 16)
 
 
 class Renderer(object):
