@@ -74,7 +74,8 @@ def test_matches_scatter_and_oracle(ngt_ops, monkeypatch, dims, out_dhw, C, view
 
 
 def test_thresholds_of_a_one_cell_grid():
-    """q < border_end(n) is q + 0.5f < n in float, at the last floats below."""
+    """q < the largest valid position (n - 0.5; for one cell the float below 0.5)
+    is q + 0.5f < n in float, at the last floats below."""
     for n in (1, 2, 3, 4, 7, 8, 127, 128, 129, 4096):
         end = np.float32(0.5) - np.float32(2.0) ** -25 if n == 1 else np.float32(n) - np.float32(0.5)
         q = np.float32(n) - np.float32(0.5)
