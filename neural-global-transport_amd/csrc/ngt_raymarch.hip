@@ -782,7 +782,7 @@ NGT_DEVICE void wave_lds_sync() {
   __builtin_amdgcn_wave_barrier();
 }
 
-// Pass 2: one work-group per brick of BX x BY x BZ voxels.  For every view it
+// Pass 2: one work-group of NT work-items per brick of BX x BY x BZ voxels.  For every view it
 // projects the brick's sample-support box (positions whose trilinear corners
 // can fall in the brick: p in [b0 - 0.5, b1 + 1.5)) to a pixel rectangle,
 // walks the rays of those pixels over the k interval inside the box, and adds
@@ -802,7 +802,7 @@ NGT_DEVICE void wave_lds_sync() {
 // exact and independent of the order of the atomics (the gradient is
 // reproducible bit for bit).  A non-finite bound makes the brick's gradient
 // NaN.
-template <int CG, int BX, int BY, int BZ>
+template <int CG, int BX, int BY, int BZ, int NT = 256>
 NGT_DEVICE void raymarch_bwd_brick_kernel_body(const VBlock& vb, const RayArgs& a, const CamBatch& cb, int pair_base,
                                                                  const RayRec* __restrict__ rays,
                                                                  const float* __restrict__ bound,
@@ -816,7 +816,7 @@ NGT_DEVICE void raymarch_bwd_brick_kernel_body(const VBlock& vb, const RayArgs& 
   __shared__ unsigned long long acc[CG][NP];
   __shared__ int rect[kMaxCamsPerLaunch][4];  // x0, y0, nx, ny (nx = 0: view skipped)
   __shared__ int ray_begin[kMaxCamsPerLaunch + 1];
-  __shared__ float s_wmax[4];
+  __shared__ float s_wmax[NT / 64];
   const int tid = threadIdx.x;
   const int bricks_x = (a.din.x + BX - 1) / BX, bricks_y = (a.din.y + BY - 1) / BY;
   const int bricks_z = (a.din.z + BZ - 1) / BZ;
@@ -827,7 +827,7 @@ NGT_DEVICE void raymarch_bwd_brick_kernel_body(const VBlock& vb, const RayArgs& 
   const int b0y = ((brem / bricks_x) % bricks_y) * BY;
   const int b0z = (brem / (bricks_x * bricks_y)) * BZ;
   const int b1x = min(b0x + BX, a.din.x) - 1, b1y = min(b0y + BY, a.din.y) - 1, b1z = min(b0z + BZ, a.din.z) - 1;
-  for (int i = tid; i < CG * NP; i += 256) (&acc[0][0])[i] = 0ull;
+  for (int i = tid; i < CG * NP; i += NT) (&acc[0][0])[i] = 0ull;
 
   // pixel rectangles of the views: wavefront 0 projects the 8 corners of the
   // support box for up to 8 views at once (lane = view * 8 + corner), then
@@ -918,13 +918,13 @@ NGT_DEVICE void raymarch_bwd_brick_kernel_body(const VBlock& vb, const RayArgs& 
            pixel % kGPix * kGQuad;
     rr = rays[pair * static_cast<uint32_t>(npix) + pixel];
   };
-  // Rays are taken 256 at a time, every fourth one by a wavefront: the samples
-  // that its lanes add at one time are then some cells apart (neighbouring rays
+  // Rays are taken NT at a time, every (NT / 64)-th one by a wavefront: the
+  // samples that its lanes add at one time are then some cells apart (neighbouring rays
   // add to the same cells, and equal addresses in one LDS atomic are taken one
   // by one: 340 -> 293 us at 160^3 x 8 views of 480x270, the rays there being
   // closer than cells)
   const int lane = tid & 63, wave = tid >> 6;
-  const int slot = lane * 4 + wave;
+  const int slot = lane * (NT / 64) + wave;
   // each work-item's ray of the next chunk is loaded one chunk ahead, so that
   // its latency overlaps the current chunk's samples (the first one overlaps
   // the gradient bounds' loads)
@@ -940,7 +940,7 @@ NGT_DEVICE void raymarch_bwd_brick_kernel_body(const VBlock& vb, const RayArgs& 
       const int tx0 = rect[ci][0] / kRayTile, tx1 = (rect[ci][0] + rect[ci][2] - 1) / kRayTile;
       const int ty0 = rect[ci][1] / kRayTile, ty1 = (rect[ci][1] + rect[ci][3] - 1) / kRayTile;
       const int ntiles = (tx1 - tx0 + 1) * (ty1 - ty0 + 1);
-      for (int t = tid; t < ntiles; t += 256) {
+      for (int t = tid; t < ntiles; t += NT) {
         const int tx = tx0 + t % (tx1 - tx0 + 1), ty = ty0 + t / (tx1 - tx0 + 1);
         const float bnd = bound[static_cast<int64_t>(pair_base + ci) * per_pair + ty * ntx + tx];
         m = (bnd > m || bnd != bnd) ? bnd : m;  // NaN propagates
@@ -956,7 +956,7 @@ NGT_DEVICE void raymarch_bwd_brick_kernel_body(const VBlock& vb, const RayArgs& 
   __syncthreads();
   float wmax = s_wmax[0];
 #pragma unroll
-  for (int w = 1; w < 4; ++w) wmax = (s_wmax[w] > wmax || s_wmax[w] != s_wmax[w]) ? s_wmax[w] : wmax;
+  for (int w = 1; w < NT / 64; ++w) wmax = (s_wmax[w] > wmax || s_wmax[w] != s_wmax[w]) ? s_wmax[w] : wmax;
   const bool finite = wmax < 3.0e38f;  // false for +inf and NaN
   // |contribution| <= wmax < 2^e  ->  |contribution * 2^S| < 2^30 with S = 30 - e
   const int S = wmax > 0.f && finite ? 30 - ilogbf(wmax) - 1 : 0;
@@ -981,24 +981,24 @@ NGT_DEVICE void raymarch_bwd_brick_kernel_body(const VBlock& vb, const RayArgs& 
   // reference uses ceil = floor at integer positions carries weight exactly 0.)
   // The wavefronts do not wait for each other, so that one's address arithmetic
   // runs beside another's LDS atomics, which bound the kernel about equally.
-  // 128^3 x 5 views of 256x144: 51 -> 46 us, 160^3 x 8 of 480x270: 340 -> 240,
+  // 128^3 x 5 views of 256x144: 51 -> 46 us, 160^3 x 8 of 480x270: 340 -> 254,
   // four channels at 96^3 x 5: 125 -> 101 (a work-group-wide scan and deal, with
   // a barrier before and after each 2048 samples, is what it was measured
-  // against).  6 samples in flight per work-item: 4 take 44.7 / 264 / 102 us,
-  // where 6 take 44.2 / 255 / 100; 9 need more than 128 VGPRs, which halves the
-  // wavefronts (62.5 / 278).
+  // against; bricks chosen by size: 42 and 239).  6 samples in flight per
+  // work-item: 4 take 44.7 / 264 / 102 us, where 6 take 44.2 / 255 / 100; 9 need
+  // more than 128 VGPRs, which halves the wavefronts (62.5 / 278).
   constexpr int kMark = 768, kPer = 6, CS = stored_channels(CG);
-  __shared__ int s_kb[256];           // each ray's first k in the box minus its first item
-  __shared__ int64_t s_gofs[256];     // each ray's sample 0 in G
-  __shared__ float4 s_ps[256];        // each ray's start and step x
-  __shared__ float4 s_pd[256];        // each ray's step y, z and loss-gradient scale, offset
-  __shared__ float s_blue[CS != CG ? 256 : 1];  // each ray's third colour gradient where factors are stored
-  __shared__ unsigned char s_ray[4][kMark];
-  for (int base_r = 0; base_r < total; base_r += 256) {
+  __shared__ int s_kb[NT];           // each ray's first k in the box minus its first item
+  __shared__ int64_t s_gofs[NT];     // each ray's sample 0 in G
+  __shared__ float4 s_ps[NT];        // each ray's start and step x
+  __shared__ float4 s_pd[NT];        // each ray's step y, z and loss-gradient scale, offset
+  __shared__ float s_blue[CS != CG ? NT : 1];  // each ray's third colour gradient where factors are stored
+  __shared__ unsigned char s_ray[NT / 64][kMark];
+  for (int base_r = 0; base_r < total; base_r += NT) {
     const int r = base_r + slot;
     const RayRec rr = next_rr;
     const int64_t gofs = r < total ? next_gofs : 0;
-    if (r + 256 < total) fetch_ray(r + 256, next_rr, next_gofs);
+    if (r + NT < total) fetch_ray(r + NT, next_rr, next_gofs);
     int cnt = 0, k0 = 0;
     if (r < total) {
       s_ps[tid] = make_float4(rr.sx, rr.sy, rr.sz, rr.dx);
@@ -1043,7 +1043,7 @@ NGT_DEVICE void raymarch_bwd_brick_kernel_body(const VBlock& vb, const RayArgs& 
         const int r0 = max(incl - cnt, m0), r1 = min(incl, m_end);
 #pragma clang loop unroll(disable)
         for (int i = r0; i < r1; ++i) {
-          s_ray[wave][i - m0] = static_cast<unsigned char>(tid);
+          s_ray[wave][i - m0] = static_cast<unsigned char>(lane);
           asm volatile("");  // a few bytes: no fill routine
         }
       }
@@ -1061,7 +1061,7 @@ NGT_DEVICE void raymarch_bwd_brick_kernel_body(const VBlock& vb, const RayArgs& 
           const int i = i0 + lane + u * 64;
           oks[u] = false;
           if (i < m_end) {
-            const int lo_j = s_ray[wave][i - m0];
+            const int lo_j = wave * 64 + s_ray[wave][i - m0];
             const int k = s_kb[lo_j] + i;
             const float4 ps = s_ps[lo_j];
             const float4 pd = s_pd[lo_j];
@@ -1115,13 +1115,13 @@ NGT_DEVICE void raymarch_bwd_brick_kernel_body(const VBlock& vb, const RayArgs& 
   // the brick's own voxels, kOwn per work-item: every value is formed first,
   // then all are stored together (a store loop that read-added per voxel
   // behind a select waited for each voxel's load in turn: 11 us at 128^3)
-  constexpr int kOwn = (NV + 255) / 256;
+  constexpr int kOwn = (NV + NT - 1) / NT;
   float vals[kOwn][CG];
   int64_t offs[kOwn];
   bool own[kOwn];
 #pragma unroll
   for (int m = 0; m < kOwn; ++m) {
-    const int i = tid + 256 * m;
+    const int i = tid + NT * m;
     const int lx = i % BX, ly = (i / BX) % BY, lz = i / (BX * BY);
     const int x = b0x + lx, y = b0y + ly, z = b0z + lz;
     own[m] = i < NV && x <= b1x && y <= b1y && z <= b1z;
@@ -1150,14 +1150,14 @@ NGT_DEVICE void raymarch_bwd_brick_kernel_body(const VBlock& vb, const RayArgs& 
   }
 }
 
-template <int CG, int BX, int BY, int BZ>
-__global__ __launch_bounds__(256) void raymarch_bwd_brick_kernel(RayArgs a, CamBatch cb, int pair_base,
+template <int CG, int BX, int BY, int BZ, int NT = 256>
+__global__ __launch_bounds__(NT) void raymarch_bwd_brick_kernel(RayArgs a, CamBatch cb, int pair_base,
                                                                  const RayRec* __restrict__ rays,
                                                                  const float* __restrict__ bound,
                                                                  const float* __restrict__ G, int kcap,
                                                                  float* __restrict__ in_grad, int accumulate,
                                                                  const float* __restrict__ grad_scale) {
-  raymarch_bwd_brick_kernel_body<CG, BX, BY, BZ>(VBlock{static_cast<int>(blockIdx.x), static_cast<int>(blockIdx.y), static_cast<int>(blockIdx.z)}, a, cb, pair_base, rays, bound, G, kcap, in_grad, accumulate, grad_scale);
+  raymarch_bwd_brick_kernel_body<CG, BX, BY, BZ, NT>(VBlock{static_cast<int>(blockIdx.x), static_cast<int>(blockIdx.y), static_cast<int>(blockIdx.z)}, a, cb, pair_base, rays, bound, G, kcap, in_grad, accumulate, grad_scale);
 }
 
 // Reference gradient of one camera: reverse walk from `end` with the
@@ -1542,26 +1542,32 @@ void run_gather(const std::vector<Pair>& pairs, const float* M, const float* V, 
                              base, output, output_grad, gp.G, gp.rays, gp.bound, gp.kcap)));
     }
     // bricks: larger ones visit fewer samples twice (the support box is one
-    // cell wider than the brick), smaller ones leave room for more work-groups
-    // beside their 64-bit accumulators.  One channel, 128^3 x 5 views / 160^3 x 8:
-    // 16 x 16 x 8 takes 49 / 285 us, 16 x 8 x 8 58 / 306, 8 x 8 x 8 71 / 350,
-    // 16 x 16 x 16 56 / 358; four channels at 96^3 x 5: 8 x 8 x 8 105 us,
-    // 16 x 8 x 8 113.
-    constexpr int BX = 8, BY = 8, BZ = 8;
-    constexpr int BX1 = 16, BY1 = 16, BZ1 = 8;
+    // cell wider than the brick), smaller ones give more work-groups.  One
+    // channel, bricks of 16^3 (512 work-items) / 16 x 8 x 8 / 8^3 (256), edge of
+    // the grid x views of the image:  160 x 8 of 480x270: 239 / 281 / - us;
+    // 128 x 5 of 256x144: 42 / 58 / 71;  112 x 3 of 256x144: 33 / 36 / 41;  96 x
+    // 5 of 256x144: 45 / 42 / 48;  96 x 8 of 480x270: 205 / 185 / 188;  80 x 4 of
+    // 150x100: 23 / 19 / 18;  64 x 5 of 256x144: 84 / 52 / 37;  24 x 3 of 128x72:
+    // 81 / 50 / 32.  So 16^3 from 320 bricks on (112^3 has 343, 96^3 216), then 16
+    // x 8 x 8 from 768 on (96^3 has 864, 80^3 500).  (16 x 16 x 8 with 256
+    // work-items: 254 / 47 / 33 / 51 / 226 / 25 / 84 / 83.)  Four channels at 96 x
+    // 5: 8^3 105 us, 16 x 8 x 8 113.
     const int accumulate = b > 0 ? 1 : 0;
     const int CG = LIGHT ? 1 : C;
-    if (CG == 1) {
-      const unsigned bricks = blocks_for(a.din.x, BX1) * blocks_for(a.din.y, BY1) * blocks_for(a.din.z, BZ1);
-      hipLaunchKernelGGL((raymarch_bwd_brick_kernel<1, BX1, BY1, BZ1>), dim3(bricks * n_data), dim3(256), 0, s, a,
-                         cb, base, gp.rays, gp.bound, gp.G, gp.kcap, in_grad, accumulate,
-                         recorded ? grad_scale : nullptr);
+    const auto bricks = [&](int bx, int by, int bz) {
+      return static_cast<unsigned>(blocks_for(a.din.x, bx) * blocks_for(a.din.y, by) * blocks_for(a.din.z, bz) * n_data);
+    };
+    const float* const scale = recorded ? grad_scale : nullptr;
+    if (CG == 1 && bricks(16, 16, 16) >= 320) {
+      hipLaunchKernelGGL((raymarch_bwd_brick_kernel<1, 16, 16, 16, 512>), dim3(bricks(16, 16, 16)), dim3(512), 0, s, a, cb,
+                         base, gp.rays, gp.bound, gp.G, gp.kcap, in_grad, accumulate, scale);
+    } else if (CG == 1 && bricks(16, 8, 8) >= 768) {
+      hipLaunchKernelGGL((raymarch_bwd_brick_kernel<1, 16, 8, 8>), dim3(bricks(16, 8, 8)), dim3(256), 0, s, a, cb, base,
+                         gp.rays, gp.bound, gp.G, gp.kcap, in_grad, accumulate, scale);
     } else {
-      const unsigned bricks = blocks_for(a.din.x, BX) * blocks_for(a.din.y, BY) * blocks_for(a.din.z, BZ);
       NGT_SWITCH_C(CG,
-          hipLaunchKernelGGL((raymarch_bwd_brick_kernel<CC, BX, BY, BZ>), dim3(bricks * n_data), dim3(256), 0, s, a,
-                             cb, base, gp.rays, gp.bound, gp.G, gp.kcap, in_grad, accumulate,
-                             recorded ? grad_scale : nullptr));
+          hipLaunchKernelGGL((raymarch_bwd_brick_kernel<CC, 8, 8, 8>), dim3(bricks(8, 8, 8)), dim3(256), 0, s, a, cb, base,
+                             gp.rays, gp.bound, gp.G, gp.kcap, in_grad, accumulate, scale));
     }
   }
 }

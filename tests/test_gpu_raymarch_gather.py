@@ -73,6 +73,21 @@ def test_matches_scatter_and_oracle(ngt_ops, monkeypatch, dims, out_dhw, C, view
         assert rel(got, eg) < 1e-4
 
 
+@pytest.mark.parametrize("dims,C", [((9, 100, 121), 1), ((72, 100, 100), 1), ((101, 113, 120), 1), ((101, 113, 120), 2)])
+def test_brick_shapes_match_scatter(ngt_ops, monkeypatch, dims, C):
+    """Grids that take bricks of 8^3, 16 x 8 x 8 and 16^3 cells, off their extents."""
+    out_dhw = (48, 21, 30)
+    rng = np.random.default_rng(8100 + sum(dims))
+    Ms, Vs, Ps, Fs = cameras(dims, out_dhw, 3, 30.0)
+    x = dev(rng.uniform(0.0, 0.5, (1,) + dims + (C,)))
+    out = ngt_ops.raymarch_grid_transform(x, Ms, Vs, Ps, Fs, out_dhw)
+    g = dev(rng.standard_normal(tuple(out.shape)))
+    got = ngt_ops.raymarch_grid_transform_grad(x, out, g, Ms, Vs, Ps, Fs, out_dhw)
+    monkeypatch.setattr(ngt_ops, "use_gather_adjoint", False)
+    scatter = ngt_ops.raymarch_grid_transform_grad(x, out, g, Ms, Vs, Ps, Fs, out_dhw)
+    assert rel(got, scatter.cpu().double().numpy()) < 1e-4
+
+
 def test_thresholds_of_a_one_cell_grid():
     """q < the largest valid position (n - 0.5; for one cell the float below 0.5)
     is q + 0.5f < n in float, at the last floats below."""
