@@ -660,7 +660,7 @@ def main():
     #   render + L2 bwd 8 B/voxel + 28 B/pixel (image and RGB target in)
     algo = {"advect_fwd": cells * 20, "advect_bwd": cells * 36, "render_fwd": cells * 4 + pixels * 28,
             "render_bwd": cells * 8 + pixels * 28}
-    # the roofline names the step's dominant kernel (rocprofv3 kernel-trace
+    # the roofline names the largest kernel that a call launches alone (kernel-trace
     # summary of this workload): the render adjoint's brick gather,
     # raymarch_bwd_brick_kernel, which the render + L2 backward launches alone,
     # so that call's HIP-event duration is the kernel's
