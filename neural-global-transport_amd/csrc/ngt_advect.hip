@@ -546,11 +546,11 @@ NGT_DEVICE void scatter_linear_tile(double* tile, int planes, int ox, int oy, in
   if constexpr (BM == BORDER) {
     // the common case, floor and floor + 1 of every axis in the tile, at fixed
     // offsets from one address (where ceil is floor, at an integer position,
-    // the upper weight is 0; a corner outside the grid has a tile slot of its
-    // own, which no cell reads)
+    // the upper weight is 0, and adds 0 as long as the value is finite; a corner
+    // outside the grid has a tile slot of its own, which no cell reads)
     if (static_cast<unsigned>(lx0) < static_cast<unsigned>(kTileX - 1) &&
         static_cast<unsigned>(ly0) < static_cast<unsigned>(kTileY - 1) &&
-        static_cast<unsigned>(lz0) < static_cast<unsigned>(planes - 1)) {
+        static_cast<unsigned>(lz0) < static_cast<unsigned>(planes - 1) && __builtin_isfinite(val)) {
       double* t = tile + (lz0 * kTileY + ly0) * kTileX + lx0;
 #pragma unroll
       for (int k = 0; k < 8; ++k) {
