@@ -798,6 +798,22 @@ NGT_HOST_DEVICE_INLINE BrickList level_bricks(const Dims& d, int m) {
   return BrickList{(dm.x + b.x - 1) / b.x, (dm.y + b.y - 1) / b.y, (dm.z + b.z - 1) / b.z};
 }
 
+// Work-groups that share the candidates of a brick of level m, which is split
+// from level `first` on: its voxels have 8^m times the finest ones' candidates
+// to try, and the coarse levels have few bricks.  Split levels are cleared
+// first and take the shares' sums by atomics.  96^3 into three 128x72x96
+// frustums, 1 channel, 3 / 4 / 6 levels: 228 / 274 / 306 us, unsplit 1582 / 6446
+// / 11462 (the coarsest level's one brick tries every output cell).
+NGT_HOST_DEVICE_INLINE int level_splits(int m, int first) {
+  return m < first ? 1 : (m < 4 ? 1 << (3 * m - 4) : 256);
+}
+
+// Level 2 is split too where its bricks are few, or little of the time is the
+// finer levels': the same frustums with 2 levels, 1 channel: 183 us, split from
+// level 3 on 274; 4 channels (216 bricks) 304 against 276; 64^3 into 64^3 cells
+// x 3, 4 channels (64 bricks): 99 against 157.
+inline int first_split_level(int64_t c, int64_t bricks2) { return c < 4 || bricks2 < 128 ? 2 : 3; }
+
 // i / n and i % n for 0 <= i < 2^30, n > 0, from a float estimate that is off
 // by at most a few hundred (by one for i below 2^22).
 NGT_DEVICE int div_rem(int i, int n, float inv, int& rem) {
@@ -810,7 +826,8 @@ NGT_DEVICE int div_rem(int i, int n, float inv, int& rem) {
 
 template <int C, int MM, int BX, int BY, int BZ>
 __global__ __launch_bounds__(256) void xform_bwd_gather_kernel(XformArgs a, CamBatch cb, MipSet grad,
-                                                               const float* __restrict__ out_grad, int accumulate) {
+                                                               const float* __restrict__ out_grad, int accumulate,
+                                                               int first_split) {
   static_assert(BX >= 8 && BY >= 4 && BZ >= 4, "the coarser levels' bricks fit the finest one's accumulator");
   // one plane per channel: consecutive cells on consecutive banks
   constexpr int NP = (BX + 2) * (BY + 2) * (BZ + 2);
@@ -820,10 +837,12 @@ __global__ __launch_bounds__(256) void xform_bwd_gather_kernel(XformArgs a, CamB
   // the coarsest level's bricks, which see the most samples, come first
   int bid = blockIdx.x, m = grad.num_levels;
   BrickList bl = level_bricks<BX, BY, BZ>(grad.d0, m);
-  while (m > 0 && bid >= bl.count() * grad.n_data) {
-    bid -= bl.count() * grad.n_data;
+  while (m > 0 && bid >= bl.count() * level_splits(m, first_split) * grad.n_data) {
+    bid -= bl.count() * level_splits(m, first_split) * grad.n_data;
     bl = level_bricks<BX, BY, BZ>(grad.d0, --m);
   }
+  const int splits = level_splits(m, first_split), split = bid % splits;
+  bid /= splits;
   const int n = bid / bl.count(), brem = bid % bl.count();
   Dims dm;
   float* const out = level_ptr<C>(grad, n, m, dm);
@@ -896,7 +915,7 @@ __global__ __launch_bounds__(256) void xform_bwd_gather_kernel(XformArgs a, CamB
     const CamParams& cp = cb.cam[ci];
     const float* const g = out_grad + static_cast<int64_t>(cp.out_index) * out_cells * C;
     const float inv_nx = 1.f / static_cast<float>(nx), inv_ny = 1.f / static_cast<float>(ny);
-    for (int i = tid; i < total; i += 256) {
+    for (int i = split * 256 + tid; i < total; i += splits * 256) {
       int x, y;
       const int row = div_rem(i, nx, inv_nx, x);
       const int z = box[ci][2] + div_rem(row, ny, inv_ny, y);
@@ -939,7 +958,7 @@ __global__ __launch_bounds__(256) void xform_bwd_gather_kernel(XformArgs a, CamB
       }
     }
   }
-  if (accumulate && !any) return;  // uniform
+  if ((accumulate || splits > 1) && !any) return;  // uniform
   __syncthreads();
   for (int i = tid; i < lb.x * lb.y * lb.z; i += 256) {
     const int lx = i % lb.x, ly = i / lb.x % lb.y, lz = i / (lb.x * lb.y);  // powers of two, uniform
@@ -950,6 +969,12 @@ __global__ __launch_bounds__(256) void xform_bwd_gather_kernel(XformArgs a, CamB
     Vec<C> v;
 #pragma unroll
     for (int j = 0; j < C; ++j) v.v[j] = static_cast<float>(t[j * NP]);
+    if (splits > 1) {
+#pragma unroll
+      for (int j = 0; j < C; ++j)
+        if (v.v[j] != 0.f) atomic_add(o + j, v.v[j]);
+      continue;
+    }
     if (accumulate) {
       const Vec<C> old = vload<C>(o);
 #pragma unroll
@@ -1193,27 +1218,42 @@ bool maps_agree(const CamParams& cp, const Dims& dout, int coord_mode) {
   return true;
 }
 
+// Whether the sample support of every level's grid lies before the camera, so
+// that each brick's projection is bounded by its corners'.
+bool grid_in_front(const CamParams& cp, const Dims& din, const Dims& dout, int levels) {
+  const double reach = 0.502 * static_cast<double>(int64_t(1) << levels);
+  for (int c = 0; c < 8; ++c) {
+    double o[3];
+    if (!(output_index<double>(cp, dout, false, (c & 1) ? din.x + reach : -reach, (c & 2) ? din.y + reach : -reach,
+                               (c & 4) ? din.z + reach : -reach, o) > 0.0))
+      return false;
+  }
+  return true;
+}
+
 // The gather serves LINEAR, BORDER and the forward modes, for cameras whose
-// maps agree; other calls scatter.
+// maps agree and that stand before the grid (a brick that the camera's plane
+// cuts would try every output cell in one work-group); other calls scatter.
 bool use_xform_gather(const std::vector<Pair>& pairs, const float* M, const float* V, const float* P, const float* F,
-                      const XformArgs& a, int64_t n_data, int interpolation, int boundary) {
+                      const XformArgs& a, int64_t n_data, int levels, int interpolation, int boundary) {
   if (interpolation != LINEAR || boundary != BORDER) return false;
   if (a.coord_mode != NGT_COORD_TRANSFORM && a.coord_mode != NGT_COORD_TRANSFORM_LINDEPTH) return false;
   if (dims_cells(a.dout) >= (int64_t(1) << 30) || dims_cells(a.din) * n_data >= (int64_t(1) << 36)) return false;
-  for (const Pair& p : pairs)
-    if (!maps_agree(make_cam(M + 16 * p.n, V + 16 * p.v, P + 16 * p.v, F + 6 * p.v, p.n, p.out), a.dout, a.coord_mode))
-      return false;
+  for (const Pair& p : pairs) {
+    const CamParams cp = make_cam(M + 16 * p.n, V + 16 * p.v, P + 16 * p.v, F + 6 * p.v, p.n, p.out);
+    if (!maps_agree(cp, a.dout, a.coord_mode) || !grid_in_front(cp, a.din, a.dout, levels)) return false;
+  }
   return true;
 }
 
 template <int C, int MM, int BX, int BY, int BZ>
 void launch_xform_gather(const XformArgs& a, const CamBatch& cb, const MipSet& grad, const float* out_grad,
-                         int accumulate, hipStream_t s) {
+                         int accumulate, int first_split, hipStream_t s) {
   int64_t bricks = 0;
   for (int m = 0; m <= grad.num_levels; ++m)
-    bricks += static_cast<int64_t>(level_bricks<BX, BY, BZ>(grad.d0, m).count()) * grad.n_data;
+    bricks += static_cast<int64_t>(level_bricks<BX, BY, BZ>(grad.d0, m).count()) * level_splits(m, first_split) * grad.n_data;
   hipLaunchKernelGGL((xform_bwd_gather_kernel<C, MM, BX, BY, BZ>), dim3(static_cast<unsigned>(bricks)), dim3(256), 0, s,
-                     a, cb, grad, out_grad, accumulate);
+                     a, cb, grad, out_grad, accumulate, first_split);
 }
 
 }  // namespace
@@ -1408,7 +1448,13 @@ int ngt_sample_grid_transform_bwd(const float* input, const int64_t* input_shape
   const bool mip = mipmapping != NGT_MIP_NONE;
   const MipSet grad = make_mips(input_grad, input_shape, mip ? workspace : nullptr, mip ? num_mipmaps : 0);
   hipStream_t s = as_stream(stream);
-  if (!ref && use_xform_gather(pairs, matrix_m, matrix_v, matrix_p, frustum, a, si.n, interpolation, boundary)) {
+  if (!ref && use_xform_gather(pairs, matrix_m, matrix_v, matrix_p, frustum, a, si.n, grad.num_levels, interpolation,
+                               boundary)) {
+    const int first_split = first_split_level(si.c, level_bricks<8, 8, 8>(grad.d0, 2).count() * si.n);
+    if (grad.num_levels >= first_split) {
+      const int64_t stored = mip_floats(si.dims(), si.n, si.c, first_split - 1);
+      fill_zero(grad.levels + stored, mip_floats(si.dims(), si.n, si.c, grad.num_levels) - stored, s);
+    }
     for (size_t b = 0; b < pairs.size(); b += kMaxCamsPerLaunch) {
       const CamBatch cb = cam_batch(pairs, b, matrix_m, matrix_v, matrix_p, frustum);
       // 8x8x8 bricks visit fewer samples twice and pay fewer prologues than
@@ -1418,8 +1464,8 @@ int ngt_sample_grid_transform_bwd(const float* input, const int64_t* input_shape
       // few and too uneven (22.2 and 160 us)
       const bool large = level_bricks<8, 8, 8>(grad.d0, 0).count() * si.n >= 512;
       NGT_SWITCH_C(si.c, NGT_SWITCH_MM(mipmapping,
-          if (large) launch_xform_gather<CC, MMM, 8, 8, 8>(a, cb, grad, output_grad, b > 0, s);
-          else launch_xform_gather<CC, MMM, 8, 4, 4>(a, cb, grad, output_grad, b > 0, s)));
+          if (large) launch_xform_gather<CC, MMM, 8, 8, 8>(a, cb, grad, output_grad, b > 0, first_split, s);
+          else launch_xform_gather<CC, MMM, 8, 4, 4>(a, cb, grad, output_grad, b > 0, first_split, s)));
     }
     if (mip) NGT_SWITCH_C(si.c, launch_mip_collapse<CC>(grad, s));
     return check_launch("ngt_sample_grid_transform_bwd");
