@@ -18,6 +18,7 @@
 // order z, y, x: resample_grid.cu.cc:58-84).  The exact adjoint scatters into
 // per-level gradient buffers and collapses them coarse to fine, each fine
 // cell adding 1/8 of its parent (no atomics in the collapse).
+#include <algorithm>
 #include <cmath>
 
 #include "ngt_host.hpp"
@@ -805,14 +806,25 @@ NGT_HOST_DEVICE_INLINE BrickList level_bricks(const Dims& d, int m) {
 // frustums, 1 channel, 3 / 4 / 6 levels: 228 / 274 / 306 us, unsplit 1582 / 6446
 // / 11462 (the coarsest level's one brick tries every output cell).
 NGT_HOST_DEVICE_INLINE int level_splits(int m, int first) {
-  return m < first ? 1 : (m < 4 ? 1 << (3 * m - 4) : 256);
+  const int above = m - (first < 2 ? first : 2);
+  return m < first ? 1 : (above < 2 ? 4 << (3 * above) : 256);
 }
 
-// Level 2 is split too where its bricks are few, or little of the time is the
-// finer levels': the same frustums with 2 levels, 1 channel: 183 us, split from
-// level 3 on 274; 4 channels (216 bricks) 304 against 276; 64^3 into 64^3 cells
-// x 3, 4 channels (64 bricks): 99 against 157.
-inline int first_split_level(int64_t c, int64_t bricks2) { return c < 4 || bricks2 < 128 ? 2 : 3; }
+// Split from level 2 on where its bricks are few, or little of the time is the
+// finer levels' (the same frustums with 2 levels, 1 channel: 183 us, split from
+// level 3 on 274; 4 channels, 216 bricks, 304 against 276; 64^3 into 64^3 cells x
+// 3, 4 channels, 64 bricks: 99 against 157), from level 1 on where its bricks
+// leave half of the CUs idle (48^3 into 128x72x96 x 3, 1 channel, 1 / 2 / 3 levels:
+// 146 / 200 / 250 us against 425 / 434 / 461; 24^3 into 24^3: 49 / 52 / 52 against
+// 55 / 61 / 64), and from the finest on where that has few bricks and each of
+// its voxels 16 or more cells of a view (16^3 into 64^3 x 3, 1 channel, 0 / 1 / 3
+// levels: 52 / 90 / 100 us against 156 / 365 / 372; 24^3 into 96^3: 61 / 131 / 200
+// against 166 / 472 / 516).
+inline int first_split_level(const Dims& d, const Dims& dout, int64_t n, int64_t c) {
+  const auto bricks = [&](int m) { return level_bricks<8, 4, 4>(d, m).count() * n; };
+  if (bricks(0) < 128 && dims_cells(dout) >= 16 * dims_cells(d)) return 0;
+  return bricks(1) < 128 ? 1 : (c < 4 || bricks(2) < 128 ? 2 : 3);
+}
 
 // i / n and i % n for 0 <= i < 2^30, n > 0, from a float estimate that is off
 // by at most a few hundred (by one for i below 2^22).
@@ -1450,11 +1462,11 @@ int ngt_sample_grid_transform_bwd(const float* input, const int64_t* input_shape
   hipStream_t s = as_stream(stream);
   if (!ref && use_xform_gather(pairs, matrix_m, matrix_v, matrix_p, frustum, a, si.n, grad.num_levels, interpolation,
                                boundary)) {
-    const int first_split = first_split_level(si.c, level_bricks<8, 8, 8>(grad.d0, 2).count() * si.n);
-    if (grad.num_levels >= first_split) {
-      const int64_t stored = mip_floats(si.dims(), si.n, si.c, first_split - 1);
-      fill_zero(grad.levels + stored, mip_floats(si.dims(), si.n, si.c, grad.num_levels) - stored, s);
-    }
+    const int first_split = first_split_level(grad.d0, a.dout, si.n, si.c);
+    const int64_t stored = mip_floats(si.dims(), si.n, si.c, std::max(first_split - 1, 0));
+    const int64_t cleared = mip_floats(si.dims(), si.n, si.c, grad.num_levels) - stored;
+    if (first_split == 0) fill_zero2(input_grad, si.elems(), grad.levels, cleared, s);
+    else if (grad.num_levels >= first_split) fill_zero(grad.levels + stored, cleared, s);
     for (size_t b = 0; b < pairs.size(); b += kMaxCamsPerLaunch) {
       const CamBatch cb = cam_batch(pairs, b, matrix_m, matrix_v, matrix_p, frustum);
       // 8x8x8 bricks visit fewer samples twice and pay fewer prologues than
