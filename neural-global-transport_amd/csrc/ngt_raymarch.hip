@@ -555,6 +555,19 @@ NGT_DEVICE void store_tile_bound(const RayArgs& a, float* __restrict__ bound, in
   }
 }
 
+// A ray's part of its tile's bound: the largest absolute value of its samples'
+// gradients, or NaN if one of them is no finite number.  The differences are
+// summed beside the maximum, which drops a NaN: whatever follows on the ray,
+// the sum keeps it.
+struct GradBound {
+  float largest = 0.f, not_finite = 0.f;
+  NGT_DEVICE void add(float v) {
+    largest = fmaxf(largest, fabsf(v));
+    not_finite += v - v;
+  }
+  NGT_DEVICE float value() const { return largest + not_finite; }
+};
+
 // Image gradient of the fused L2 loss at one pixel (img: the pixel's C
 // channels, tpix: its first target value).
 template <int C>
@@ -605,19 +618,19 @@ NGT_DEVICE float raymarch_bwd_prepass_pixel(const VBlock& vb, const RayArgs& a, 
     float* gp;
     int64_t pixel;
     int kcap;
-    float g_max, bound;
-    // NaN stays NaN in the bound, and an infinite gradient makes it NaN
+    float g_max;
+    GradBound bound;
     NGT_DEVICE void one(int k, float, float, float, const Vec<C>& g, float t, float gd) {
       float* const at = gp + g_offset(k, pixel, kcap) * CS;
       if constexpr (CS != CG) {
         vstore<2>(at, Vec<2>{{t, gd}});
-        const float c = t * g_max;
-        bound = fmaxf(bound, fmaxf(fabsf(c), fabsf(gd))) + (c - c) + (gd - gd);
+        bound.add(t * g_max);
+        bound.add(gd);
       } else {
         const Vec<CG> v = fold_cell_grad<C, LIGHT>(a, cell_grad(g, t, gd));
         vstore<CG>(at, v);
 #pragma unroll
-        for (int i = 0; i < CG; ++i) bound = fmaxf(bound, fabsf(v.v[i])) + (v.v[i] - v.v[i]);
+        for (int i = 0; i < CG; ++i) bound.add(v.v[i]);
       }
     }
     // a round of two samples starts at an even k: its factors are one 16-byte
@@ -630,8 +643,8 @@ NGT_DEVICE float raymarch_bwd_prepass_pixel(const VBlock& vb, const RayArgs& a, 
         vstore<4>(gp + g_offset(k, pixel, kcap) * CS, Vec<4>{{t[0], gd[0], t[1], gd[1]}});
 #pragma unroll
         for (int u = 0; u < kUnroll; ++u) {
-          const float c = k + u < steps ? t[u] * g_max : 0.f, d = k + u < steps ? gd[u] : 0.f;
-          bound = fmaxf(bound, fmaxf(fabsf(c), fabsf(d))) + (c - c) + (d - d);
+          bound.add(k + u < steps ? t[u] * g_max : 0.f);
+          bound.add(k + u < steps ? gd[u] : 0.f);
         }
       } else {
 #pragma unroll
@@ -639,9 +652,9 @@ NGT_DEVICE float raymarch_bwd_prepass_pixel(const VBlock& vb, const RayArgs& a, 
           if (k + u < steps) one(k + u, qx[u], qy[u], qz[u], g, t[u], gd[u]);
       }
     }
-  } sink{a, G + static_cast<int64_t>(pair) * kcap * g_pixels(npix) * CS, pixel, kcap, g_max, 0.f};
+  } sink{a, G + static_cast<int64_t>(pair) * kcap * g_pixels(npix) * CS, pixel, kcap, g_max, {}};
   walk_ray_gradient<C, LINEAR, BM, MODE, LIGHT, BRICKED>(a, src, r, g_img, out + pix, sink);
-  return sink.bound;  // the gather's fixed-point unit comes from this bound
+  return sink.bound.value();  // the gather's fixed-point unit comes from this bound
 }
 
 template <int C, int BM, int MODE, bool LIGHT, bool BRICKED>
