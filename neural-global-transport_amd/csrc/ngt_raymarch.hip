@@ -605,11 +605,11 @@ NGT_DEVICE float raymarch_bwd_prepass_pixel(const VBlock& vb, const RayArgs& a, 
   Vec<C> g_img = vzero<C>();
   if (r.steps > 0) g_img = a.l2_target ? l2_image_grad<C>(a, out + pix, pix / C * 3) : vload<C>(out_grad + pix);
   constexpr int CS = stored_channels(CG);
-  float g_max = 0.f;  // largest colour gradient where only factors are stored
+  GradBound colours;  // of the image gradient, where only factors are stored
   if constexpr (CS != CG) {
     rec.g_scale = g_img.v[0]; rec.g_off = g_img.v[1]; rec.g_blue = g_img.v[2];
 #pragma unroll
-    for (int i = 0; i < 3; ++i) g_max = fmaxf(g_max, fabsf(g_img.v[i])) + (g_img.v[i] - g_img.v[i]);
+    for (int i = 0; i < 3; ++i) colours.add(g_img.v[i]);
   }
   rays[pair * npix + pixel] = rec;
   if (r.steps <= 0) return 0.f;
@@ -652,7 +652,7 @@ NGT_DEVICE float raymarch_bwd_prepass_pixel(const VBlock& vb, const RayArgs& a, 
           if (k + u < steps) one(k + u, qx[u], qy[u], qz[u], g, t[u], gd[u]);
       }
     }
-  } sink{a, G + static_cast<int64_t>(pair) * kcap * g_pixels(npix) * CS, pixel, kcap, g_max, {}};
+  } sink{a, G + static_cast<int64_t>(pair) * kcap * g_pixels(npix) * CS, pixel, kcap, colours.value(), {}};
   walk_ray_gradient<C, LINEAR, BM, MODE, LIGHT, BRICKED>(a, src, r, g_img, out + pix, sink);
   return sink.bound.value();  // the gather's fixed-point unit comes from this bound
 }

@@ -42,3 +42,10 @@ def check(ops, monkeypatch, C, blend, channel):
                          [(4, b, c) for b in ("BEER_LAMBERT", "ALPHA_ADDITIVE") for c in range(4)])
 def test_nonfinite_gradient_reaches_the_bound(ngt_ops, monkeypatch, C, blend, channel):  # noqa: F811
     check(ngt_ops, monkeypatch, C, blend, channel)
+
+
+@pytest.mark.parametrize("blend", ["ADDITIVE", "ALPHA"])
+@pytest.mark.parametrize("channel", range(4))
+def test_nonfinite_colour_reaches_the_bound(ngt_ops, monkeypatch, blend, channel):  # noqa: F811
+    """Blends whose last channel's gradient can stay finite beside a colour's that is not."""
+    check(ngt_ops, monkeypatch, 4, blend, channel)
