@@ -769,8 +769,9 @@ __global__ __launch_bounds__(256) void xform_bwd_kernel(XformArgs a, CamBatch cb
 //
 // A launch takes up to kMaxCamsPerLaunch (grid, camera) pairs and the bricks of
 // the grids that these view, so that the bricks of all launches grow with the
-// pairs: 64 grids of 64^3 into 16^3 cells, 1 channel, 137 us, 1024 of 32^3
-// into 8^3 1.1 ms (the bricks of every grid in each launch: 648 us and 18.6 ms).
+// pairs: 64 grids of 64^3 into 32^3 cells around them, 4 channels, 223 us
+// (with the bricks of every grid in each launch 64 grids of 64^3 into 16^3
+// cells, 1 channel, took 648 us, without 137; these scatter now, in 55).
 struct GridRange {
   int begin, count;  // the grids that the launch's pairs view
   int begin_new;     // the first of them that no earlier launch has stored
@@ -1259,6 +1260,36 @@ bool grid_in_front(const CamParams& cp, const Dims& din, const Dims& dout, int l
   return true;
 }
 
+// Output cells in the box that a grid before the camera takes of its view: 1.4
+// to 2.5 times the cells that sample it, and exactly these where the map is one
+// of the axes.
+double cells_around_grid(const CamParams& cp, const Dims& din, const Dims& dout, int coord_mode) {
+  double lo[3] = {1e300, 1e300, 1e300}, hi[3] = {-1e300, -1e300, -1e300};
+  for (int c = 0; c < 8; ++c) {
+    double o[3];
+    output_index<double>(cp, dout, coord_mode != NGT_COORD_TRANSFORM, (c & 1) ? din.x : 0, (c & 2) ? din.y : 0,
+                         (c & 4) ? din.z : 0, o);
+    for (int k = 0; k < 3; ++k) {
+      lo[k] = std::min(lo[k], o[k]);
+      hi[k] = std::max(hi[k], o[k]);
+    }
+  }
+  const double dims[3] = {static_cast<double>(dout.x), static_cast<double>(dout.y), static_cast<double>(dout.z)};
+  double cells = 1.0;
+  for (int k = 0; k < 3; ++k) cells *= std::max(0.0, std::min(hi[k], dims[k]) - std::max(lo[k], 0.0));
+  return cells;
+}
+
+// Whether output index and grid position differ by a scale and a shift per axis
+// (resampling between grids): consecutive cells then scatter to consecutive
+// voxels, which the atomics take several times faster.
+bool maps_axes(const CamParams& cp) {
+  for (int r = 0; r < 4; ++r)
+    for (int c = 0; c < 4; ++c)
+      if (r != c && (cp.p_inv[4 * r + c] != 0.f || (c < 3 && cp.mv_inv[4 * r + c] != 0.f))) return false;
+  return true;
+}
+
 bool same_maps(const CamParams& a, const CamParams& b) {
   return std::memcmp(a.mv, b.mv, sizeof(a.mv)) == 0 && std::memcmp(a.mv_inv, b.mv_inv, sizeof(a.mv_inv)) == 0 &&
          std::memcmp(a.p, b.p, sizeof(a.p)) == 0 && std::memcmp(a.p_inv, b.p_inv, sizeof(a.p_inv)) == 0 &&
@@ -1267,21 +1298,47 @@ bool same_maps(const CamParams& a, const CamParams& b) {
 
 // The gather serves LINEAR, BORDER and the forward modes, for cameras whose
 // maps agree and that stand before the grid (a brick that the camera's plane
-// cuts would try every output cell in one work-group); other calls scatter.
-bool use_xform_gather(const std::vector<CamParams>& cams, const XformArgs& a, int64_t n_data, int levels,
+// cuts would try every output cell in one work-group), where the values that
+// sample the grids are not too few: it visits every brick of every level, the
+// scatter only the samples.  Other calls scatter.  The lines, in values (cells
+// around the grid times channels) per voxel, and scatter / gather in us of
+// 128^3 grids of one channel, the one grid in a 128^3-cell view scaled by t:
+//   perspective, no mips   0.05   t = 0.4 (0.012): 11 / 17, 0.5 (0.025): 14 / 17, 0.75 (0.08): 27 / 17
+//   perspective, 2 levels  0.15   0.5: 28 / 53, 0.75: 60 / 56, 1 (0.2): 93 / 64
+//   axes, no mips          0.1    0.4 (0.06): 14 / 17, 0.5 (0.12): 18 / 17, 0.75 (0.42): 37 / 18
+//   axes, 2 levels         1.5    0.5: 29 / 56, 1 (1): 75 / 118, 1.5 (3.4): 1372 / 294
+// the last divided by the channels once more (four of them in 0.5: 143 / 69, the
+// scatter's atomics then lying 16 bytes apart).  With more pairs than one launch
+// takes, each launch also needs enough values to be worth its 6 us (12 with
+// levels) against the scatter's 3: 128 grids of 32^3 with three views each of
+// 16^3 / 32^3 / 48^3 cells, 48 launches, 1.48 / 1.15 / 0.27 times the scatter.
+bool use_xform_gather(const std::vector<CamParams>& cams, const XformArgs& a, int64_t n_data, int channels, int levels,
                       int interpolation, int boundary) {
   if (interpolation != LINEAR || boundary != BORDER) return false;
   if (a.coord_mode != NGT_COORD_TRANSFORM && a.coord_mode != NGT_COORD_TRANSFORM_LINDEPTH) return false;
   if (dims_cells(a.dout) >= (int64_t(1) << 30) || dims_cells(a.din) * n_data >= (int64_t(1) << 36)) return false;
   // the views of the grids after the first are mostly the first one's again
-  // (comparing takes 0.02 us of the host, checking 0.45)
+  // (comparing takes 0.02 us of the host, checking 0.6)
   const size_t views = static_cast<size_t>(
       std::find_if(cams.begin(), cams.end(), [](const CamParams& c) { return c.data_index != 0; }) - cams.begin());
+  const double voxels = static_cast<double>(dims_cells(a.din)) * static_cast<double>(n_data);
+  double values = 0.0;
+  bool axes = true;
+  std::vector<double> cells(cams.size());
   for (size_t i = 0; i < cams.size(); ++i) {
-    if (i >= views && same_maps(cams[i], cams[i - views])) continue;
-    if (!maps_agree(cams[i], a.dout, a.coord_mode) || !grid_in_front(cams[i], a.din, a.dout, levels)) return false;
+    if (i >= views && same_maps(cams[i], cams[i - views])) {
+      cells[i] = cells[i - views];
+    } else {
+      if (!maps_agree(cams[i], a.dout, a.coord_mode) || !grid_in_front(cams[i], a.din, a.dout, levels)) return false;
+      cells[i] = cells_around_grid(cams[i], a.din, a.dout, a.coord_mode);
+      axes = axes && maps_axes(cams[i]);
+    }
+    values += cells[i] * channels;
   }
-  return true;
+  const double line = levels == 0 ? (axes ? 0.1 : 0.05) : (axes ? 1.5 / channels : 0.15);
+  if (!(values >= line * voxels)) return false;
+  const double launches = std::ceil(static_cast<double>(cams.size()) / kMaxCamsPerLaunch);
+  return launches == 1.0 || values >= launches * (levels == 0 ? 32768.0 : 49152.0);
 }
 
 template <int C, int MM, int BX, int BY, int BZ>
@@ -1496,7 +1553,8 @@ int ngt_sample_grid_transform_bwd(const float* input, const int64_t* input_shape
   const MipSet grad = make_mips(input_grad, input_shape, mip ? workspace : nullptr, mip ? num_mipmaps : 0);
   hipStream_t s = as_stream(stream);
   const std::vector<CamParams> cams = make_cams(pairs, matrix_m, matrix_v, matrix_p, frustum);
-  if (!ref && use_xform_gather(cams, a, si.n, grad.num_levels, interpolation, boundary)) {
+  if (!ref && use_xform_gather(cams, a, si.n, static_cast<int>(si.c), grad.num_levels, interpolation,
+                               boundary)) {
     const int64_t at_once = grid_range(cams, 0).count;  // grids of a launch
     const int first_split = first_split_level(grad.d0, a.dout, at_once, si.c);
     const int64_t stored = mip_floats(si.dims(), si.n, si.c, std::max(first_split - 1, 0));

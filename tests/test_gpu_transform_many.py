@@ -1,7 +1,9 @@
-"""GPU parity of the transform adjoint's brick gather over many grids, whose
-launches each take the bricks of the grids that their camera pairs view, against
-the FP64 oracle: grids that end a launch, grids whose views are split between
-launches, levels that work-groups share.
+"""GPU parity of the transform adjoint against the FP64 oracle on both sides of
+its line between the brick gather, which visits every voxel, and the scatter,
+which visits the samples; and of the gather over many grids, whose launches each
+take the bricks of the grids that their camera pairs view: grids that end a
+launch, grids whose views are split between launches, levels that work-groups
+share.
 
 Tolerance: gradients 1e-4 of the largest value, as for the other adjoints.
 """
@@ -9,6 +11,7 @@ import numpy as np
 import pytest
 
 from oracle import BORDER, LINEAR
+from oracle import geometry as G
 from oracle import mips as MP
 from oracle import resample as R
 from test_gpu_transform_gather import cameras, dev, f32, host, ngt_ops, rel  # noqa: F401  (the module's fixture)
@@ -39,7 +42,25 @@ def check(ops, cams, dims, out_dhw, C, n, views, levels, mode, seed):
     ((17, 23, 19), (28, 26, 29), 2, 2, 5, 4),    # shared levels in two launches
     ((11, 9, 13), (40, 33, 35), 1, 2, 5, 0),     # the finest level shared, two launches
     ((96, 64, 94), (33, 32, 34), 4, 1, 2, 3),    # level 2 not shared: 4 channels, 144 bricks
+    ((9, 8, 10), (5, 4, 6), 1, 17, 1, 0),        # too few values for three launches: scatter
+    ((40, 36, 33), (7, 6, 5), 1, 1, 1, 0),       # too few for the voxels
+    ((40, 36, 33), (7, 6, 5), 2, 2, 5, 2),
 ])
 def test_adjoint_of_many_grids(ngt_ops, dims, out_dhw, C, n, views, levels):  # noqa: F811
     check(ngt_ops, cameras(dims, out_dhw, views, n, *CLOSE), dims, out_dhw, C, n, views, levels, "TRANSFORM_LINDEPTH",
           300 + n + 7 * C + 3 * views + levels)
+
+
+@pytest.mark.parametrize("dims,out_dhw,C,levels", [
+    ((24, 20, 22), (10, 9, 8), 1, 0),    # 0.07 values a voxel: scatter
+    ((24, 20, 22), (15, 14, 13), 1, 0),  # 0.26: gather
+    ((24, 20, 22), (26, 21, 23), 1, 2),  # 1.2: scatter
+    ((24, 20, 22), (30, 26, 24), 1, 2),  # 1.8: gather
+    ((24, 20, 22), (15, 14, 13), 4, 2),  # 1.03 with 4 channels: gather
+])
+def test_adjoint_along_the_axes(ngt_ops, dims, out_dhw, C, levels):  # noqa: F811
+    """A grid over the [-1, 1] cube through an orthographic camera of it, as resampling has it."""
+    M = G.grid_transform(dims, center=True, scale_=[2.0 / dims[2], 2.0 / dims[1], 2.0 / dims[0]])
+    cams = ([G.op_matrix(M).astype(np.float32)], [np.eye(4, dtype=np.float32).reshape(16)],
+            [np.eye(4, dtype=np.float32).reshape(16)], [np.asarray([-1, 1, -1, 1, 1, -1], dtype=np.float32)])
+    check(ngt_ops, cams, dims, out_dhw, C, 1, 1, levels, "TRANSFORM", 700 + C + levels)
