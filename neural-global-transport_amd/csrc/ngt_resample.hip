@@ -829,12 +829,13 @@ NGT_HOST_DEVICE_INLINE int level_splits(int m, int first) {
 // leave half of the CUs idle (48^3 into 128x72x96 x 3, 1 channel, 1 / 2 / 3 levels:
 // 146 / 200 / 250 us against 425 / 434 / 461; 24^3 into 24^3: 49 / 52 / 52 against
 // 55 / 61 / 64), and from the finest on where that has few bricks and each of
-// its voxels 16 or more cells of a view (16^3 into 64^3 x 3, 1 channel, 0 / 1 / 3
-// levels: 52 / 90 / 100 us against 156 / 365 / 372; 24^3 into 96^3: 61 / 131 / 200
-// against 166 / 472 / 516).
+// its voxels 4 or more cells of a view (16^3 into 64^3 x 3, 1 channel, 0 / 1 / 3
+// levels: 52 / 90 / 100 us against 156 / 365 / 372; 16^3 that fill a 26^3-cell
+// view, 4.3 cells a voxel, 0 / 1: 7.8 / 12.2 against 9.0 / 17.9, and 13.4 with the
+// scatter).
 inline int first_split_level(const Dims& d, const Dims& dout, int64_t n, int64_t c) {
   const auto bricks = [&](int m) { return level_bricks<8, 4, 4>(d, m).count() * n; };
-  if (bricks(0) < 128 && dims_cells(dout) >= 16 * dims_cells(d)) return 0;
+  if (bricks(0) < 128 && dims_cells(dout) >= 4 * dims_cells(d)) return 0;
   return bricks(1) < 128 ? 1 : (c < 4 || bricks(2) < 128 ? 2 : 3);
 }
 

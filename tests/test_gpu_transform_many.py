@@ -42,6 +42,8 @@ def check(ops, cams, dims, out_dhw, C, n, views, levels, mode, seed):
     ((17, 23, 19), (28, 26, 29), 2, 2, 5, 4),    # shared levels in two launches
     ((11, 9, 13), (40, 33, 35), 1, 2, 5, 0),     # the finest level shared, two launches
     ((96, 64, 94), (33, 32, 34), 4, 1, 2, 3),    # level 2 not shared: 4 channels, 144 bricks
+    ((11, 9, 13), (18, 17, 19), 1, 1, 2, 1),     # 4.5 cells a voxel: the finest level shared
+    ((11, 9, 13), (16, 15, 17), 1, 1, 2, 1),     # 3.2: not shared
     ((9, 8, 10), (5, 4, 6), 1, 17, 1, 0),        # too few values for three launches: scatter
     ((40, 36, 33), (7, 6, 5), 1, 1, 1, 0),       # too few for the voxels
     ((40, 36, 33), (7, 6, 5), 2, 2, 5, 2),
