@@ -199,39 +199,53 @@ struct Corner8 {
   bool ok[8];
 };
 
-// The 8 corner loads, branch-free: issued unconditionally from in-grid
-// addresses (BORDER corners clamped into the grid for the address only; the
-// out-of-grid ones are zeroed by mask8 afterwards), so the loads of several
-// samples can be in flight together.  Offsets are 32-bit (a grid slice holds
-// fewer than 2^32 floats, checked on the host).
+// Where the 8 corners of a sample lie: the floor corner's offset and the steps
+// to the ceil corners, in floats.  Offsets are 32-bit (a grid slice holds fewer
+// than 2^32 floats, checked on the host).
+struct CornerSteps {
+  uint32_t base, x, y, z;
+};
+
+// Of in-grid addresses: BORDER corners are clamped into the grid for the address
+// only (the out-of-grid ones are zeroed by mask8 afterwards).
 template <int C, int BM>
-NGT_DEVICE void fetch8_raw(const float* __restrict__ g, const Dims& d, const Corners& c, Vec<C> (&v)[8]) {
+NGT_DEVICE CornerSteps corner_steps(const Dims& d, const Corners& c) {
   int x0 = c.x0, x1 = c.x1, y0 = c.y0, y1 = c.y1, z0 = c.z0, z1 = c.z1;
   if constexpr (BM == BORDER) {
     x0 = min(max(x0, 0), d.x - 1); x1 = min(max(x1, 0), d.x - 1);
     y0 = min(max(y0, 0), d.y - 1); y1 = min(max(y1, 0), d.y - 1);
     z0 = min(max(z0, 0), d.z - 1); z1 = min(max(z1, 0), d.z - 1);
   }
-  const uint32_t W = static_cast<uint32_t>(d.x), H = static_cast<uint32_t>(d.y);
-  if constexpr (BM == WRAP) {
-    const uint32_t rows[4] = {(static_cast<uint32_t>(z0) * H + static_cast<uint32_t>(y0)) * W,
-                              (static_cast<uint32_t>(z0) * H + static_cast<uint32_t>(y1)) * W,
-                              (static_cast<uint32_t>(z1) * H + static_cast<uint32_t>(y0)) * W,
-                              (static_cast<uint32_t>(z1) * H + static_cast<uint32_t>(y1)) * W};
-    const uint32_t xs[2] = {static_cast<uint32_t>(x0), static_cast<uint32_t>(x1)};
-#pragma unroll
-    for (int k = 0; k < 8; ++k) v[k] = vload<C>(g + (rows[k >> 1] + xs[k & 1]) * static_cast<uint32_t>(C));
+  const uint32_t W = static_cast<uint32_t>(d.x), H = static_cast<uint32_t>(d.y), CC = static_cast<uint32_t>(C);
+  CornerSteps s;
+  s.base = ((static_cast<uint32_t>(z0) * H + static_cast<uint32_t>(y0)) * W + static_cast<uint32_t>(x0)) * CC;
+  if constexpr (BM == WRAP) {  // modulo 2^32: a wrapped ceil corner lies below
+    s.x = static_cast<uint32_t>(x1 - x0) * CC;
+    s.y = static_cast<uint32_t>(y1 - y0) * (W * CC);
+    s.z = static_cast<uint32_t>(z1 - z0) * (W * H * CC);
   } else {
     // the clamped ceil index is the floor index or the next: one address is
     // multiplied out (32-bit multiplies run at a quarter of the rate), the
     // other corners are selected steps away
-    const uint32_t base = ((static_cast<uint32_t>(z0) * H + static_cast<uint32_t>(y0)) * W + static_cast<uint32_t>(x0)) * static_cast<uint32_t>(C);
-    const uint32_t sx = x1 != x0 ? static_cast<uint32_t>(C) : 0u, sy = y1 != y0 ? W * static_cast<uint32_t>(C) : 0u,
-                   sz = z1 != z0 ? W * H * static_cast<uint32_t>(C) : 0u;
-    const uint32_t rows[4] = {base, base + sy, base + sz, base + sy + sz};
-#pragma unroll
-    for (int k = 0; k < 8; ++k) v[k] = vload<C>(g + (rows[k >> 1] + ((k & 1) ? sx : 0u)));
+    s.x = x1 != x0 ? CC : 0u;
+    s.y = y1 != y0 ? W * CC : 0u;
+    s.z = z1 != z0 ? W * H * CC : 0u;
   }
+  return s;
+}
+
+// The 8 corner loads, branch-free, so that the loads of several samples can be
+// in flight together.
+template <int C>
+NGT_DEVICE void load8(const float* __restrict__ g, const CornerSteps& s, Vec<C> (&v)[8]) {
+  const uint32_t rows[4] = {s.base, s.base + s.y, s.base + s.z, s.base + s.y + s.z};
+#pragma unroll
+  for (int k = 0; k < 8; ++k) v[k] = vload<C>(g + (rows[k >> 1] + ((k & 1) ? s.x : 0u)));
+}
+
+template <int C, int BM>
+NGT_DEVICE void fetch8_raw(const float* __restrict__ g, const Dims& d, const Corners& c, Vec<C> (&v)[8]) {
+  load8<C>(g, corner_steps<C, BM>(d, c), v);
 }
 
 // Haloed brick layout of a grid slice: the grid is cut into 4x4x4-cell
@@ -348,20 +362,40 @@ NGT_DEVICE void fetch_corners(const float* __restrict__ g, const Dims& d, float 
                        (static_cast<unsigned>(y0) < static_cast<unsigned>(d.y - 1)) &
                        (static_cast<unsigned>(z0) < static_cast<unsigned>(d.z - 1)) & (wx > 0.f) & (wy > 0.f) &
                        (wz > 0.f);
-  if (__all(between)) {
-    c.wx = wx; c.wy = wy; c.wz = wz;
-    c.inside = true;
-    const uint32_t row = static_cast<uint32_t>(d.x) * C;
-    const uint32_t plane = static_cast<uint32_t>(d.y) * row;
-    const float* const p = g + ((static_cast<uint32_t>(z0) * static_cast<uint32_t>(d.y) + static_cast<uint32_t>(y0)) * row +
-                                static_cast<uint32_t>(x0) * static_cast<uint32_t>(C));
-    const float* const rows[4] = {p, p + row, p + plane, p + plane + row};
+  const uint32_t row = static_cast<uint32_t>(d.x) * C;
+  const uint32_t plane = static_cast<uint32_t>(d.y) * row;
+  const auto floor_corner = [&] {
+    return (static_cast<uint32_t>(z0) * static_cast<uint32_t>(d.y) + static_cast<uint32_t>(y0)) * row +
+           static_cast<uint32_t>(x0) * static_cast<uint32_t>(C);
+  };
+  if constexpr (BM == BORDER) {
+    if (__all(between)) {
+      c.wx = wx; c.wy = wy; c.wz = wz;
+      c.inside = true;
+      const float* const p = g + floor_corner();
+      const float* const rows[4] = {p, p + row, p + plane, p + plane + row};
 #pragma unroll
-    for (int k = 0; k < 8; ++k) v[k] = vload<C>(rows[k >> 1] + (k & 1) * C);
+      for (int k = 0; k < 8; ++k) v[k] = vload<C>(rows[k >> 1] + (k & 1) * C);
+    } else {
+      c = make_corners<BM>(d, qx, qy, qz);
+      fetch8_raw<C, BM>(g, d, c, v);
+      mask8<C, BM>(c, v);
+    }
   } else {
-    c = make_corners<BM>(d, qx, qy, qz);
-    fetch8_raw<C, BM>(g, d, c, v);
-    mask8<C, BM>(c, v);
+    // nothing is masked after the loads, so only the addresses are formed in
+    // branches: with the loads in them the compiler merges the two sets and
+    // splits each into single floats (a 128^3 table read of four channels, CLAMP
+    // / WRAP: 39.2 / 40.2 us against 22.3 / 23.5)
+    CornerSteps s;
+    if (__all(between)) {
+      c.wx = wx; c.wy = wy; c.wz = wz;
+      c.inside = true;
+      s = CornerSteps{floor_corner(), static_cast<uint32_t>(C), row, plane};
+    } else {
+      c = make_corners<BM>(d, qx, qy, qz);
+      s = corner_steps<C, BM>(d, c);
+    }
+    load8<C>(g, s, v);
   }
 }
 
