@@ -474,7 +474,7 @@ __global__ __launch_bounds__(256) void mac_component_luts_bwd_kernel(Dims d, Mac
 
 // ---------------------------------------------------------------------------
 // Brick-tiled exact backward.  A work-group owns a brick of
-// kBrickX x kBrickY x kBrickZ cells and an LDS tile of the brick grown by
+// kBrickX x kBrickY cells, 4, 8 or 16 deep, and an LDS tile of the brick grown by
 // kHalo cells on every side.  The trilinear scatter of the brick's samples
 // lands in the tile whenever the displacement s = ts*v per axis satisfies
 // -kHalo < s <= kHalo (the corners floor(x - s), floor(x - s) + 1 then lie in
@@ -488,27 +488,23 @@ __global__ __launch_bounds__(256) void mac_component_luts_bwd_kernel(Dims d, Mac
 // The tile holds doubles: the LDS adds fp64 atomically at 6.7 lanes per clock
 // and CU (3.0 at random addresses) but fp32 at 0.33, so a sample's 8 corners
 // are added as they are.  (Within a tile the atomics add in no fixed order;
-// in fp64 that changes the stored fp32 partials hardly ever.)  One channel's
-// tile is 41 KB, three work-groups per CU; several channels take turns in it.
+// in fp64 that changes the stored fp32 partials hardly ever.)  Several channels
+// take turns in it.
 // Measured: 128^3, one channel, B1 / B2 45.6 / 45.7 us with fp32 tiles and
 // merged neighbours -> 40.1 / 38.6 with fp64 tiles -> 31.4 / 37.0 with the
 // unmasked corner reads and the offsets of gather_tiles, at 3.3 / 3.6 TB/s of
 // their fields, tiles and velocity gradients; 96x160x96, three channels, 717 /
 // 597 us with global fp32 atomics -> 58 / 68.  The halo sets the partial-buffer
-// traffic: tile cells per brick cell 2.53 with kHalo = 2 (2.11 with bricks 16
-// deep, which measured the same at 128^3 and 30 % slower at 96x160x96).
-constexpr int kBrickX = 32, kBrickY = 8, kBrickZ = 8, kHalo = 2;
+// traffic: tile cells per brick cell 2.11, 2.53 or 3.38 with kHalo = 2 and
+// bricks 16, 8 or 4 deep.
+constexpr int kBrickX = 32, kBrickY = 8, kHalo = 2;
 // a work-group is kBrickX x kBrickY x kBrickZT work-items; each visits the
 // brick's z extent / kBrickZT cells of its (x, y) column
 constexpr int kBrickZT = 2;
 constexpr int kBrickThreads = kBrickX * kBrickY * kBrickZT;
-constexpr int kTileX = kBrickX + 2 * kHalo, kTileY = kBrickY + 2 * kHalo, kTileZ = kBrickZ + 2 * kHalo;
-constexpr int kTilePlane = kTileX * kTileY, kTileCells = kTilePlane * kTileZ;
+constexpr int kTileX = kBrickX + 2 * kHalo, kTileY = kBrickY + 2 * kHalo;
+constexpr int kTilePlane = kTileX * kTileY;
 
-// Bricks are 8 cells deep in z, or 4 where that leaves a CU with fewer than two
-// of them: the halves then run on more CUs (64^3: B1 / B2 14.6 / 15.9 us ->
-// 12.3 / 12.1; at 96x160x96, 720 deep bricks, 30.0 / 26.5 us against 31.4 /
-// 29.1 with flat ones, whose halos weigh more).
 struct BrickGrid {
   int nx, ny, nz;
   int zl;  // log2 of the z extent
@@ -516,6 +512,7 @@ struct BrickGrid {
   __host__ __device__ int depth() const { return 1 << zl; }
   __host__ __device__ int tile_planes() const { return depth() + 2 * kHalo; }
   __host__ __device__ int tile_cells() const { return kTilePlane * tile_planes(); }
+  unsigned tile_bytes() const { return static_cast<unsigned>(tile_cells() * sizeof(double)); }  // of LDS
 };
 
 inline BrickGrid brick_grid_of_depth(const Dims& d, int zl) {
@@ -523,12 +520,24 @@ inline BrickGrid brick_grid_of_depth(const Dims& d, int zl) {
                    static_cast<int>(blocks_for(d.z, 1 << zl)), zl};
 }
 
-constexpr int64_t kFewBricks = 512;  // two per CU
+// Bricks are as shallow as all of them run at once, three to a CU, else 16 cells
+// deep: while CUs stand idle, more of them share the cells, and after that the
+// halos and the corners that leave the tiles count.  Both passes of order 2,
+// bricks 4 / 8 / 16 deep (bricks 8 deep: 64^3 128, 96^3 432, 96x160x96 720, 112^3
+// 784, 128^3 1024), in us: one channel, smooth displacements up to 2 cells: 25 / 31
+// / 48, 47 / 47 / 57, 63 / 60 / 74, 71 / 74 / 72, 83 / 82 / 80; random ones up to 8,
+// most of whose corners leave the tile: 131 / 110 / 131, 427 / 354 / 289, 695 / 553
+// / 491, 664 / 559 / 468, 1024 / 798 / 676; three channels, smooth: 96^3 105 / 98 /
+// 115, 128^3 227 / 206 / 201.
+constexpr int64_t kBricksAtOnce = 768;
+
+inline int brick_depth_log2(int64_t count4, int64_t count8) {
+  return count4 <= kBricksAtOnce ? 2 : (count8 <= kBricksAtOnce ? 3 : 4);
+}
 
 inline BrickGrid brick_grid(const Dims& d, int64_t pairs) {
-  static_assert(kBrickZ == 8, "depths 8 and 4");
-  const BrickGrid deep = brick_grid_of_depth(d, 3);
-  return deep.count() * pairs < kFewBricks ? brick_grid_of_depth(d, 2) : deep;
+  return brick_grid_of_depth(d, brick_depth_log2(brick_grid_of_depth(d, 2).count() * pairs,
+                                                 brick_grid_of_depth(d, 3).count() * pairs));
 }
 
 // Scatter val * w to the 8 corners of q: into the LDS tile (origin o*, that
@@ -711,7 +720,7 @@ NGT_DEVICE void advect_mc_bwd_brick_kernel_body(const VBlock& vb, const AdvArgs&
                                                 const float* __restrict__ sl, const float* __restrict__ g_out,
                                                 float* __restrict__ g_dir, float* r_dir, float* __restrict__ ovf,
                                                 float* __restrict__ tiles, const GradVel& gv, int vel_mode) {
-  __shared__ double tile[kTileCells];
+  extern __shared__ double tile[];  // bg.tile_cells()
   tile_clear(tile, bg);
   const BrickCell b = brick_cell(bg, vb);
   int n, v;
@@ -791,7 +800,7 @@ NGT_DEVICE void advect_sl_bwd_brick_kernel_body(const VBlock& vb, const AdvArgs&
                                                 const float* __restrict__ tiles1, float* __restrict__ g_rho,
                                                 float* __restrict__ tiles2, const GradVel& gv, int vel_mode,
                                                 float* val) {
-  __shared__ double tile[kTileCells];
+  extern __shared__ double tile[];  // bg.tile_cells()
   tile_clear(tile, bg);
   const BrickCell b = brick_cell(bg, vb);
   int n, v;
@@ -1001,6 +1010,7 @@ void launch_faces(const AdvPlan& p, const GradVel& gv, float* gx, float* gy, flo
 struct AdvBatchHeader {
   int n, order, clamp, boundary, staggered;
   int tiles_cell, tiles_brick, tiles_fill;
+  unsigned tile_bytes;  // LDS of the brick kernels
   size_t off_items, off_cell, off_brick, off_fill;
   int64_t ws_bytes;
 };
@@ -1342,16 +1352,16 @@ int ngt_advect_bwd(const float* input, const int64_t* input_shape, const float* 
       float* rd = direct ? input_grad : r_dir;
       const float* g_b2 = pass_g ? output_grad : g_sl;
       NGT_SWITCH_C(p.C, NGT_SWITCH_BM(boundary, NGT_SWITCH_CLAMP(clamp,
-          hipLaunchKernelGGL((advect_mc_bwd_brick_kernel<CC, BB, KK>), bgrid, bblock, 0, s, p.a, bg, input, slp,
+          hipLaunchKernelGGL((advect_mc_bwd_brick_kernel<CC, BB, KK>), bgrid, bblock, bg.tile_bytes(), s, p.a, bg, input, slp,
                              output_grad, g_dir, rd, ovf1, tiles1, gv, vel_mode);
-          hipLaunchKernelGGL((advect_sl_bwd_brick_kernel<CC, BB, false, true>), bgrid, bblock, 0, s, p.a, bg, input,
+          hipLaunchKernelGGL((advect_sl_bwd_brick_kernel<CC, BB, false, true>), bgrid, bblock, bg.tile_bytes(), s, p.a, bg, input,
                              g_b2, ovf1, tiles1, input_grad, tiles2, gv, vel_mode, val))));
     } else {
       NGT_SWITCH_C(p.C, NGT_SWITCH_BM(boundary,
-          if (neg) hipLaunchKernelGGL((advect_sl_bwd_brick_kernel<CC, BB, true, false>), bgrid, bblock, 0, s, p.a, bg,
+          if (neg) hipLaunchKernelGGL((advect_sl_bwd_brick_kernel<CC, BB, true, false>), bgrid, bblock, bg.tile_bytes(), s, p.a, bg,
                                       input, output_grad, nullptr, nullptr, input_grad, tiles2, gv, vel_mode,
                                       val);
-          else hipLaunchKernelGGL((advect_sl_bwd_brick_kernel<CC, BB, false, false>), bgrid, bblock, 0, s, p.a, bg,
+          else hipLaunchKernelGGL((advect_sl_bwd_brick_kernel<CC, BB, false, false>), bgrid, bblock, bg.tile_bytes(), s, p.a, bg,
                                   input, output_grad, nullptr, nullptr, input_grad, tiles2, gv, vel_mode, val)));
     }
     const dim3 dgrid(blocks_for(p.a.d.x, kBX), blocks_for(p.a.d.y, kBY), static_cast<unsigned>(p.a.d.z * p.a.n_data));
@@ -1420,11 +1430,16 @@ int ngt_advect_batch_plan(const ngt_advect_instance* inst, int n, int order, int
   int* brick = blob_at<int>(plan, off_brick);
   int* fill = blob_at<int>(plan, off_fill);
   const int staggered = inst[0].vel_y != nullptr ? 1 : 0;
-  // the bricks of all instances share the CUs, so their depth is one
-  int64_t deep = 0;
-  for (int i = 0; i < n; ++i)
-    deep += brick_grid_of_depth(Dims{inst[i].dhw[2], inst[i].dhw[1], inst[i].dhw[0]}, 3).count();
-  const int zl = deep < kFewBricks ? 2 : 3;
+  // the bricks of all instances share the CUs, so their depth is one; the few
+  // work-groups of a persistent launch end too unevenly with bricks 16 deep
+  // (eight instances of 48^3 to 128^3: 811 us a step against 773)
+  int64_t count4 = 0, count8 = 0;
+  for (int i = 0; i < n; ++i) {
+    const Dims d{inst[i].dhw[2], inst[i].dhw[1], inst[i].dhw[0]};
+    count4 += brick_grid_of_depth(d, 2).count();
+    count8 += brick_grid_of_depth(d, 3).count();
+  }
+  const int zl = std::min(brick_depth_log2(count4, count8), 3);
   int64_t tc = 0, tb = 0, tl = 0, ws = 0;
   cell[0] = brick[0] = fill[0] = 0;
   for (int i = 0; i < n; ++i) {
@@ -1470,6 +1485,7 @@ int ngt_advect_batch_plan(const ngt_advect_instance* inst, int n, int order, int
   h->n = n; h->order = order; h->clamp = clamp; h->boundary = boundary; h->staggered = staggered;
   h->tiles_cell = static_cast<int>(tc); h->tiles_brick = static_cast<int>(tb);
   h->tiles_fill = static_cast<int>(tl);
+  h->tile_bytes = items[0].bg.tile_bytes();
   h->off_items = off_items; h->off_cell = off_cell; h->off_brick = off_brick; h->off_fill = off_fill;
   h->ws_bytes = ws * static_cast<int64_t>(sizeof(float));
   if (workspace_bytes) *workspace_bytes = static_cast<size_t>(h->ws_bytes);
@@ -1517,13 +1533,13 @@ int ngt_advect_batch_bwd(const void* plan_host, const void* plan_device, void* w
   const dim3 gb(persistent_grid(h.tiles_brick, blocks_per_cu)), bb(kBrickX, kBrickY, kBrickZT);
   if (h.order == 2) {
     NGT_SWITCH_BM(h.boundary, NGT_SWITCH_CLAMP(h.clamp,
-        hipLaunchKernelGGL((advect_mc_bwd_batch_kernel<BB, KK>), gb, bb, 0, s, plan_device, ws);
-        hipLaunchKernelGGL((advect_sl_bwd_batch_kernel<BB, false, true>), gb, bb, 0, s, plan_device, ws)));
+        hipLaunchKernelGGL((advect_mc_bwd_batch_kernel<BB, KK>), gb, bb, h.tile_bytes, s, plan_device, ws);
+        hipLaunchKernelGGL((advect_sl_bwd_batch_kernel<BB, false, true>), gb, bb, h.tile_bytes, s, plan_device, ws)));
   } else {
     const bool neg = h.clamp == NGT_CLAMP_NEGATIVE;
     NGT_SWITCH_BM(h.boundary,
-        if (neg) hipLaunchKernelGGL((advect_sl_bwd_batch_kernel<BB, true, false>), gb, bb, 0, s, plan_device, ws);
-        else hipLaunchKernelGGL((advect_sl_bwd_batch_kernel<BB, false, false>), gb, bb, 0, s, plan_device, ws));
+        if (neg) hipLaunchKernelGGL((advect_sl_bwd_batch_kernel<BB, true, false>), gb, bb, h.tile_bytes, s, plan_device, ws);
+        else hipLaunchKernelGGL((advect_sl_bwd_batch_kernel<BB, false, false>), gb, bb, h.tile_bytes, s, plan_device, ws));
   }
   hipLaunchKernelGGL(advect_rho_gather_batch_kernel, dim3(persistent_grid(h.tiles_cell, blocks_per_cu)), b, 0, s,
                      plan_device, ws);
