@@ -563,7 +563,7 @@ struct GradBound {
   float largest = 0.f, not_finite = 0.f;
   NGT_DEVICE void add(float v) {
     largest = fmaxf(largest, fabsf(v));
-    not_finite += v - v;
+    not_finite = fmaf(v, 0.f, not_finite);
   }
   NGT_DEVICE float value() const { return largest + not_finite; }
 };
@@ -620,37 +620,40 @@ NGT_DEVICE float raymarch_bwd_prepass_pixel(const VBlock& vb, const RayArgs& a, 
     int kcap;
     float g_max;
     GradBound bound;
-    NGT_DEVICE void one(int k, float, float, float, const Vec<C>& g, float t, float gd) {
-      float* const at = gp + g_offset(k, pixel, kcap) * CS;
+    // the stored values of a sample
+    NGT_DEVICE Vec<CS> factors(const Vec<C>& g, float t, float gd, bool live) {
+      Vec<CS> v;
       if constexpr (CS != CG) {
-        vstore<2>(at, Vec<2>{{t, gd}});
-        bound.add(t * g_max);
-        bound.add(gd);
+        v = Vec<CS>{{t, gd}};
+        bound.add(live ? t * g_max : 0.f);
+        bound.add(live ? gd : 0.f);
       } else {
-        const Vec<CG> v = fold_cell_grad<C, LIGHT>(a, cell_grad(g, t, gd));
-        vstore<CG>(at, v);
+        v = fold_cell_grad<C, LIGHT>(a, cell_grad(g, t, gd));
 #pragma unroll
-        for (int i = 0; i < CG; ++i) bound.add(v.v[i]);
+        for (int i = 0; i < CG; ++i) bound.add(live ? v.v[i] : 0.f);
       }
+      return v;
     }
-    // a round of two samples starts at an even k: its factors are one 16-byte
-    // store inside the quad (past the ray's end: a slot that is never read)
+    NGT_DEVICE void one(int k, float, float, float, const Vec<C>& g, float t, float gd) {
+      vstore<CS>(gp + g_offset(k, pixel, kcap) * CS, factors(g, t, gd, true));
+    }
+    // a round of two samples starts at an even k: its values are one 8- or 16-byte
+    // store inside the quad (past the ray's end: a slot that is never read).  A
+    // store of its own for each live sample lets the compiler move the second
+    // one's corner loads behind the first one's store (128^3, 8 views of 480x270,
+    // ALPHA_ADDITIVE, with the image: 239 us, one store 215).
     NGT_DEVICE void round(int k, int steps, const float (&qx)[kUnroll], const float (&qy)[kUnroll],
                           const float (&qz)[kUnroll], const Vec<C>& g, const float (&t)[kUnroll],
                           const float (&gd)[kUnroll]) {
-      if constexpr (CS != CG) {
-        static_assert(kUnroll == 2 && CS == 2, "two samples of two factors");
-        vstore<4>(gp + g_offset(k, pixel, kcap) * CS, Vec<4>{{t[0], gd[0], t[1], gd[1]}});
+      static_assert(kUnroll == 2 && kGQuad % kUnroll == 0 && CS <= 2, "two samples of one or two values");
+      const Vec<CS> v0 = factors(g, t[0], gd[0], true), v1 = factors(g, t[1], gd[1], k + 1 < steps);
+      Vec<2 * CS> v;
 #pragma unroll
-        for (int u = 0; u < kUnroll; ++u) {
-          bound.add(k + u < steps ? t[u] * g_max : 0.f);
-          bound.add(k + u < steps ? gd[u] : 0.f);
-        }
-      } else {
-#pragma unroll
-        for (int u = 0; u < kUnroll; ++u)
-          if (k + u < steps) one(k + u, qx[u], qy[u], qz[u], g, t[u], gd[u]);
+      for (int i = 0; i < CS; ++i) {
+        v.v[i] = v0.v[i];
+        v.v[CS + i] = v1.v[i];
       }
+      vstore<2 * CS>(gp + g_offset(k, pixel, kcap) * CS, v);
     }
   } sink{a, G + static_cast<int64_t>(pair) * kcap * g_pixels(npix) * CS, pixel, kcap, colours.value(), {}};
   walk_ray_gradient<C, LINEAR, BM, MODE, LIGHT, BRICKED>(a, src, r, g_img, out + pix, sink);
