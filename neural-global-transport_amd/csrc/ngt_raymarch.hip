@@ -1570,8 +1570,12 @@ void run_gather(const std::vector<Pair>& pairs, const float* M, const float* V, 
     // 150x100: 23 / 19 / 18;  64 x 5 of 256x144: 84 / 52 / 37;  24 x 3 of 128x72:
     // 81 / 50 / 32.  So 16^3 from 320 bricks on (112^3 has 343, 96^3 216), then 16
     // x 8 x 8 from 768 on (96^3 has 864, 80^3 500).  (16 x 16 x 8 with 256
-    // work-items: 254 / 47 / 33 / 51 / 226 / 25 / 84 / 83.)  Four channels at 96 x
-    // 5: 8^3 105 us, 16 x 8 x 8 113.
+    // work-items: 254 / 47 / 33 / 51 / 226 / 25 / 84 / 83.)  Two and four channels,
+    // walk and gather with bricks of 8^3 / 16 x 8 x 8:  64 x 8 of 480x270 273 / 366
+    // and 390 / 492;  96 x 5 of 256x144 110 / 119 and 181 / 189;  112 x 5 136 / 136
+    // and 224 / 233, x 2 of 128x72 62 / 58 and 88 / 86;  128 x 5 166 / 162 and 279 /
+    // 279, x 2 77 / 70 and 114 / 108;  160 x 5 254 / 241 and 433 / 432, x 2 121 / 108
+    // and 197 / 187.  So 16 x 8 x 8 from 2048 on (128^3 has 2048, 112^3 1372).
     const int accumulate = b > 0 ? 1 : 0;
     const int CG = LIGHT ? 1 : C;
     const auto bricks = [&](int bx, int by, int bz) {
@@ -1581,9 +1585,10 @@ void run_gather(const std::vector<Pair>& pairs, const float* M, const float* V, 
     if (CG == 1 && bricks(16, 16, 16) >= 320) {
       hipLaunchKernelGGL((raymarch_bwd_brick_kernel<1, 16, 16, 16, 512>), dim3(bricks(16, 16, 16)), dim3(512), 0, s, a, cb,
                          base, gp.rays, gp.bound, gp.G, gp.kcap, in_grad, accumulate, scale);
-    } else if (CG == 1 && bricks(16, 8, 8) >= 768) {
-      hipLaunchKernelGGL((raymarch_bwd_brick_kernel<1, 16, 8, 8>), dim3(bricks(16, 8, 8)), dim3(256), 0, s, a, cb, base,
-                         gp.rays, gp.bound, gp.G, gp.kcap, in_grad, accumulate, scale);
+    } else if (bricks(16, 8, 8) >= (CG == 1 ? 768u : 2048u)) {
+      NGT_SWITCH_C(CG,
+          hipLaunchKernelGGL((raymarch_bwd_brick_kernel<CC, 16, 8, 8>), dim3(bricks(16, 8, 8)), dim3(256), 0, s, a, cb, base,
+                             gp.rays, gp.bound, gp.G, gp.kcap, in_grad, accumulate, scale));
     } else {
       NGT_SWITCH_C(CG,
           hipLaunchKernelGGL((raymarch_bwd_brick_kernel<CC, 8, 8, 8>), dim3(bricks(8, 8, 8)), dim3(256), 0, s, a, cb, base,
