@@ -284,7 +284,7 @@ template <int C>
 struct ScatterTile {
   static constexpr int S = C == 4 ? 1 : 2;
   static constexpr int X = C == 4 ? 8 : 16, Y = 8, Z = 4;
-  static constexpr int kValues = C == 4 ? 6144 : 4096;  // 48 and 32 KB: three and five work-groups per CU
+  static constexpr int kValues = C == 4 ? 6144 : 4096;  // 48 and 32 KB, with the box: three and four work-groups per CU
 
   static dim3 block() { return dim3(X, Y, Z / S); }
   // Tiles along x and y, and along z for every slot: no axis has more
@@ -515,8 +515,10 @@ __global__ __launch_bounds__(256) void lut_bwd_tile_kernel(LutArgs a, MipSet dat
   }
 }
 
-// One work-item per (camera slot, output cell); loops over the data entries
-// that use this camera so the LUT gradient is summed in registers.
+// The table adjoint without mips of NEAREST / MIN / MAX, whose LUT gradient is
+// 0, and the reference's (REF: FM is LINEAR where it has a LUT gradient).  One
+// work-item per (camera slot, output cell); loops over the data entries that
+// use this camera.
 template <int C, int FM, int BM, bool REF>
 __global__ __launch_bounds__(256) void lut_bwd_kernel(LutArgs a, const float* __restrict__ out_grad,
                                                       float* __restrict__ in_grad, float* __restrict__ lut_grad,
@@ -539,23 +541,16 @@ __global__ __launch_bounds__(256) void lut_bwd_kernel(LutArgs a, const float* __
     const int slot = a.separate ? n * a.n_cams + v : n;
     const Vec<C> dy = vload<C>(out_grad + (static_cast<int64_t>(slot) * out_cells + cell) * C);
     const float* src = a.input + n * in_cells * C;
-    if constexpr (FM == LINEAR) {
-      Vec<C> dx, dyy, dz;
-      read_gradient<C, BM>(src, a.din, px, py, pz, dx, dyy, dz);
-      if constexpr (REF) {  // written per camera, the last batch entry wins
-        g0 = vdot(dy, dx); g1 = vdot(dy, dyy); g2 = vdot(dy, dz);
-      } else {
-        g0 += vdot(dy, dx); g1 += vdot(dy, dyy); g2 += vdot(dy, dz);
-      }
-    }
     if constexpr (REF) {
+      if constexpr (FM == LINEAR) {  // written per camera, the last batch entry wins
+        Vec<C> dx, dyy, dz;
+        read_gradient<C, BM>(src, a.din, px, py, pz, dx, dyy, dz);
+        g0 = vdot(dy, dx); g1 = vdot(dy, dyy); g2 = vdot(dy, dz);
+      }
       scatter_linear<C, BM, true>(in_grad + n * in_cells * C, a.din, px, py, pz, dy, hits + n * in_cells);
     } else {
       scatter_filtered<C, FM, BM>(src, in_grad + n * in_cells * C, a.din, px, py, pz, dy);
     }
-  }
-  if (!REF && a.normalized) {
-    g0 *= static_cast<float>(a.dout.x); g1 *= static_cast<float>(a.dout.y); g2 *= static_cast<float>(a.dout.z);
   }
   *reinterpret_cast<float4*>(lut_grad + (static_cast<int64_t>(v) * out_cells + cell) * 4) = make_float4(g0, g1, g2, 0.f);
 }
@@ -892,7 +887,9 @@ __global__ __launch_bounds__(256) void xform_bwd_gather_kernel(XformArgs a, CamB
       const float pz = s * ((c & 4) ? static_cast<float>(b1z) + 1.502f : static_cast<float>(b0z) - 0.502f);
       float o[3];
       const float cw = output_index<float>(cp, a.dout, a.coord_mode != NGT_COORD_TRANSFORM, px, py, pz, o);
-      // behind the camera, or no number: every output cell is a candidate
+      // the grid stands before the camera (checked on the host), so only the
+      // rounding of a corner next to the camera's plane gives a w that is not
+      // positive or an index that is huge or no number: every cell is a candidate
       unknown = !(cw > 0.f) || !(fabsf(o[0]) < 1.0e9f) || !(fabsf(o[1]) < 1.0e9f) || !(fabsf(o[2]) < 1.0e9f);
 #pragma unroll
       for (int k = 0; k < 3; ++k) lo[k] = hi[k] = o[k];

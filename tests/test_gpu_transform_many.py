@@ -53,6 +53,14 @@ def test_adjoint_of_many_grids(ngt_ops, dims, out_dhw, C, n, views, levels):  # 
           300 + n + 7 * C + 3 * views + levels)
 
 
+@pytest.mark.parametrize("mode", ["TRANSFORM_LINDEPTH", "TRANSFORM"])
+@pytest.mark.parametrize("C,levels", [(1, 0), (4, 2)])
+def test_camera_close_before_the_grid(ngt_ops, C, levels, mode):  # noqa: F811
+    """Bricks next to the camera's plane: corners far outside the view, boxes up to all of it."""
+    dims, out_dhw = (16, 12, 20), (26, 22, 24)
+    check(ngt_ops, cameras(dims, out_dhw, 3, 1, 0.75, 0.01, 1.6), dims, out_dhw, C, 1, 3, levels, mode, 800 + C)
+
+
 @pytest.mark.parametrize("dims,out_dhw,C,levels", [
     ((24, 20, 22), (10, 9, 8), 1, 0),    # 0.07 values a voxel: scatter
     ((24, 20, 22), (15, 14, 13), 1, 0),  # 0.26: gather
