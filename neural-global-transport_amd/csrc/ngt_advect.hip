@@ -492,9 +492,10 @@ __global__ __launch_bounds__(256) void mac_component_luts_bwd_kernel(Dims d, Mac
 // take turns in it.
 // Measured: 128^3, one channel, B1 / B2 45.6 / 45.7 us with fp32 tiles and
 // merged neighbours -> 40.1 / 38.6 with fp64 tiles -> 31.4 / 37.0 with the
-// unmasked corner reads and the offsets of gather_tiles, at 3.3 / 3.6 TB/s of
-// their fields, tiles and velocity gradients; 96x160x96, three channels, 717 /
-// 597 us with global fp32 atomics -> 58 / 68.  The halo sets the partial-buffer
+// unmasked corner reads and the offsets of gather_tiles -> 32.3 / 33.9 with
+// bricks 16 deep, whose second pass gathers fewer tiles (0.14 and 0.19 GB moved,
+// 0.15 and 0.21 before); 96x160x96, three channels, 717 / 597 us with global fp32
+// atomics -> 62 / 76.  The halo sets the partial-buffer
 // traffic: tile cells per brick cell 2.11, 2.53 or 3.38 with kHalo = 2 and
 // bricks 16, 8 or 4 deep.
 constexpr int kBrickX = 32, kBrickY = 8, kHalo = 2;
